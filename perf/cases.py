@@ -71,7 +71,7 @@ def _draw_model(rng, lo, hi, lattice=True, lo_n=4, hi_n=12):
     for _ in range(60):
         if lattice and rng.random() < 0.3:
             dx, dy = rng.randint(3, 6), rng.randint(3, 6)
-            n = rng.randint(3, min(hi_n, dx * dy - 2))
+            n = rng.randint(3, min(hi_n if dx * dy < 36 else 8, dx * dy - 2))  # what the tiled layout holds
             c = {"model": "lattice", "dim_x": dx, "dim_y": dy, "n": n, "kx": rng.randrange(dx), "ky": rng.randrange(dy)}
         else:
             n = rng.randint(lo_n, hi_n)
