@@ -9,7 +9,7 @@
 //     features (n_bits occupations, n_params parameters, zero padded to 64)
 //     -> 256 -> 256 -> 256 (SiLU) -> 2 S
 //
-// All layers run through one GEMM kernel, C[M x N] = A[M x K] . B[N x K]^T with
+// Training runs its layers through one GEMM kernel, C[M x N] = A[M x K] . B[N x K]^T with
 // both operands K-contiguous in BF16, FP32 accumulation in
 // v_mfma_f32_32x32x16_bf16 (a 64-lane wavefront owns a 32x32 output tile; four
 // waves make a 64x64 block tile).  Epilogues fuse bias + SiLU (forward) and the
@@ -193,124 +193,287 @@ __global__ void k_to_bf16(int rows, int cols, const float* __restrict__ w, __bf1
 
 // ---------------------------------------------------------------- inference
 //
-// The whole network for kIT states per workgroup in one launch: each of the
-// kIT/32 waves owns 32 states (one MFMA row tile) and keeps their features and
-// activations in LDS (32 x 256 BF16); the weights are staged through LDS in
-// K chunks of kIKc shared by the waves.  Every output is the MFMA sequence of
-// k_gemm (same 32x32x16 tiles, K ascending in steps of 16) with the same
-// epilogues, so the outputs equal the layer-by-layer path bit for bit, while
-// HBM sees only the states and the outputs.
-constexpr int kIT = 128;            // states per workgroup
-constexpr int kIWaves = kIT / 32;   // waves per workgroup, one 32-state strip each
-constexpr int kIKc = 32;            // K chunk of the staged weights
+// The whole network for NW * 32 states per group in one launch, a wavefront per
+// 32 states.  The products run transposed, D = W . H^T: the weights are the A
+// operand, the activations the B operand, so a lane's 16 outputs all belong to
+// its own state (column l%32) and go through bias and SiLU into the next
+// layer's B operand without leaving the registers: only the rows 4-7 / 8-11 of
+// every 16 change lane halves (v_permlane32_swap).  Every output is the MFMA
+// sequence of k_gemm (32x32x16 tiles, K ascending in steps of 16).
+//
+// The weights are read in the order of the A fragments (k_pack_infer: 1 KiB per
+// 32 x 16 fragment, lane l's 16 bytes at 16 l), ten chunks of 32 fragments
+// (layer 1 in one, layers 2 and 3 in four each, the output layer in the last),
+// double-buffered in LDS: the next chunk's loads are in flight into registers
+// while the waves multiply the current one.  Blocks are persistent (one per CU)
+// and walk the state groups, so the pipeline also runs across groups.
+//
+// Bound: the vector instructions (67% of the cycles; the SiLU is 768 of 44 cycles
+// per state) beside the MFMAs (31%) and the fragment reads from LDS.  Over the
+// N=12, 2S=33 sector (7.76M states, S = 5) 3.55 ms, 0.67 PFLOP/s on the padded
+// work, against 11.6 ms for a kernel that kept the activations in LDS (512-byte
+// rows, every access a bank conflict, two barriers per 32 columns of weights).
+// Two sets of 32 states per wave, which halve the fragment reads, need the AGPRs
+// for the activations and were slower (4.1 ms), as was a SiLU pass after each
+// tile pair's products instead of between them (3.9 ms).
+constexpr int kFrag = 512;          // BF16 elements of one 32 x 16 weight fragment
+constexpr int kChunk = 32 * kFrag;  // elements of one staged chunk (32 KiB)
+constexpr int kChunks = 10;
+constexpr int kOutT = 32;           // outputs of the last layer's tile (n_out <= 32)
 
 struct InferArgs {
     int64_t n;
     const uint64_t* states;
     const float* params;  // n_params values, per state when per_sample
     int per_sample, n_bits, n_params;
-    const __bf16* w[4];   // BF16 weights, padded shapes (out x in)
+    const __bf16* wf;     // packed weights, kChunks * kChunk elements
     const float* b[4];
     int n_out;            // live outputs per state: 2 per amplitude (log|psi|, sign logit)
     float* out;           // n x n_out
     float* partial_max;   // per workgroup and amplitude s: largest output 2s over its states
 };
 
-__global__ void __launch_bounds__(kIWaves * 64) k_mlp_infer(InferArgs g)
+// Fragment-ordered copy of the four layers: fragment f = tile * (K/16) + k/16 of
+// each layer in turn, lane l's eight values W[32 tile + l%32][16 (k/16) + 8 (l/32) ..+7].
+__global__ void __launch_bounds__(256) k_pack_infer(const float* __restrict__ w0, const float* __restrict__ w1,
+                                                    const float* __restrict__ w2, const float* __restrict__ w3,
+                                                    __bf16* __restrict__ wf)
 {
-    __shared__ __bf16 act[kIT * kW];
-    __shared__ __bf16 wc[kW * kIKc];
-    __shared__ float red[kIWaves][32];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = lane & 31, kh = (lane >> 5) * 8;
-    const int64_t s0 = (int64_t)blockIdx.x * kIT + wave * 32;
-    __bf16* strip = act + (size_t)wave * 32 * kW;
-    {   // features of state s0 + r: lane halves build columns 0-31 and 32-63
-        const int64_t b = s0 + r;
-        const bool live = b < g.n;
-        const uint64_t st = live ? g.states[b] : 0ull;
-        const float* p = g.params + (g.per_sample && live ? b * g.n_params : 0);
-        for (int k = (lane >> 5) * 32; k < (lane >> 5) * 32 + 32; ++k) {
-            float f = 0.f;
-            if (live) {
-                if (k < g.n_bits) f = (float)((st >> k) & 1ull);
-                else if (k < g.n_bits + g.n_params) f = p[k - g.n_bits];
-            }
-            strip[r * kW + k] = (__bf16)f;
-        }
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= kChunks * kChunk) return;
+    const int frag = e / kFrag, lane = (e % kFrag) >> 3, j = e & 7;
+    const float* w = w0;
+    int f = frag, ks = kIn / 16;
+    if (frag >= 288) { w = w3; f = frag - 288; ks = kW / 16; }
+    else if (frag >= 160) { w = w2; f = frag - 160; ks = kW / 16; }
+    else if (frag >= 32) { w = w1; f = frag - 32; ks = kW / 16; }
+    const int row = (f / ks) * 32 + (lane & 31), k = (f % ks) * 16 + (lane >> 5) * 8 + j;
+    // the last chunk is half used: the output tile's 16 fragments
+    wf[e] = frag >= 304 ? (__bf16)0.f : (__bf16)w[row * (ks * 16) + k];
+}
+
+// z / (1 + exp(-z)) with the quotient from v_rcp_f32 and one correction step (the
+// remainder z - q d, exact in the fma), instead of the IEEE division sequence; the
+// same bits as the division on every network compared.  The exponent is capped so
+// that the denominator stays finite: below z = -87 the value is z 2^-126 instead
+// of -0.  z = +inf gives NaN (the division: +inf), NaN stays NaN.
+HD_DEV float silu_fast(float z)
+{
+    const float d = 1.f + __builtin_amdgcn_exp2f(fminf(z * -1.44269504088896341f, 126.f));
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float q = z * r;
+    return fmaf(fmaf(-q, d, z), r, q);
+}
+
+HD_DEV uint32_t pack_bf16(float a, float b)
+{
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    bf16x2 v;
+    v[0] = (__bf16)a;
+    v[1] = (__bf16)b;
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+// Eight consecutive outputs (bias and SiLU applied) of the lane's state for one
+// 16-row block: lo holds rows 4h .. 4h+3 and hi rows 8+4h .. 8+4h+3 of lane half h;
+// the swap leaves half h with rows 8h .. 8h+7, the B operand's order.
+HD_DEV bf16x8 to_operand(const float (&lo)[4], const float (&hi)[4])
+{
+    uint32_t v[4];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const auto r = __builtin_amdgcn_permlane32_swap(pack_bf16(lo[2 * q], lo[2 * q + 1]),
+                                                        pack_bf16(hi[2 * q], hi[2 * q + 1]), false, false);
+        v[q] = r[0];
+        v[2 + q] = r[1];
     }
-    // hidden layers: 64 -> 256 -> 256 -> 256, bias + SiLU
-    for (int l = 0; l < 3; ++l) {
-        const int K = l == 0 ? kIn : kW;
-        f32x16 acc[8];
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 p = {v[0], v[1], v[2], v[3]};
+    return __builtin_bit_cast(bf16x8, p);
+}
+
+// One output tile (32 rows): acc = the tile's weights times `in`, KS steps of one
+// fragment each.  Between the MFMAs the previous tile's 16 outputs `prev` go
+// through bias (pb, in LDS) and SiLU into out[0] and out[1]: a step's vector
+// instructions issue while its MFMA runs in the matrix core.  All of `prev` is
+// done two steps before the end, so a tile that opens the next layer may have the
+// previous layer's last tile as its last two inputs.
+template <int KS, bool PREV>
+HD_DEV f32x16 infer_tile(const __bf16* wt, const bf16x8* in, const f32x16& prev, const float* pb, bf16x8* out, int lane)
+{
+    const bf16x8* w = reinterpret_cast<const bf16x8*>(wt) + lane;
+    const float* pl = pb + (lane >> 5) * 4;
+    constexpr int kAhead = 2;  // fragments read ahead
+    bf16x8 a[kAhead];
 #pragma unroll
-        for (int t = 0; t < 8; ++t) acc[t] = f32x16{};
-        for (int kc = 0; kc < K; kc += kIKc) {
-            __syncthreads();  // the previous chunk is consumed
-            for (int i = threadIdx.x; i < kW * (kIKc / 8); i += kIWaves * 64) {
-                const int nr = i / (kIKc / 8), kp = (i % (kIKc / 8)) * 8;
-                *reinterpret_cast<bf16x8*>(&wc[nr * kIKc + kp]) =
-                    *reinterpret_cast<const bf16x8*>(g.w[l] + (size_t)nr * K + kc + kp);
-            }
-            __syncthreads();
+    for (int i = 0; i < kAhead; ++i) a[i] = w[i * (kFrag / 8)];
+    f32x16 acc = {};
+    float v[16];
+    float4 b4 = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-            for (int k16 = 0; k16 < kIKc; k16 += 16) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(&strip[r * kW + kc + k16 + kh]);
+    for (int ks = 0; ks < KS; ++ks) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks % kAhead], in[ks], acc, 0, 0, 0);
+        if (ks + kAhead < KS) a[ks % kAhead] = w[(ks + kAhead) * (kFrag / 8)];
+        if constexpr (PREV) {
+            // steps 0 and 1 take two elements, steps 2 to 13 one (KS = 16); four each (KS = 4)
+            const int e0 = KS == 4 ? 4 * ks : ks < 2 ? 2 * ks : ks + 2;
+            const int e1 = KS == 4 ? 4 * ks + 4 : ks < 2 ? 2 * ks + 2 : ks < 14 ? ks + 3 : ks + 2;
 #pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&wc[(t * 32 + r) * kIKc + k16 + kh]);
-                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bv, acc[t], 0, 0, 0);
+            for (int e = e0; e < e1; ++e) {
+                if ((e & 3) == 0) b4 = *reinterpret_cast<const float4*>(pl + (e >> 2) * 8);
+                const float be = (e & 3) == 0 ? b4.x : (e & 3) == 1 ? b4.y : (e & 3) == 2 ? b4.z : b4.w;
+                v[e] = silu_fast(prev[e] + be);
+                if ((e & 7) == 7) {
+                    const float lo[4] = {v[e - 7], v[e - 6], v[e - 5], v[e - 4]};
+                    const float hi[4] = {v[e - 3], v[e - 2], v[e - 1], v[e]};
+                    out[e >> 3] = to_operand(lo, hi);
                 }
             }
         }
-        // every read of this wave's strip has been consumed by the MFMAs above;
-        // other waves never read it
+        // keeps pairs of steps apart: hoisting more fragments and SiLUs spills
+        if (ks % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    }
+    return acc;
+}
+
+template <int NW>
+__global__ void __launch_bounds__(NW * 64, NW / 4) k_mlp_infer(InferArgs g)
+{
+    constexpr int T = NW * 64, NS = NW * 32, NP = kChunk / (T * 8);
+    __shared__ __align__(16) __bf16 wbuf[2][kChunk];
+    __shared__ __align__(16) float sb[3 * kW + kOutT];
+    __shared__ float stage[NS * kOutT];  // one group's outputs, n_out per state
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 31, half = lane >> 5;
+    for (int i = tid; i < 3 * kW + kOutT; i += T) sb[i] = g.b[i / kW][i % kW];
+    // chunk c into buffer `buf`, straight from global memory to LDS (each wave
+    // instruction moves 64 x 16 bytes to consecutive LDS addresses); settle() waits
+    // for the loads and for every wave
+    auto fetch = [&](int c, int buf) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int i = 0; i < NP; ++i)
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)(g.wf + (size_t)c * kChunk + (i * T + tid) * 8),
+                (__attribute__((address_space(3))) void*)&wbuf[buf][(i * T + wave * 64) * 8], 16, 0, 0);
+    };
+    auto settle = [&]() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+    fetch(0, 0);
+    settle();
+    float mx[16 / NW];  // running maxima of amplitudes wave + NW q (16 at most)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int row = (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-                const int col = t * 32 + r;
-                strip[row * kW + col] = (__bf16)silu(acc[t][i] + g.b[l][col]);
+    for (float& m : mx) m = -3.0e38f;
+    const int64_t groups = (g.n + NS - 1) / NS;
+    for (int64_t grp = blockIdx.x; grp < groups; grp += gridDim.x) {
+        const int64_t s0 = grp * NS + wave * 32;
+        bf16x8 x[kIn / 16], h1[kW / 16], h2[kW / 16];
+        {   // features of state s0 + r, columns 16 ks + 8 half ..+7
+            const int64_t b = s0 + r;
+            const bool live = b < g.n;
+            uint64_t st = live ? g.states[b] : 0ull;
+            if (g.n_bits < 64) st &= (1ull << g.n_bits) - 1;
+            const float* p = g.params + (g.per_sample && live ? b * g.n_params : 0);
+            uint32_t xd[kIn / 16][4];  // two features per word, 0 or 1.0 (0x3F80) each
+#pragma unroll
+            for (int ks = 0; ks < kIn / 16; ++ks)
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const uint32_t t = (uint32_t)(st >> (ks * 16 + half * 8 + 2 * d));
+                    xd[ks][d] = ((t & 1u) | ((t & 2u) << 15)) * 0x3F80u;
+                }
+            for (int i = 0; i < g.n_params; ++i) {
+                const int k = g.n_bits + i;
+                const uint32_t v = pack_bf16(live ? p[i] : 0.f, 0.f) << ((k & 1) * 16);
+                const bool mine = half == ((k >> 3) & 1);
+#pragma unroll
+                for (int w = 0; w < kIn / 4; ++w)  // word w: columns 16 (w/4) + 8 half + 2 (w%4)
+                    if (w == (k >> 4) * 4 + ((k & 7) >> 1) && mine) xd[w >> 2][w & 3] |= v;
             }
-    }
-    // output layer: 256 -> the first 32 (padded) outputs, bias
-    f32x16 acc = f32x16{};
-    for (int kc = 0; kc < kW; kc += kIKc) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < 32 * (kIKc / 8); i += kIWaves * 64) {
-            const int nr = i / (kIKc / 8), kp = (i % (kIKc / 8)) * 8;
-            *reinterpret_cast<bf16x8*>(&wc[nr * kIKc + kp]) =
-                *reinterpret_cast<const bf16x8*>(g.w[3] + (size_t)nr * kW + kc + kp);
-        }
-        __syncthreads();
 #pragma unroll
-        for (int k16 = 0; k16 < kIKc; k16 += 16) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&strip[r * kW + kc + k16 + kh]);
-            const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&wc[r * kIKc + k16 + kh]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bv, acc, 0, 0, 0);
+            for (int ks = 0; ks < kIn / 16; ++ks) x[ks] = __builtin_bit_cast(bf16x8, xd[ks]);
         }
-    }
-    float mx = -3.0e38f;  // this lane's column (even columns are log-amplitudes)
+        // chunk c is in wbuf[c & 1]; ten chunks per group keep the parity
+        fetch(1, 1);
+        f32x16 acc = infer_tile<kIn / 16, false>(wbuf[0], x, f32x16{}, sb, h1, lane);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int row = (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-        const int64_t b = s0 + row;
-        if (r < g.n_out && b < g.n) {
-            const float v = acc[i] + g.b[3][r];
-            g.out[b * g.n_out + r] = v;
-            mx = fmaxf(mx, v);
+        for (int t = 1; t < 8; ++t)
+            acc = infer_tile<kIn / 16, true>(wbuf[0] + t * (kIn / 16) * kFrag, x, acc, sb + (t - 1) * 32, h1 + 2 * t - 2, lane);
+        settle();
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            fetch(2 + c, c & 1);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int t = 2 * c + u;  // tile t of layer 2; tile t - 1 (or layer 1's last) is finished
+                acc = infer_tile<kW / 16, true>(wbuf[(1 + c) & 1] + u * (kW / 16) * kFrag, h1, acc,
+                                                sb + (t ? kW + (t - 1) * 32 : 7 * 32), t ? h2 + 2 * t - 2 : h1 + 14, lane);
+            }
+            settle();
         }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            fetch(6 + c, c & 1);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int t = 2 * c + u;
+                acc = infer_tile<kW / 16, true>(wbuf[(5 + c) & 1] + u * (kW / 16) * kFrag, h2, acc,
+                                                sb + kW + (t ? kW + (t - 1) * 32 : 7 * 32), t ? h1 + 2 * t - 2 : h2 + 14, lane);
+            }
+            settle();
+        }
+        fetch(0, 0);
+        acc = infer_tile<kW / 16, true>(wbuf[1], h1, acc, sb + 2 * kW + 7 * 32, h1 + 14, lane);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int row = (i >> 2) * 8 + half * 4 + (i & 3);
+            if (row < g.n_out) stage[(wave * 32 + r) * g.n_out + row] = acc[i] + sb[3 * kW + row];
+        }
+        settle();
+        // the group's outputs are contiguous in g.out
+        const int64_t left = g.n - grp * NS;
+        const int live_states = left < NS ? (int)left : NS;
+        const int live = live_states * g.n_out;
+        float* o = g.out + grp * NS * g.n_out;
+        for (int i = tid; i < live; i += T) o[i] = stage[i];
+#pragma unroll
+        for (int q = 0; q < 16 / NW; ++q) {
+            const int s = wave + NW * q;
+            if (2 * s < g.n_out)
+                for (int i = lane; i < live_states; i += 64) mx[q] = fmaxf(mx[q], stage[i * g.n_out + 2 * s]);
+        }
+        // the next write to `stage` comes after the next group's barriers
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));  // the two half-waves hold the same column
-    if (lane < 32) red[wave][lane] = mx;
-    __syncthreads();
-    if ((int)threadIdx.x < g.n_out / 2) {
-        const int c = 2 * threadIdx.x;
-        float m = red[0][c];
-        for (int w = 1; w < kIWaves; ++w) m = fmaxf(m, red[w][c]);
-        g.partial_max[(int64_t)blockIdx.x * (g.n_out / 2) + threadIdx.x] = m;
+#pragma unroll
+    for (int q = 0; q < 16 / NW; ++q) {
+        const int s = wave + NW * q;
+        float m = mx[q];
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+        if (lane == 0 && 2 * s < g.n_out) g.partial_max[(int64_t)blockIdx.x * (g.n_out / 2) + s] = m;
     }
+}
+
+// Launch shape: one persistent block per CU.  Eight waves (two per SIMD, so one's
+// SiLU overlaps the other's MFMAs) once every CU has a group of 256 states; below
+// that four waves and 128 states, which spreads a small sector over twice the CUs.
+struct InferGrid {
+    int nw;
+    unsigned blocks;
+};
+static InferGrid infer_grid(int64_t n, int n_cu)
+{
+    InferGrid q;
+    q.nw = n >= (int64_t)n_cu * 256 ? 8 : 4;
+    q.blocks = (unsigned)std::min<int64_t>(n_cu, (n + q.nw * 32 - 1) / (q.nw * 32));
+    return q;
+}
+
+static void infer_launch(const InferArgs& a, const InferGrid& q, hipStream_t st)
+{
+    if (q.nw == 8) hipLaunchKernelGGL(k_mlp_infer<8>, dim3(q.blocks), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL(k_mlp_infer<4>, dim3(q.blocks), dim3(256), 0, st, a);
 }
 
 // shift[s] = max over workgroups of partial[w * S + s] (one block per amplitude, fixed order)
@@ -330,34 +493,55 @@ __global__ void __launch_bounds__(256) k_max_states(int64_t nblk, int S, const f
     if (threadIdx.x == 0) shift[s] = red[0];
 }
 
-// part[blk * S + s] = sum over this block's states of exp(2 (o_2s - shift_s))
+// part[blk * S + s] = sum over this block's states of exp(2 (o_2s - shift_s)); all
+// amplitudes in one pass over the outputs (S <= MS), each state's outputs read by
+// one thread.
+template <int MS>
 __global__ void __launch_bounds__(256) k_norm2_states(int64_t n, int S, const float* __restrict__ out,
                                                       const float* __restrict__ shift, double* __restrict__ part)
 {
-    __shared__ double red[256];
-    for (int s = 0; s < S; ++s) {
-        double acc = 0.0;
-        for (int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x; b < n; b += (int64_t)gridDim.x * 256)
-            acc += exp(2.0 * (double)(out[b * 2 * S + 2 * s] - shift[s]));
-        red[threadIdx.x] = acc;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) part[(int64_t)blockIdx.x * S + s] = red[0];
-        __syncthreads();
+    __shared__ double red[4][MS];
+    double acc[MS];
+    float sh[MS];
+#pragma unroll
+    for (int s = 0; s < MS; ++s) {
+        acc[s] = 0.0;
+        sh[s] = s < S ? shift[s] : 0.f;
+    }
+    for (int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x; b < n; b += (int64_t)gridDim.x * 256) {
+#pragma unroll
+        for (int s = 0; s < MS; ++s)
+            if (s < S) acc[s] += exp(2.0 * (double)(out[b * 2 * S + 2 * s] - sh[s]));
+    }
+#pragma unroll
+    for (int s = 0; s < MS; ++s) {
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) acc[s] += __shfl_xor(acc[s], d, 64);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][s] = acc[s];
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < S) {
+        const int s = threadIdx.x;
+        part[(int64_t)blockIdx.x * S + s] = (red[0][s] + red[1][s]) + (red[2][s] + red[3][s]);
     }
 }
 
-// inv[s] = 1 / sqrt(sum over blocks of part[blk * S + s]) (one thread per amplitude, block order)
-__global__ void k_inv_norm_states(int nb, int S, const double* __restrict__ part, double* __restrict__ inv)
+// inv[s] = 1 / sqrt(sum over blocks of part[blk * S + s]) (one block per amplitude,
+// fixed order)
+__global__ void __launch_bounds__(256) k_inv_norm_states(int nb, int S, const double* __restrict__ part,
+                                                         double* __restrict__ inv)
 {
-    const int s = threadIdx.x;
-    if (s >= S) return;
+    __shared__ double red[256];
+    const int s = blockIdx.x;
     double t = 0.0;
-    for (int b = 0; b < nb; ++b) t += part[(int64_t)b * S + s];
-    inv[s] = t > 0.0 ? 1.0 / sqrt(t) : 0.0;
+    for (int b = threadIdx.x; b < nb; b += 256) t += part[(int64_t)b * S + s];
+    red[threadIdx.x] = t;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) inv[s] = red[0] > 0.0 ? 1.0 / sqrt(red[0]) : 0.0;
 }
 
 // psi_b = sum_s exp(o_2s - shift_s) sign(o_2s+1) * scale_s; with one amplitude
@@ -395,6 +579,7 @@ struct hd_mlp {
     float* b[4] = {};
     __bf16* wb[4] = {};   // BF16 copy
     __bf16* wbT[4] = {};  // BF16 transposed copy
+    __bf16* wf = nullptr; // BF16 copy in the inference kernel's fragment order
     float *mw[4] = {}, *vw[4] = {}, *mb[4] = {}, *vb[4] = {};  // Adam moments
     float *gw[4] = {}, *gb[4] = {};
     int64_t step = 0;
@@ -463,6 +648,8 @@ int mlp_refresh_bf16(hd_mlp* m)
         hipLaunchKernelGGL(k_to_bf16, dim3((n + 255) / 256), dim3(256), 0, m->stream, m->rows[l], m->cols[l], m->w[l],
                            m->wb[l], m->wbT[l]);
     }
+    hipLaunchKernelGGL(k_pack_infer, dim3(kChunks * kChunk / 256), dim3(256), 0, m->stream, m->w[0], m->w[1], m->w[2],
+                       m->w[3], m->wf);
     HD_HIP(hipGetLastError());
     return HD_OK;
 }
@@ -496,10 +683,8 @@ InferArgs infer_args(const hd_mlp* m, int64_t n, const uint64_t* states, const f
     a.per_sample = per_sample;
     a.n_bits = m->n_bits;
     a.n_params = m->n_params;
-    for (int l = 0; l < 4; ++l) {
-        a.w[l] = m->wb[l];
-        a.b[l] = m->b[l];
-    }
+    a.wf = m->wf;
+    for (int l = 0; l < 4; ++l) a.b[l] = m->b[l];
     a.n_out = m->live_rows[3];
     a.out = out;
     a.partial_max = partial_max;
@@ -665,6 +850,7 @@ int hd_mlp_create_states(int32_t n_bits, int32_t n_params, int32_t n_states, uin
         HD_ENQ(q, hipMemsetAsync(m->vb[l], 0, (size_t)R * 4, m->stream));
     }
     if (st == HD_OK) st = q.status();
+    if (st == HD_OK) st = dalloc_t(&m->wf, (size_t)kChunks * kChunk, "MLP packed weights");
     if (st == HD_OK) st = mlp_refresh_bf16(m);
     if (st == HD_OK && hipStreamSynchronize(m->stream) != hipSuccess) st = fail(HD_ERR_HIP, "MLP init failed");
     if (st != HD_OK) {
@@ -686,7 +872,7 @@ int hd_mlp_destroy(hd_mlp* m)
                         (void*)m->gb[l], (void*)m->mw[l], (void*)m->vw[l], (void*)m->mb[l], (void*)m->vb[l]})
             dfree(p);
     }
-    dfree(m->st_buf); dfree(m->pr_buf); dfree(m->tg_buf);
+    dfree(m->st_buf); dfree(m->pr_buf); dfree(m->tg_buf); dfree(m->wf);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
     return HD_OK;
@@ -741,14 +927,17 @@ int hd_mlp_forward(hd_mlp* m, const uint64_t* h_states, const float* h_params, i
     const uint64_t* ds;
     const float *dp, *dt;
     HD_CHECK(stage_batch(m, h_states, h_params, nullptr, n, true, &ds, &dp, &dt, 1));
-    const int64_t nblk = (n + kIT - 1) / kIT;
+    int n_cu = 256;
+    HD_CHECK(device_props(&n_cu, nullptr));
+    const InferGrid grid = infer_grid(n, n_cu);
+    const int64_t nblk = grid.blocks;
     float *dout = nullptr, *dmax = nullptr;
     const int S = m->n_states;
     HD_CHECK(dalloc_t(&dout, (size_t)n * 2 * S, "MLP outputs"));
     int st = dalloc_t(&dmax, (size_t)nblk * S, "MLP output maxima");
     if (st == HD_OK) {
         InferArgs a = infer_args(m, n, ds, dp, 1, dout, dmax);
-        hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)nblk), dim3(kIWaves * 64), 0, m->stream, a);
+        infer_launch(a, grid, m->stream);
         HipErrors q;
         HD_ENQ(q, hipGetLastError());
         HD_ENQ(q, hipMemcpyAsync(h_out, dout, sizeof(float) * 2 * S * n, hipMemcpyDeviceToHost, m->stream));
@@ -795,7 +984,10 @@ int hd_mlp_start_vector(hd_mlp* m, const hd_basis* basis, const float* h_params,
     const int64_t n = basis->dim;
     if (n == 0) return HD_OK;
     const int S = m->n_states;
-    const int64_t nblk = (n + kIT - 1) / kIT;
+    int n_cu = 256;
+    HD_CHECK(device_props(&n_cu, nullptr));
+    const InferGrid grid = infer_grid(n, n_cu);
+    const int64_t nblk = grid.blocks;
     const int nred = (int)std::min<int64_t>((n + 255) / 256, 1024);
     float *dpar = nullptr, *dout = nullptr, *dmax = nullptr;
     double* dnorm = nullptr;
@@ -810,15 +1002,18 @@ int hd_mlp_start_vector(hd_mlp* m, const hd_basis* basis, const float* h_params,
         HipErrors q;
         HD_ENQ(q, hipMemcpyAsync(dpar, h_params, sizeof(float) * m->n_params, hipMemcpyHostToDevice, m->stream));
         InferArgs a = infer_args(m, n, basis->d_states, dpar, 0, dout, dmax);
-        hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)nblk), dim3(kIWaves * 64), 0, m->stream, a);
+        infer_launch(a, grid, m->stream);
         HD_ENQ(q, hipGetLastError());
         float* shift = dpar + np;
         hipLaunchKernelGGL(k_max_states, dim3(S), dim3(256), 0, m->stream, nblk, S, dmax, shift);
         HD_ENQ(q, hipGetLastError());
         double* inv = dnorm + (size_t)nred * S;
         if (S > 1) {
-            hipLaunchKernelGGL(k_norm2_states, dim3(nred), dim3(256), 0, m->stream, n, S, dout, shift, dnorm);
-            hipLaunchKernelGGL(k_inv_norm_states, dim3(1), dim3(64), 0, m->stream, nred, S, dnorm, inv);
+            if (S <= 8)
+                hipLaunchKernelGGL(k_norm2_states<8>, dim3(nred), dim3(256), 0, m->stream, n, S, dout, shift, dnorm);
+            else
+                hipLaunchKernelGGL(k_norm2_states<16>, dim3(nred), dim3(256), 0, m->stream, n, S, dout, shift, dnorm);
+            hipLaunchKernelGGL(k_inv_norm_states, dim3(S), dim3(256), 0, m->stream, nred, S, dnorm, inv);
             HD_ENQ(q, hipGetLastError());
         }
         hipLaunchKernelGGL(k_amplitude, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, n, S, dout, shift,

@@ -162,3 +162,41 @@ def test_multi_amplitude_start_vector():
     assert np.max(np.abs(v - want / np.linalg.norm(want))) < 1e-12
     r = h.lanczos(nev=3, tol=1e-10, start=net.start_vector(basis, held))
     assert r.converged and np.max(np.abs(r.evals - ref.evals)) < 1e-9
+
+
+@pytest.mark.parametrize("n_bits,n_params,n_states,n", [
+    (34, 3, 5, 1), (20, 0, 16, 31), (22, 3, 1, 33), (61, 3, 8, 127), (30, 2, 3, 129), (34, 3, 5, 256 * 256 + 37)])
+def test_inference_tiles_match_oracle(n_bits, n_params, n_states, n):
+    """The inference kernel at the edges of its 32-state tiles, its 128- and
+    256-state groups and its output widths.  A BF16 activation that falls on
+    the other side of a rounding boundary moves by 2^-8 of itself; a few such
+    flips among the 256 inputs of an output stay below 2^-8 of the outputs'
+    scale.  A batch large enough for the 256-state groups gives its first
+    states the outputs they have alone, bit for bit."""
+    say("mlp inference", n_bits, n_params, n_states, n)
+    rng = np.random.default_rng(n)
+    net = learned.AmplitudeNet(n_bits, n_params, seed=2, n_states=n_states)
+    w = net.get_weights()
+    states = rng.integers(0, 1 << n_bits, size=n).astype(np.uint64)
+    params = rng.random((n, n_params)).astype(np.float32)
+    out = net.forward(states, params)
+    want = mo.forward(w, states, params, n_bits, n_params, bf=True)[0][:, :2 * n_states]
+    assert np.max(np.abs(out - want)) <= 2.0 ** -8 * max(1.0, np.max(np.abs(want)))
+    k = min(n, 129)
+    assert np.array_equal(out[:k], net.forward(states[:k], params[:k]))
+
+
+def test_start_vector_large_sector_matches_forward():
+    """Above 65,536 states the start vector runs 256-state groups; it equals the
+    sum of the normalised amplitudes assembled from the forward outputs."""
+    say("start vector N=8 2S=28, 81446 states")
+    basis = hd.FockBasis(hd.Sector.lz(4, 28), 8, 29)
+    net = learned.AmplitudeNet(29, 3, seed=4, n_states=9)
+    p = np.array([0.7, 0.2, 0.1], dtype=np.float32)
+    v = net.start_vector(basis, p).to_array(np.float64, basis.dim)
+    out = net.forward(basis.states(), np.repeat(p[None, :], basis.dim, axis=0))
+    want = np.zeros(basis.dim)
+    for s in range(9):
+        a = np.exp((out[:, 2 * s] - out[:, 2 * s].max()).astype(np.float64)) * np.where(out[:, 2 * s + 1] >= 0, 1.0, -1.0)
+        want += a / np.linalg.norm(a)
+    assert np.linalg.norm(v - want) <= 1e-13 * np.linalg.norm(want)
