@@ -962,7 +962,7 @@ int hd_batch_create(const hd_basis* const* bases, int32_t n_sectors, const hd_ta
         return st;
     };
     if (hipGetDevice(&b->device) != hipSuccess ||
-        hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
+        stream_get(&b->stream) != hipSuccess)
         return bail(fail(HD_ERR_HIP, "stream creation failed"));
     // per-sector coded patterns with one shared tuple dictionary
     BatchTables bt;
@@ -1061,7 +1061,7 @@ int hd_batch_destroy(hd_batch* b)
     dfree(b->d_code);
     dfree(b->d_dict);
     dfree(b->d_diag);
-    if (b->stream) (void)hipStreamDestroy(b->stream);
+    if (b->stream) stream_put(b->stream);
     delete b;
     return HD_OK;
 }

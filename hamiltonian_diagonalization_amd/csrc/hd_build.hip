@@ -1800,7 +1800,7 @@ static int build_batch_merged(const hd_basis* b, const Derived& M, double tol, h
     h->dim = b->dim;
     h->storage = HD_STORAGE_FULL;
     if (hipGetDevice(&h->device) != hipSuccess ||
-        hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
+        stream_get(&h->stream) != hipSuccess) {
         delete h;
         return fail(HD_ERR_HIP, "stream creation failed");
     }
@@ -2061,7 +2061,7 @@ int hd_ham_build(const hd_basis* b, const hd_tables* t, int32_t storage, double 
         h->storage = storage;
         h->is_complex = t->is_complex;
         if (hipGetDevice(&h->device) != hipSuccess ||
-            hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
+            stream_get(&h->stream) != hipSuccess) {
             delete h;
             return fail(HD_ERR_HIP, "stream creation failed");
         }
@@ -2085,7 +2085,7 @@ int hd_ham_build(const hd_basis* b, const hd_tables* t, int32_t storage, double 
     h->storage = storage;
     h->is_complex = t->is_complex;
     if (hipGetDevice(&h->device) != hipSuccess ||
-        hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
+        stream_get(&h->stream) != hipSuccess) {
         delete h;
         return fail(HD_ERR_HIP, "stream creation failed");
     }
@@ -2116,7 +2116,7 @@ int hd_ham_destroy(hd_hamiltonian* h)
     dfree(h->d_mf_pval);
     dfree(h->d_mf_split);
     tiled_free(h);
-    if (h->stream) (void)hipStreamDestroy(h->stream);
+    if (h->stream) stream_put(h->stream);
     delete h;
     return HD_OK;
 }

@@ -814,7 +814,7 @@ int hd_mlp_create_states(int32_t n_bits, int32_t n_params, int32_t n_states, uin
     m->n_params = n_params;
     m->n_states = n_states;
     m->live_rows[3] = 2 * n_states;
-    if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) {
+    if (stream_get(&m->stream) != hipSuccess) {
         delete m;
         return fail(HD_ERR_HIP, "stream creation failed");
     }
@@ -873,7 +873,7 @@ int hd_mlp_destroy(hd_mlp* m)
             dfree(p);
     }
     dfree(m->st_buf); dfree(m->pr_buf); dfree(m->tg_buf); dfree(m->wf);
-    if (m->stream) (void)hipStreamDestroy(m->stream);
+    if (m->stream) stream_put(m->stream);
     delete m;
     return HD_OK;
 }

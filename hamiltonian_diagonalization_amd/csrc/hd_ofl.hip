@@ -287,7 +287,7 @@ int hd_ofl_vtable(int32_t dim_x, int32_t dim_y, int32_t cutoff, const double* h_
     const size_t bloch_n = (size_t)a.K * 2 * a.n;
     double2 *d_bloch = nullptr, *d_out = nullptr;
     hipStream_t st = nullptr;
-    if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess)
+    if (stream_get(&st) != hipSuccess)
         return fail(HD_ERR_HIP, "stream creation failed");
     int rc = dalloc_t(&d_bloch, bloch_n, "Bloch coefficients");
     if (rc == HD_OK) rc = dalloc_t(&d_out, (size_t)a.entries, "quartic terms");
@@ -311,7 +311,7 @@ int hd_ofl_vtable(int32_t dim_x, int32_t dim_y, int32_t cutoff, const double* h_
     }
     dfree(d_bloch);
     dfree(d_out);
-    (void)hipStreamDestroy(st);
+    stream_put(st);
     return rc;
 }
 
@@ -376,7 +376,7 @@ int hd_ofl_wannier(int32_t dim_x, int32_t dim_y, double offset_x, const uint16_t
     double2 *d_vt = nullptr, *d_u = nullptr, *d_v = nullptr;
     uint8_t *d_nk1 = nullptr, *d_k1 = nullptr;
     hipStream_t st = nullptr;
-    if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess)
+    if (stream_get(&st) != hipSuccess)
         return fail(HD_ERR_HIP, "stream creation failed");
     int rc = dalloc_t(&d_kt, (size_t)folded, "Bloch k table");
     if (rc == HD_OK) rc = dalloc_t(&d_vt, (size_t)folded, "Bloch V table");
@@ -414,7 +414,7 @@ int hd_ofl_wannier(int32_t dim_x, int32_t dim_y, double offset_x, const uint16_t
     dfree(d_v);
     dfree(d_nk1);
     dfree(d_k1);
-    (void)hipStreamDestroy(st);
+    stream_put(st);
     return rc;
 }
 

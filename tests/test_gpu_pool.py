@@ -1,0 +1,89 @@
+"""The library's pool of device blocks: contents of blocks handed out to several
+threads, blocks of every size class, and the bound on what it keeps."""
+import ctypes
+import gc
+import sys
+import threading
+
+import numpy as np
+import pytest
+
+import hamiltonian_diagonalization_amd as hd
+from hamiltonian_diagonalization_amd import models
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print("[gpu-case]", *a, flush=True)
+    sys.stdout.flush()
+
+
+def test_blocks_of_several_threads_stay_apart():
+    say("pool: 4 threads, blocks of 1 byte to 8 MiB")
+    errors = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        held = []
+        for i in range(60):
+            n = int(np.exp(rng.uniform(0, np.log(8 << 20))))
+            a = rng.integers(0, 256, size=n, dtype=np.uint8)
+            held.append((hd.DeviceBuffer.from_array(a), a))
+            while len(held) > 3 or (i == 59 and held):
+                b, want = held.pop(int(rng.integers(len(held))))
+                if not np.array_equal(b.to_array(np.uint8, len(want)), want):
+                    errors.append((seed, i, len(want)))
+                del b
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+
+
+@pytest.mark.parametrize("nbytes", [1, 256, 257, 1 << 20, (1 << 20) + 1, (2 << 20) - 1, 2 << 20, (2 << 20) + 1])
+def test_block_sizes(nbytes):
+    say("pool: block of", nbytes)
+    for fill in (1, 2):  # the second one reuses the first one's block
+        a = np.full(nbytes, fill, dtype=np.uint8)
+        assert np.array_equal(hd.DeviceBuffer.from_array(a).to_array(np.uint8, nbytes), a)
+
+
+def _mem_info():
+    """(free, total) bytes from the HIP runtime that the library is linked to."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64.so" in line)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value, total.value
+
+
+def test_idle_blocks_are_bounded():
+    say("pool: 12 blocks of 8 GiB returned")
+    gc.collect()
+    hd._check(hd.lib().hd_synchronize())
+    free0, total = _mem_info()
+    keep = hd.DeviceBuffer(16)
+    blocks = [hd.DeviceBuffer(8 << 30) for _ in range(12)]
+    assert _mem_info()[0] <= free0 - (90 << 30)
+    del blocks
+    assert _mem_info()[0] >= free0 - total // 6 - (1 << 30)
+    del keep
+
+
+def test_builds_in_a_loop_are_identical():
+    """Blocks that held another sector's arrays change nothing."""
+    say("pool: alternating builds, N=8 2S=21 and N=7 2S=18")
+    want = {}
+    for _ in range(3):
+        for n, two_s in ((8, 21), (7, 18)):
+            b, t = models.sphere_problem(n, two_s, 0)
+            h = hd.Hamiltonian(b, t)
+            h.tile()
+            x = np.random.default_rng(n).standard_normal(b.dim)
+            got = [*h.crs(), h.spmv(x, precision=hd.TILED), h.spmv(x, precision=hd.CODED)]
+            for a, w in zip(got, want.setdefault(n, got)):
+                assert np.array_equal(a, w)
