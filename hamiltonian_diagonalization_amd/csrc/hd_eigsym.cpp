@@ -15,13 +15,14 @@
 namespace hd {
 
 // A (n x n, row-major, symmetric) is destroyed; w ascending, eigenvector i is
-// column i of Z (row-major).  Returns false if the QL iteration does not
+// column i of Z (row-major), of which the rows from row0 on are computed.  Returns false if the QL iteration does not
 // converge (not observed for symmetric input).
-bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<double>& Z)
+bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<double>& Z, int row0)
 {
+    const int nr = n - row0;  // rows of Z
     auto a = [&](int i, int j) -> double& { return A[(size_t)i * n + j]; };
-    Z.assign((size_t)n * n, 0.0);
-    for (int i = 0; i < n; ++i) Z[(size_t)i * n + i] = 1.0;
+    Z.assign((size_t)nr * n, 0.0);
+    for (int i = 0; i < nr; ++i) Z[(size_t)i * n + row0 + i] = 1.0;
     std::vector<double> v(n), p(n), q(n);
     // --- Householder: column k below the subdiagonal is reflected onto e_{k+1}
     for (int k = 0; k + 2 < n; ++k) {
@@ -55,7 +56,7 @@ bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<
         a(k, k + 1) = alpha;
         for (int i = k + 2; i < n; ++i) a(i, k) = a(k, i) = 0.0;
         // Z <- Z (I - 2 v v^T) on columns k+1..n-1
-        for (int r = 0; r < n; ++r) {
+        for (int r = 0; r < nr; ++r) {
             double s = 0.0;
             for (int j = k + 1; j < n; ++j) s += Z[(size_t)r * n + j] * v[j];
             s *= 2.0;
@@ -100,7 +101,7 @@ bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<
                 pshift = s * r;
                 d[i + 1] = g + pshift;
                 g = c * r - bb;
-                for (int k = 0; k < n; ++k) {
+                for (int k = 0; k < nr; ++k) {
                     double& zi = Z[(size_t)k * n + i];
                     double& zi1 = Z[(size_t)k * n + i + 1];
                     const double t = zi1;
@@ -118,10 +119,10 @@ bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<
     std::iota(idx.begin(), idx.end(), 0);
     std::sort(idx.begin(), idx.end(), [&](int x, int y) { return d[x] < d[y]; });
     w.resize(n);
-    std::vector<double> Zs((size_t)n * n);
+    std::vector<double> Zs((size_t)nr * n);
     for (int c = 0; c < n; ++c) {
         w[c] = d[idx[c]];
-        for (int r = 0; r < n; ++r) Zs[(size_t)r * n + c] = Z[(size_t)r * n + idx[c]];
+        for (int r = 0; r < nr; ++r) Zs[(size_t)r * n + c] = Z[(size_t)r * n + idx[c]];
     }
     Z.swap(Zs);
     return true;

@@ -521,9 +521,10 @@ size_t tiled_bytes(const hd_hamiltonian* h);
 // eigenvalues w, eigenvectors as the columns of Z (hd_lanczos.hip).
 void jacobi_eigh(int n, std::vector<double>& A, std::vector<double>& w, std::vector<double>& Z);
 // Householder + implicit QL, same contract (hd_eigsym.cpp); false if QL fails.
-bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<double>& Z);
+// Z holds the eigenvectors' rows from row0 on.
+bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<double>& Z, int row0 = 0);
 // Block thick-restart Lanczos for opts.block > 1 (hd_block.hip).
 int run_block_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* evals, hd_lanczos_stats* stats);
-int spmv_autotune(hd_hamiltonian* h);
+int spmv_autotune(hd_hamiltonian* h, int formats = 7);  // bit p: format p (hd_precision)
 void lanczos_state_free(hd_lanczos_state* s);
 }  // namespace hd

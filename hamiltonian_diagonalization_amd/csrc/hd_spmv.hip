@@ -276,8 +276,6 @@ static int default_precision(const hd_hamiltonian* h)
     return HD_F64;
 }
 
-// Times every lanes-per-row variant on the matrix (in its fastest resident
-// format) and keeps the fastest.
 // Plain streaming copy, 16 bytes per lane per iteration (the byte-counter
 // calibration kernel).
 __global__ void __launch_bounds__(256) k_stream_copy(const int4* __restrict__ src, int4* __restrict__ dst, int64_t n)
@@ -286,13 +284,29 @@ __global__ void __launch_bounds__(256) k_stream_copy(const int4* __restrict__ sr
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
 }
 
-int spmv_autotune(hd_hamiltonian* h)
+// Times every schedule on the requested formats of the matrix (bit p of `formats`:
+// format p) and keeps the fastest of each.
+constexpr int64_t kTuneNnz = (int64_t)1 << 22;
+
+int spmv_autotune(hd_hamiltonian* h, int formats)
 {
     if (h->storage == HD_STORAGE_MATRIX_FREE) {  // one kernel, nothing to choose
         h->lanes_per_row = 1;
         return HD_OK;
     }
-    // one schedule per resident value format, each timed on zero vectors
+    const bool have[3] = {h->d_val64 != nullptr, h->d_val32 != nullptr, h->d_code != nullptr};
+    // Below kTuneNnz entries a product is one short wave of blocks (N=8, 2S=21,
+    // 0.9M entries: 5.5 us with 32 lanes per row, 5.6-6.7 us with 16) and timing
+    // the nine schedules of a format costs 36 of them: lanes by the row length.
+    if (h->nnz < kTuneNnz) {
+        const double avg = h->dim ? (double)h->nnz / (double)h->dim : 0.0;
+        for (int prec = 0; prec < 3; ++prec)
+            if (have[prec] && (formats >> prec & 1)) h->spmv_sched[prec] = sched_for_lanes(avg > 24 ? 32 : 16);
+        const int si = h->spmv_sched[default_precision(h)];
+        if (formats >> default_precision(h) & 1) h->lanes_per_row = kScheds[si >= 0 ? si : pick_default_sched(h)].lpr;
+        return HD_OK;
+    }
+    // one schedule per requested resident value format, each timed on zero vectors
     const size_t es = 8 * (h->is_complex ? 2 : 1);
     void *x = nullptr, *y = nullptr;
     HD_CHECK(dalloc(&x, (size_t)h->dim * es, "autotune x"));
@@ -305,9 +319,8 @@ int spmv_autotune(hd_hamiltonian* h)
     HD_ENQ(q, hipMemsetAsync(x, 0, (size_t)h->dim * es, h->stream));
     st = q.status();
     EventTimer timer;
-    const bool have[3] = {h->d_val64 != nullptr, h->d_val32 != nullptr, h->d_code != nullptr};
     for (int prec = 0; prec < 3 && st == HD_OK; ++prec) {
-        if (!have[prec]) continue;
+        if (!have[prec] || !(formats >> prec & 1)) continue;
         float best = 1e30f;
         int best_s = pick_default_sched(h);
         for (int si = 0; si < kNumScheds && st == HD_OK; ++si) {
@@ -324,8 +337,9 @@ int spmv_autotune(hd_hamiltonian* h)
         }
         h->spmv_sched[prec] = best_s;
     }
-    h->lanes_per_row = kScheds[h->spmv_sched[default_precision(h)] >= 0 ? h->spmv_sched[default_precision(h)]
-                                                                        : pick_default_sched(h)].lpr;
+    if (formats >> default_precision(h) & 1)
+        h->lanes_per_row = kScheds[h->spmv_sched[default_precision(h)] >= 0 ? h->spmv_sched[default_precision(h)]
+                                                                            : pick_default_sched(h)].lpr;
     dfree(x);
     dfree(y);
     return st;

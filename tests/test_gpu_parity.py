@@ -509,3 +509,35 @@ def test_block_lanczos_user_start():
     say(r0, r1)
     assert abs(r1.evals[0] - r0.evals[0]) < 1e-10 * max(1, abs(r0.evals[0]))
     assert r1.matvecs <= 4 * 8
+
+
+@pytest.mark.parametrize("model,args,nev,tol", [
+    ("sphere", (3, 9, 1), 2, 1e-12),     # dim 10: the basis fills the space and breaks down
+    ("sphere", (4, 8, 2), 4, 1e-12),     # dim 11
+    ("sphere", (7, 20, 0), 3, 1e-10),    # dim 3370: one launch per step
+    ("sphere", (7, 18, 0), 3, 1e-12),    # passes at a third of the steps
+    ("sphere", (8, 20, 0), 4, 1e-10),    # above 4096: several launches per step
+    ("lattice", (5, 4, 6), 3, 1e-10),    # dim 1932 complex, a pass at nearly every step
+    ("lattice", (5, 5, 5), 3, 1e-10)])   # dim 2130 complex: several launches per step
+def test_lanczos_step_forms(model, args, nev, tol):
+    """The one-launch and the several-launch Lanczos steps on both sides of the
+    dimension where they change over, against ARPACK (LAPACK below 100 rows) on
+    the same CRS: eigenvalues to 1e-10, true residuals of the stored vectors,
+    and orthonormal vectors."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as sla
+    say("lanczos step forms", model, args)
+    b, t = models.sphere_problem(*args) if model == "sphere" else models.ofl_problem(*args)
+    h = hd.Hamiltonian(b, t, values=(hd.F64,))
+    rp, col, val = h.crs()
+    A = sp.csr_matrix((val, col, rp), shape=(b.dim, b.dim))
+    want = np.linalg.eigvalsh(A.toarray())[:nev] if b.dim < 100 else \
+        np.sort(sla.eigsh(A, k=nev, which="SA", ncv=60, tol=1e-13, return_eigenvectors=False))
+    r = h.lanczos(nev=nev, tol=tol, seed=3)
+    say(r)
+    assert r.converged
+    assert np.max(np.abs(r.evals - want) / np.maximum(1, np.abs(want))) < 1e-10
+    X = np.stack([h.eigenvector(i) for i in range(nev)], axis=1)
+    res = np.linalg.norm(A @ X - X * r.evals, axis=0) / np.maximum(1, np.abs(r.evals))
+    assert np.all(res <= 1.01 * tol + 1e-13)
+    assert np.max(np.abs(X.conj().T @ X - np.eye(nev))) < 1e-9
