@@ -660,8 +660,6 @@ __global__ void __launch_bounds__(256) k_tile_pack(const uint4* __restrict__ in,
 
 }  // namespace
 
-// Builds the layout with TG-row groups; HD_ERR_UNSUPPORTED when a group reads
-// more than kMaxLines distinct lines.
 // Chooses the block order of the tiled product (groups per XCD window) by
 // timing each candidate on zero vectors, one warm and three timed launches
 // each: the launch order, windows of 16, 64 and 256 groups per XCD, and one
@@ -704,6 +702,8 @@ static int tiled_pick_window(hd_hamiltonian* h)
     return st;
 }
 
+// Builds the layout with TG-row groups; HD_ERR_UNSUPPORTED when a group reads
+// more than kMaxLines distinct lines.
 template <int TG>
 static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
 {
@@ -820,7 +820,14 @@ static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
     h->tg_bytes = (size_t)h->tg_entries * entry_bytes + (size_t)h->tg_lines * 4 + (size_t)h->tg_offs * 4 +
                   base.size() * 8 + (size_t)h->dim * 8 * W;
     h->bytes += h->tg_bytes;
-    return tiled_pick_window(h);
+    // Block order: 64 groups per XCD and window once every XCD has such a run.  It was
+    // the fastest of the five candidates at N=12, 2S=33 (3.360 ms; 3.366 with 16,
+    // 3.372 with 256, 3.407 in launch order) and on the 6x5 lattice, and timing them
+    // all took 65 of the 190 ms from a new set of tables to the first product at
+    // N=12, 2S=33.  Smaller grids are resident at once, so their order is free.
+    // hd_ham_tile_order(h, -1) times the candidates.
+    h->tg_win = G >= kXcds * 64 ? 64 : 0;
+    return HD_OK;
 }
 
 int tiled_build(hd_hamiltonian* h, int rows_per_group, int entry_bytes)

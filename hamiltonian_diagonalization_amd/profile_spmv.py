@@ -54,7 +54,7 @@ def main():
             out["orders"][w] = ms
             print(f"[profile] tiled block order {w} groups per XCD: {ms:.3f} ms", flush=True)
         ham.tile_order(chosen)
-        print(f"[profile] autotuned order: {chosen}", flush=True)
+        print(f"[profile] order of the layout: {chosen}", flush=True)
     # the other entry width of the tiled layout (4-byte entries always build; 3-byte ones need a
     # real dictionary of at most 2047 values)
     if not args.ofl:

@@ -6,8 +6,7 @@ python -m hamiltonian_diagonalization_amd.profile_stages [--n 12 --two-s 33 --it
 Stages, in order, on the N=12, 2S=33, L_z=0 Coulomb sphere sector
 (dim 7,764,392): the basis (k_unrank), the full-storage build with FP64,
 FP32 and coded values (k_count, the scan, k_fill_sorted), the tiled layout
-(k_tile_count, k_tile_fill, k_tile_pack for 3-byte entries, then its
-block-order autotune), `iters` tiled products with FP64 x and with FP32 x (one
+(k_tile_count, k_tile_fill, k_tile_pack for 3-byte entries), `iters` tiled products with FP64 x and with FP32 x (one
 warm-up each), the amplitude network over the whole sector (k_mlp_infer and
 the normalisation kernels), and the plain streaming copy over 1 GiB `iters`
 times, which calibrates FETCH_SIZE / WRITE_SIZE against a known byte count.
