@@ -56,6 +56,31 @@ struct GemmArgs {
     __bf16* HT; int ldht;       // BF16 output, transposed (nullable)
 };
 
+// acc += A . B^T over K columns (a multiple of 16) from a lane's operand addresses.
+// Eight steps' loads are issued together: the grids leave few waves per CU, so
+// a step that waited for its own loads cost a memory latency.
+HD_DEV f32x16 mfma_strip(const __bf16* pa, const __bf16* pb, int K, f32x16 acc)
+{
+    constexpr int U = 8;
+    int k = 0;
+    for (; k + 16 * U <= K; k += 16 * U) {
+        bf16x8 a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            a[u] = *reinterpret_cast<const bf16x8*>(pa + k + 16 * u);
+            b[u] = *reinterpret_cast<const bf16x8*>(pb + k + 16 * u);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], b[u], acc, 0, 0, 0);
+    }
+    for (; k < K; k += 16) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(pa + k);
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(pb + k);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+    }
+    return acc;
+}
+
 // M, N multiples of 64, K a multiple of 16 (buffers are padded by the callers).
 template <int EPI>
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
@@ -67,11 +92,7 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
     const __bf16* pa = g.A + (size_t)(m0 + r) * g.lda + kh;
     const __bf16* pb = g.B + (size_t)(n0 + r) * g.ldb + kh;
     f32x16 acc = {};
-    for (int k0 = 0; k0 < g.K; k0 += 16) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(pa + k0);
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(pb + k0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
+    acc = mfma_strip(pa, pb, g.K, acc);
     const int col = n0 + r;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -87,58 +108,70 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g)
     }
 }
 
-// Input features: occupations of n_bits orbitals, then n_params parameters.
-__global__ void k_featurize(int64_t n, int64_t npad, const uint64_t* __restrict__ states,
+// Input features: occupations of n_bits orbitals, then n_params parameters.  A
+// thread makes eight columns of one state: 16 bytes of the row-major copy, and
+// two bytes in each of eight rows of the transposed one, neighbouring states
+// side by side (32 states x 8 column groups per block).
+__global__ void __launch_bounds__(256) k_featurize(int64_t n, int64_t npad, const uint64_t* __restrict__ states,
                             const float* __restrict__ params, int per_sample, int n_bits, int n_params,
                             __bf16* __restrict__ H0, __bf16* __restrict__ H0T)
 {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t b = (int64_t)blockIdx.x * 32 + (threadIdx.x & 31);
+    const int k0 = (threadIdx.x >> 5) * 8;
     if (b >= npad) return;
     const bool live = b < n;
     const uint64_t s = live ? states[b] : 0ull;
     const float* p = params + (per_sample ? b * n_params : 0);
-    for (int k = 0; k < kIn; ++k) {
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int k = k0 + j;
         float f = 0.f;
         if (live) {
             if (k < n_bits) f = (float)((s >> k) & 1ull);
             else if (k < n_bits + n_params) f = p[k - n_bits];
         }
-        H0[b * kIn + k] = (__bf16)f;
-        if (H0T) H0T[(size_t)k * npad + b] = (__bf16)f;
+        v[j] = (__bf16)f;
+        H0T[(size_t)k * npad + b] = v[j];
     }
+    *reinterpret_cast<bf16x8*>(H0 + b * kIn + k0) = v;
 }
 
 // loss and dL/dout for out = (log|psi_s|, sign logit_s), s < S, against
 // targets (log|psi_s|, sign_s, weight_s) per state (3 S floats per sample);
-// lambda weights the sign term.
-__global__ void k_loss(int64_t n, int64_t npad, int S, const float* __restrict__ out, const float* __restrict__ tgt,
+// lambda weights the sign term.  A thread takes four amplitudes (eight columns)
+// of one state, as k_featurize.
+__global__ void __launch_bounds__(256) k_loss(int64_t n, int64_t npad, int S, const float* __restrict__ out, const float* __restrict__ tgt,
                        float lambda, float inv_n, __bf16* __restrict__ d4, __bf16* __restrict__ d4T,
                        float* __restrict__ partial)
 {
     __shared__ float red[256];
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t b = (int64_t)blockIdx.x * 32 + (threadIdx.x & 31);
+    const int c0 = (threadIdx.x >> 5) * 8;
     float l = 0.f;
     if (b < npad) {
-        for (int c = 0; c < kOutPad; ++c) {
-            const int st = c >> 1;
-            float g = 0.f;
+        bf16x8 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int st = (c0 >> 1) + j;
+            float g0 = 0.f, g1 = 0.f;
             if (b < n && st < S) {
                 const float o0 = out[b * kOutPad + 2 * st], o1 = out[b * kOutPad + 2 * st + 1];
                 const float* t = tgt + (b * S + st) * 3;
                 const float a = t[0], sg = t[1], w = t[2];
                 const float e = o0 - a;
                 const float m = -sg * o1;  // softplus(m) = log(1 + exp(-s o1))
-                if (c & 1) {
-                    g = -lambda * w * sg * (1.f / (1.f + __expf(-m))) * inv_n;
-                } else {
-                    const float sp = m > 20.f ? m : log1pf(__expf(m));
-                    l += w * (e * e + lambda * sp) * inv_n;
-                    g = 2.f * w * e * inv_n;
-                }
+                const float sp = m > 20.f ? m : log1pf(__expf(m));
+                l += w * (e * e + lambda * sp) * inv_n;
+                g0 = 2.f * w * e * inv_n;
+                g1 = -lambda * w * sg * (1.f / (1.f + __expf(-m))) * inv_n;
             }
-            d4[b * kOutPad + c] = (__bf16)g;
-            d4T[(size_t)c * npad + b] = (__bf16)g;
+            v[2 * j] = (__bf16)g0;
+            v[2 * j + 1] = (__bf16)g1;
         }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) d4T[(size_t)(c0 + j) * npad + b] = v[j];
+        *reinterpret_cast<bf16x8*>(d4 + b * kOutPad + c0) = v;
     }
     red[threadIdx.x] = l;
     __syncthreads();
@@ -149,46 +182,116 @@ __global__ void k_loss(int64_t n, int64_t npad, int S, const float* __restrict__
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// db[c] = sum_b dT[c][b] (one block per output channel, fixed-order tree).
-__global__ void k_bias_grad(const __bf16* __restrict__ dT, int64_t npad, float* __restrict__ db)
+// The parameters, their moments and gradients are flat arrays in the order of
+// hd_mlp_get_weights: per layer W (rows x cols, padded shape), then b.
+constexpr int kRows[4] = {kW, kW, kW, kOutPad};
+constexpr int kCols[4] = {kIn, kW, kW, kW};
+HD_DEV constexpr int rows_of(int l) { return l == 3 ? kOutPad : kW; }
+HD_DEV constexpr int cols_of(int l) { return l == 0 ? kIn : kW; }
+constexpr int kOff[5] = {0, kW * kIn + kW, kW * kIn + kW + kW * kW + kW, kW * kIn + kW + 2 * (kW * kW + kW),
+                         kW * kIn + kW + 2 * (kW * kW + kW) + kOutPad * kW + kOutPad};
+constexpr int kParams = kOff[4];
+HD_DEV constexpr int off_of(int l)
 {
-    __shared__ float red[256];
-    const int c = blockIdx.x;
-    float s = 0.f;
-    for (int64_t b = threadIdx.x; b < npad; b += 256) s += (float)dT[(size_t)c * npad + b];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
+    return l == 0 ? 0 : l == 1 ? kW * kIn + kW : l == 2 ? kW * kIn + kW + kW * kW + kW : kW * kIn + kW + 2 * (kW * kW + kW);
+}
+
+// Weight and bias gradients of all layers, dW_l = d_{l+1}^T h_l and db_l = sum d_{l+1},
+// split over the batch: block (t, z) adds the samples [z kc, (z+1) kc) of one 64 x 64
+// tile into part[z].  A batch of 4,096 gives 40 tiles, 16 for the largest layer alone:
+// unsplit, 16 blocks walked 256 K-steps each (66 us per layer); split 16 ways the four
+// layers take 18 us together.
+struct WgradArgs {
+    const __bf16* dT[4];  // [rows][M]
+    const __bf16* hT[4];  // [cols][M]
+    int64_t M;
+    int kc;
+    float* part;
+};
+constexpr int kWgradTiles = 4 + 16 + 16 + 4;
+constexpr int kMaxSplits = 16;
+
+__global__ void __launch_bounds__(256) k_wgrad(WgradArgs g)
+{
+    int t = blockIdx.x, l = 0;
+    if (t >= 36) { l = 3; t -= 36; }
+    else if (t >= 20) { l = 2; t -= 20; }
+    else if (t >= 4) { l = 1; t -= 4; }
+    const int cols = cols_of(l), nt = cols / 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m0 = (t / nt) * 64 + (wave >> 1) * 32, n0 = (t % nt) * 64 + (wave & 1) * 32;
+    const int r = lane & 31, kh = (lane >> 5) * 8;
+    const int64_t k0 = (int64_t)blockIdx.y * g.kc, k1 = min(k0 + g.kc, g.M);
+    const __bf16* pa = g.dT[l] + (size_t)(m0 + r) * g.M + kh;
+    const __bf16* pb = g.hT[l] + (size_t)(n0 + r) * g.M + kh;
+    const bool bias = n0 == 0;
+    f32x16 acc = {};
+    float bs = 0.f;
+    const int K = (int)(k1 - k0);
+    acc = mfma_strip(pa + k0, pb + k0, K, acc);
+    if (bias)
+        for (int k = 0; k < K; k += 16) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(pa + k0 + k);
+            bs += (((float)a[0] + (float)a[1]) + ((float)a[2] + (float)a[3])) +
+                  (((float)a[4] + (float)a[5]) + ((float)a[6] + (float)a[7]));
+        }
+    float* w = g.part + (size_t)blockIdx.y * kParams + off_of(l);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w[(m0 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)) * cols + n0 + r] = acc[i];
+    if (bias) {
+        bs += __shfl_xor(bs, 32, 64);
+        if (lane < 32) w[rows_of(l) * cols + m0 + r] = bs;
     }
-    if (threadIdx.x == 0) db[c] = red[0];
 }
 
-// Adam (Kingma and Ba, ICLR 2015) on the FP32 master copy.
-__global__ void k_adam(int64_t n, float* __restrict__ w, const float* __restrict__ gr, float* __restrict__ m,
-                       float* __restrict__ v, float lr, float b1, float b2, float c1, float c2, float eps)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float g = gr[i];
-    const float mi = b1 * m[i] + (1.f - b1) * g;
-    const float vi = b2 * v[i] + (1.f - b2) * g * g;
-    m[i] = mi;
-    v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
+// One pass over all parameters.  GRAD: the splits' partial gradients summed in
+// order.  STEP: Adam (Kingma and Ba, ICLR 2015) on the FP32 master copy.  COPY: the
+// BF16 copies W, W^T and, for inference, the fragment order.  One launch instead
+// of four bias sums, eight Adam launches, four conversions and a packing.
+struct ParamArgs {
+    const float* part;
+    int splits;
+    float *w, *g, *m, *v;
+    float lr, b1, b2, c1, c2, eps;
+    __bf16* wb[4];
+    __bf16* wbT[4];
+    __bf16* wf;
+};
 
-// BF16 copies W (rows x cols) and W^T from the FP32 master.
-__global__ void k_to_bf16(int rows, int cols, const float* __restrict__ w, __bf16* __restrict__ wb,
-                          __bf16* __restrict__ wbT)
+template <bool GRAD, bool STEP, bool COPY>
+__global__ void __launch_bounds__(256) k_params(ParamArgs a)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * cols) return;
-    const int r = i / cols, c = i % cols;
-    const __bf16 v = (__bf16)w[i];
-    wb[i] = v;
-    wbT[(size_t)c * rows + r] = v;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= kParams) return;
+    float gr = 0.f;
+    if (GRAD) {
+        for (int z = 0; z < a.splits; ++z) gr += a.part[(size_t)z * kParams + i];
+        a.g[i] = gr;
+    }
+    float w = a.w[i];
+    if (STEP) {
+        const float mi = a.b1 * a.m[i] + (1.f - a.b1) * gr;
+        const float vi = a.b2 * a.v[i] + (1.f - a.b2) * gr * gr;
+        a.m[i] = mi;
+        a.v[i] = vi;
+        w -= a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+        a.w[i] = w;
+    }
+    if (COPY) {
+        const int l = i >= off_of(3) ? 3 : i >= off_of(2) ? 2 : i >= off_of(1) ? 1 : 0;
+        const int q = i - off_of(l), cols = cols_of(l), rows = rows_of(l);
+        if (q >= rows * cols) return;  // a bias
+        const int r = q / cols, k = q % cols;
+        const __bf16 v = (__bf16)w;
+        a.wb[l][q] = v;
+        a.wbT[l][(size_t)k * rows + r] = v;
+        // fragment f = tile * (K/16) + k/16 of each layer in turn, lane's eight
+        // values W[32 tile + lane%32][16 (k/16) + 8 (lane/32) ..+7]; of the last layer
+        // the first 32 rows
+        const int base = l == 0 ? 0 : l == 1 ? 32 : l == 2 ? 160 : 288;
+        if (r < (l == 3 ? 32 : kW))
+            a.wf[(size_t)(base + (r >> 5) * (cols >> 4) + (k >> 4)) * 512 + ((r & 31) + ((k >> 3) & 1) * 32) * 8 + (k & 7)] = v;
+    }
 }
 
 // ---------------------------------------------------------------- inference
@@ -201,7 +304,7 @@ __global__ void k_to_bf16(int rows, int cols, const float* __restrict__ w, __bf1
 // every 16 change lane halves (v_permlane32_swap).  Every output is the MFMA
 // sequence of k_gemm (32x32x16 tiles, K ascending in steps of 16).
 //
-// The weights are read in the order of the A fragments (k_pack_infer: 1 KiB per
+// The weights are read in the order of the A fragments (k_params: 1 KiB per
 // 32 x 16 fragment, lane l's 16 bytes at 16 l), ten chunks of 32 fragments
 // (layer 1 in one, layers 2 and 3 in four each, the output layer in the last),
 // double-buffered in LDS: the next chunk's loads are in flight into registers
@@ -232,25 +335,6 @@ struct InferArgs {
     float* out;           // n x n_out
     float* partial_max;   // per workgroup and amplitude s: largest output 2s over its states
 };
-
-// Fragment-ordered copy of the four layers: fragment f = tile * (K/16) + k/16 of
-// each layer in turn, lane l's eight values W[32 tile + l%32][16 (k/16) + 8 (l/32) ..+7].
-__global__ void __launch_bounds__(256) k_pack_infer(const float* __restrict__ w0, const float* __restrict__ w1,
-                                                    const float* __restrict__ w2, const float* __restrict__ w3,
-                                                    __bf16* __restrict__ wf)
-{
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= kChunks * kChunk) return;
-    const int frag = e / kFrag, lane = (e % kFrag) >> 3, j = e & 7;
-    const float* w = w0;
-    int f = frag, ks = kIn / 16;
-    if (frag >= 288) { w = w3; f = frag - 288; ks = kW / 16; }
-    else if (frag >= 160) { w = w2; f = frag - 160; ks = kW / 16; }
-    else if (frag >= 32) { w = w1; f = frag - 32; ks = kW / 16; }
-    const int row = (f / ks) * 32 + (lane & 31), k = (f % ks) * 16 + (lane >> 5) * 8 + j;
-    // the last chunk is half used: the output tile's 16 fragments
-    wf[e] = frag >= 304 ? (__bf16)0.f : (__bf16)w[row * (ks * 16) + k];
-}
 
 // z / (1 + exp(-z)) with the quotient from v_rcp_f32 and one correction step (the
 // remainder z - q d, exact in the fma), instead of the IEEE division sequence; the
@@ -571,17 +655,12 @@ struct hd_mlp {
     int n_bits = 0, n_params = 0;
     int n_states = 1;  // amplitudes the network predicts (2 outputs each)
     hipStream_t stream = nullptr;
-    // layer l: out_l x in_l ; l = 0..3 with padded shapes
-    int rows[4] = {kW, kW, kW, kOutPad};
-    int cols[4] = {kIn, kW, kW, kW};
     int live_rows[4] = {kW, kW, kW, 2};
-    float* w[4] = {};     // FP32 master (padded shape, padding kept at zero)
-    float* b[4] = {};
+    // flat arrays of kParams: FP32 master (padding kept at zero), gradients, Adam moments
+    float *params = nullptr, *grads = nullptr, *mom1 = nullptr, *mom2 = nullptr;
     __bf16* wb[4] = {};   // BF16 copy
     __bf16* wbT[4] = {};  // BF16 transposed copy
     __bf16* wf = nullptr; // BF16 copy in the inference kernel's fragment order
-    float *mw[4] = {}, *vw[4] = {}, *mb[4] = {}, *vb[4] = {};  // Adam moments
-    float *gw[4] = {}, *gb[4] = {};
     int64_t step = 0;
     // work buffers for a batch of `cap` rows
     int64_t cap = 0;
@@ -590,6 +669,7 @@ struct hd_mlp {
     float* out = nullptr;            // npad x 64
     __bf16 *d[5] = {}, *dT[5] = {};  // deltas: d[4] output layer, d[3..1] hidden
     float* partial = nullptr;
+    float* wpart = nullptr;          // kMaxSplits x kParams partial gradients
     uint64_t* st_buf = nullptr;      // staging for host-provided batches
     float* pr_buf = nullptr;
     float* tg_buf = nullptr;
@@ -609,9 +689,10 @@ void mlp_free_work(hd_mlp* m)
         dfree(m->d[l]); dfree(m->dT[l]);
         m->d[l] = m->dT[l] = nullptr;
     }
-    dfree(m->out); dfree(m->partial);
+    dfree(m->out); dfree(m->partial); dfree(m->wpart);
     m->out = nullptr;
     m->partial = nullptr;
+    m->wpart = nullptr;
     m->cap = 0;
 }
 
@@ -626,8 +707,9 @@ int mlp_work(hd_mlp* m, int64_t npad, bool train)
         HD_CHECK(dalloc_t(&m->z[l], (size_t)c * kW, "MLP pre-activations"));
     }
     HD_CHECK(dalloc_t(&m->out, (size_t)c * kOutPad, "MLP output"));
-    HD_CHECK(dalloc_t(&m->partial, (size_t)(c / 256 + 1024), "MLP partials"));
+    HD_CHECK(dalloc_t(&m->partial, (size_t)(c / 32 + 1024), "MLP partials"));
     if (train) {
+        HD_CHECK(dalloc_t(&m->wpart, (size_t)kMaxSplits * kParams, "MLP partial gradients"));
         HD_CHECK(dalloc_t(&m->hT[0], (size_t)c * kIn, "MLP features^T"));
         for (int l = 1; l < 4; ++l) HD_CHECK(dalloc_t(&m->hT[l], (size_t)c * kW, "MLP activations^T"));
         HD_CHECK(dalloc_t(&m->d[4], (size_t)c * kOutPad, "MLP output delta"));
@@ -641,15 +723,27 @@ int mlp_work(hd_mlp* m, int64_t npad, bool train)
     return HD_OK;
 }
 
+ParamArgs param_args(const hd_mlp* m, int splits)
+{
+    ParamArgs a{};
+    a.part = m->wpart;
+    a.splits = splits;
+    a.w = m->params;
+    a.g = m->grads;
+    a.m = m->mom1;
+    a.v = m->mom2;
+    for (int l = 0; l < 4; ++l) {
+        a.wb[l] = m->wb[l];
+        a.wbT[l] = m->wbT[l];
+    }
+    a.wf = m->wf;
+    return a;
+}
+const dim3 kParamGrid((kParams + 255) / 256);
+
 int mlp_refresh_bf16(hd_mlp* m)
 {
-    for (int l = 0; l < 4; ++l) {
-        const int n = m->rows[l] * m->cols[l];
-        hipLaunchKernelGGL(k_to_bf16, dim3((n + 255) / 256), dim3(256), 0, m->stream, m->rows[l], m->cols[l], m->w[l],
-                           m->wb[l], m->wbT[l]);
-    }
-    hipLaunchKernelGGL(k_pack_infer, dim3(kChunks * kChunk / 256), dim3(256), 0, m->stream, m->w[0], m->w[1], m->w[2],
-                       m->w[3], m->wf);
+    hipLaunchKernelGGL((k_params<false, false, true>), kParamGrid, dim3(256), 0, m->stream, param_args(m, 0));
     HD_HIP(hipGetLastError());
     return HD_OK;
 }
@@ -684,7 +778,7 @@ InferArgs infer_args(const hd_mlp* m, int64_t n, const uint64_t* states, const f
     a.n_bits = m->n_bits;
     a.n_params = m->n_params;
     a.wf = m->wf;
-    for (int l = 0; l < 4; ++l) a.b[l] = m->b[l];
+    for (int l = 0; l < 4; ++l) a.b[l] = m->params + kOff[l] + kRows[l] * kCols[l];
     a.n_out = m->live_rows[3];
     a.out = out;
     a.partial_max = partial_max;
@@ -697,52 +791,57 @@ void mlp_forward_core(hd_mlp* m, int64_t npad, bool train)
     const int M = (int)npad;
     for (int l = 0; l < 3; ++l) {
         const int K = l == 0 ? kIn : kW;
-        GemmArgs g = ga(M, kW, K, m->h[l], K, m->wb[l], m->cols[l]);
+        GemmArgs g = ga(M, kW, K, m->h[l], K, m->wb[l], kCols[l]);
         g.C = m->z[l + 1]; g.ldc = kW;
-        g.bias = m->b[l];
+        g.bias = m->params + kOff[l] + kRows[l] * kCols[l];
         g.H = m->h[l + 1]; g.ldh = kW;
         if (train) { g.HT = m->hT[l + 1]; g.ldht = M; }
         gemm(m->stream, EPI_BIAS_SILU, g);
     }
     GemmArgs g = ga(M, kOutPad, kW, m->h[3], kW, m->wb[3], kW);
     g.C = m->out; g.ldc = kOutPad;
-    g.bias = m->b[3];
+    g.bias = m->params + kOff[3] + kRows[3] * kCols[3];
     gemm(m->stream, EPI_BIAS, g);
 }
 
-// gradients of the loss into gw/gb; returns the loss
-int mlp_backward(hd_mlp* m, int64_t n, int64_t npad, const float* d_tgt, float lambda, float* loss)
+// partial gradients of the loss into wpart (*splits of them); the per-block losses
+// into `partial`
+int mlp_backward(hd_mlp* m, int64_t n, int64_t npad, const float* d_tgt, float lambda, int* splits)
 {
     const hipStream_t st = m->stream;
     const int M = (int)npad;
-    const int nblk = (int)((npad + 255) / 256);
-    hipLaunchKernelGGL(k_loss, dim3(nblk), dim3(256), 0, st, n, npad, m->n_states, m->out, d_tgt, lambda, 1.f / (float)n,
-                       m->d[4], m->dT[4], m->partial);
-    // dW4 = d4^T h3 ; db4
-    {
-        GemmArgs g = ga(kOutPad, kW, M, m->dT[4], M, m->hT[3], M);
-        g.C = m->gw[3]; g.ldc = kW;
-        gemm(st, EPI_STORE, g);
-        hipLaunchKernelGGL(k_bias_grad, dim3(kOutPad), dim3(256), 0, st, m->dT[4], npad, m->gb[3]);
-    }
-    // hidden layers l = 3, 2, 1: d_l = (d_{l+1} W_{l+1}) * silu'(z_l); dW_l = d_l^T h_{l-1}
+    hipLaunchKernelGGL(k_loss, dim3((unsigned)((npad + 31) / 32)), dim3(256), 0, st, n, npad, m->n_states, m->out, d_tgt,
+                       lambda, 1.f / (float)n, m->d[4], m->dT[4], m->partial);
+    // hidden layers l = 3, 2, 1: d_l = (d_{l+1} W_{l+1}) * silu'(z_l)
     for (int l = 3; l >= 1; --l) {
         const int Kd = l == 3 ? kOutPad : kW;  // width of d_{l+1}
-        GemmArgs g = ga(M, kW, Kd, m->d[l + 1 == 4 ? 4 : l + 1], Kd, m->wbT[l], m->rows[l]);
+        GemmArgs g = ga(M, kW, Kd, m->d[l + 1], Kd, m->wbT[l], kRows[l]);
         g.zin = m->z[l]; g.ldz = kW;
         g.H = m->d[l]; g.ldh = kW;
         g.HT = m->dT[l]; g.ldht = M;
         gemm(st, EPI_DSILU, g);
-        const int K_in = l == 1 ? kIn : kW;
-        GemmArgs gw = ga(kW, K_in, M, m->dT[l], M, m->hT[l - 1], M);
-        gw.C = m->gw[l - 1]; gw.ldc = K_in;
-        gemm(st, EPI_STORE, gw);
-        hipLaunchKernelGGL(k_bias_grad, dim3(kW), dim3(256), 0, st, m->dT[l], npad, m->gb[l - 1]);
     }
+    WgradArgs w{};
+    for (int l = 0; l < 4; ++l) {
+        w.dT[l] = m->dT[l + 1];
+        w.hT[l] = m->hT[l];
+    }
+    w.M = npad;
+    // at least 64 samples per block, a multiple of 16
+    w.kc = (int)std::max<int64_t>(64, ((npad + kMaxSplits - 1) / kMaxSplits + 15) / 16 * 16);
+    w.part = m->wpart;
+    *splits = (int)((npad + w.kc - 1) / w.kc);
+    hipLaunchKernelGGL(k_wgrad, dim3(kWgradTiles, *splits), dim3(256), 0, st, w);
     HD_HIP(hipGetLastError());
-    std::vector<float> part(nblk);
-    HD_HIP(hipMemcpyAsync(part.data(), m->partial, sizeof(float) * nblk, hipMemcpyDeviceToHost, st));
-    HD_HIP(hipStreamSynchronize(st));
+    return HD_OK;
+}
+
+// The loss of the batch, after everything enqueued.
+int mlp_loss(hd_mlp* m, int64_t npad, float* loss)
+{
+    std::vector<float> part((size_t)((npad + 31) / 32));
+    HD_HIP(hipMemcpyAsync(part.data(), m->partial, sizeof(float) * part.size(), hipMemcpyDeviceToHost, m->stream));
+    HD_HIP(hipStreamSynchronize(m->stream));
     double s = 0.0;
     for (float p : part) s += p;
     if (loss) *loss = (float)s;
@@ -779,8 +878,9 @@ int stage_batch(hd_mlp* m, const uint64_t* states, const float* params, const fl
 
 int64_t pad64(int64_t n) { return (n + 63) / 64 * 64; }
 
-int gradients_impl(hd_mlp* m, const uint64_t* states, const float* params, const float* tgt, int64_t n, float lambda,
-                   int host, float* loss)
+// forward and backward passes of a batch, up to the partial gradients
+int batch_pass(hd_mlp* m, const uint64_t* states, const float* params, const float* tgt, int64_t n, float lambda,
+               int host, int* splits)
 {
     if (n <= 0) return fail(HD_ERR_ARG, "empty batch");
     const int64_t npad = pad64(n);
@@ -788,10 +888,10 @@ int gradients_impl(hd_mlp* m, const uint64_t* states, const float* params, const
     const uint64_t* ds;
     const float *dp, *dt;
     HD_CHECK(stage_batch(m, states, params, tgt, n, host != 0, &ds, &dp, &dt, 1));
-    hipLaunchKernelGGL(k_featurize, dim3((unsigned)((npad + 255) / 256)), dim3(256), 0, m->stream, n, npad, ds, dp, 1,
-                       m->n_bits, m->n_params, m->h[0], m->hT[0]);
+    hipLaunchKernelGGL(k_featurize, dim3((unsigned)(npad / 32)), dim3(256), 0, m->stream, n, npad, ds, dp, 1, m->n_bits,
+                       m->n_params, m->h[0], m->hT[0]);
     mlp_forward_core(m, npad, true);
-    return mlp_backward(m, n, npad, dt, lambda, loss);
+    return mlp_backward(m, n, npad, dt, lambda, splits);
 }
 
 }  // namespace
@@ -821,36 +921,29 @@ int hd_mlp_create_states(int32_t n_bits, int32_t n_params, int32_t n_states, uin
     std::mt19937_64 rng(seed);
     int st = HD_OK;
     HipErrors q;
+    for (float** p : {&m->params, &m->grads, &m->mom1, &m->mom2})
+        if (st == HD_OK) st = dalloc_t(p, (size_t)kParams, "MLP parameters");
+    std::vector<float> flat(kParams, 0.f);
     for (int l = 0; l < 4 && st == HD_OK; ++l) {
-        const int R = m->rows[l], C = m->cols[l];
-        const size_t n = (size_t)R * C;
-        std::vector<float> w(n, 0.f), bz(R, 0.f);
+        const int R = kRows[l], C = kCols[l];
+        float* w = flat.data() + kOff[l];
         // He-normal over the live fan-in (n_bits + n_params for the first layer)
         const int fan_in = l == 0 ? n_bits + n_params : kW;
         std::normal_distribution<float> nd(0.f, std::sqrt(2.f / (float)fan_in) * (l == 3 ? 0.1f : 1.f));
         for (int r = 0; r < m->live_rows[l]; ++r)
             for (int c = 0; c < (l == 0 ? fan_in : C); ++c) w[(size_t)r * C + c] = nd(rng);
-        if ((st = dalloc_t(&m->w[l], n, "MLP weights")) != HD_OK) break;
-        if ((st = dalloc_t(&m->b[l], R, "MLP biases")) != HD_OK) break;
-        if ((st = dalloc_t(&m->wb[l], n, "MLP bf16 weights")) != HD_OK) break;
-        if ((st = dalloc_t(&m->wbT[l], n, "MLP bf16 weights^T")) != HD_OK) break;
-        if ((st = dalloc_t(&m->gw[l], n, "MLP weight grads")) != HD_OK) break;
-        if ((st = dalloc_t(&m->gb[l], R, "MLP bias grads")) != HD_OK) break;
-        for (float** p : {&m->mw[l], &m->vw[l]})
-            if ((st = dalloc_t(p, n, "Adam moments")) != HD_OK) break;
-        for (float** p : {&m->mb[l], &m->vb[l]})
-            if ((st = dalloc_t(p, R, "Adam moments")) != HD_OK) break;
-        if (st != HD_OK) break;
-        // synchronous copies: w and bz are released at the end of this iteration
-        HD_ENQ(q, hipMemcpy(m->w[l], w.data(), n * 4, hipMemcpyHostToDevice));
-        HD_ENQ(q, hipMemcpy(m->b[l], bz.data(), (size_t)R * 4, hipMemcpyHostToDevice));
-        HD_ENQ(q, hipMemsetAsync(m->mw[l], 0, n * 4, m->stream));
-        HD_ENQ(q, hipMemsetAsync(m->vw[l], 0, n * 4, m->stream));
-        HD_ENQ(q, hipMemsetAsync(m->mb[l], 0, (size_t)R * 4, m->stream));
-        HD_ENQ(q, hipMemsetAsync(m->vb[l], 0, (size_t)R * 4, m->stream));
+        if ((st = dalloc_t(&m->wb[l], (size_t)R * C, "MLP bf16 weights")) != HD_OK) break;
+        if ((st = dalloc_t(&m->wbT[l], (size_t)R * C, "MLP bf16 weights^T")) != HD_OK) break;
+    }
+    if (st == HD_OK) {
+        HD_ENQ(q, hipMemcpy(m->params, flat.data(), sizeof(float) * kParams, hipMemcpyHostToDevice));
+        HD_ENQ(q, hipMemsetAsync(m->mom1, 0, sizeof(float) * kParams, m->stream));
+        HD_ENQ(q, hipMemsetAsync(m->mom2, 0, sizeof(float) * kParams, m->stream));
     }
     if (st == HD_OK) st = q.status();
     if (st == HD_OK) st = dalloc_t(&m->wf, (size_t)kChunks * kChunk, "MLP packed weights");
+    if (st == HD_OK && hipMemsetAsync(m->wf, 0, sizeof(__bf16) * kChunks * kChunk, m->stream) != hipSuccess)
+        st = fail(HD_ERR_HIP, "MLP init failed");  // its last half chunk is padding
     if (st == HD_OK) st = mlp_refresh_bf16(m);
     if (st == HD_OK && hipStreamSynchronize(m->stream) != hipSuccess) st = fail(HD_ERR_HIP, "MLP init failed");
     if (st != HD_OK) {
@@ -868,10 +961,10 @@ int hd_mlp_destroy(hd_mlp* m)
     if (!m) return HD_OK;
     mlp_free_work(m);
     for (int l = 0; l < 4; ++l) {
-        for (void* p : {(void*)m->w[l], (void*)m->b[l], (void*)m->wb[l], (void*)m->wbT[l], (void*)m->gw[l],
-                        (void*)m->gb[l], (void*)m->mw[l], (void*)m->vw[l], (void*)m->mb[l], (void*)m->vb[l]})
-            dfree(p);
+        dfree(m->wb[l]);
+        dfree(m->wbT[l]);
     }
+    for (float* p : {m->params, m->grads, m->mom1, m->mom2}) dfree(p);
     dfree(m->st_buf); dfree(m->pr_buf); dfree(m->tg_buf); dfree(m->wf);
     if (m->stream) stream_put(m->stream);
     delete m;
@@ -881,30 +974,14 @@ int hd_mlp_destroy(hd_mlp* m)
 int hd_mlp_num_weights(const hd_mlp* m, int64_t* count)
 {
     if (!m || !count) return fail(HD_ERR_ARG, "null argument");
-    int64_t c = 0;
-    for (int l = 0; l < 4; ++l) c += (int64_t)m->rows[l] * m->cols[l] + m->rows[l];
-    *count = c;
+    *count = kParams;
     return HD_OK;
 }
 
 // Flat FP32 layout: for each layer, W (rows x cols, padded shape) then b.
-static int copy_params(hd_mlp* m, float* h, bool to_host, bool grads)
+static int copy_to_host(hd_mlp* m, float* h, const float* d)
 {
-    size_t off = 0;
-    for (int l = 0; l < 4; ++l) {
-        const size_t n = (size_t)m->rows[l] * m->cols[l];
-        float* wsrc = grads ? m->gw[l] : m->w[l];
-        float* bsrc = grads ? m->gb[l] : m->b[l];
-        if (to_host) {
-            HD_HIP(hipMemcpyAsync(h + off, wsrc, n * 4, hipMemcpyDeviceToHost, m->stream));
-            HD_HIP(hipMemcpyAsync(h + off + n, bsrc, (size_t)m->rows[l] * 4, hipMemcpyDeviceToHost, m->stream));
-        } else {
-            HD_HIP(hipMemcpyAsync(wsrc, h + off, n * 4, hipMemcpyHostToDevice, m->stream));
-            HD_HIP(hipMemcpyAsync(bsrc, h + off + n, (size_t)m->rows[l] * 4, hipMemcpyHostToDevice, m->stream));
-        }
-        off += n + m->rows[l];
-    }
-    if (!to_host && !grads) HD_CHECK(mlp_refresh_bf16(m));
+    HD_HIP(hipMemcpyAsync(h, d, sizeof(float) * kParams, hipMemcpyDeviceToHost, m->stream));
     HD_HIP(hipStreamSynchronize(m->stream));
     return HD_OK;
 }
@@ -912,13 +989,16 @@ static int copy_params(hd_mlp* m, float* h, bool to_host, bool grads)
 int hd_mlp_get_weights(hd_mlp* m, float* h_out)
 {
     if (!m || !h_out) return fail(HD_ERR_ARG, "null argument");
-    return copy_params(m, h_out, true, false);
+    return copy_to_host(m, h_out, m->params);
 }
 
 int hd_mlp_set_weights(hd_mlp* m, const float* h_in)
 {
     if (!m || !h_in) return fail(HD_ERR_ARG, "null argument");
-    return copy_params(m, const_cast<float*>(h_in), false, false);
+    HD_HIP(hipMemcpyAsync(m->params, h_in, sizeof(float) * kParams, hipMemcpyHostToDevice, m->stream));
+    HD_CHECK(mlp_refresh_bf16(m));
+    HD_HIP(hipStreamSynchronize(m->stream));
+    return HD_OK;
 }
 
 int hd_mlp_forward(hd_mlp* m, const uint64_t* h_states, const float* h_params, int64_t n, float* h_out)
@@ -953,8 +1033,12 @@ int hd_mlp_gradients(hd_mlp* m, const uint64_t* h_states, const float* h_params,
                      float lambda, float* loss, float* h_grads)
 {
     if (!m || !h_states || !h_params || !h_targets || n <= 0) return fail(HD_ERR_ARG, "hd_mlp_gradients: bad argument");
-    HD_CHECK(gradients_impl(m, h_states, h_params, h_targets, n, lambda, 1, loss));
-    if (h_grads) HD_CHECK(copy_params(m, h_grads, true, true));
+    int splits = 0;
+    HD_CHECK(batch_pass(m, h_states, h_params, h_targets, n, lambda, 1, &splits));
+    hipLaunchKernelGGL((k_params<true, false, false>), kParamGrid, dim3(256), 0, m->stream, param_args(m, splits));
+    HD_HIP(hipGetLastError());
+    HD_CHECK(mlp_loss(m, pad64(n), loss));
+    if (h_grads) HD_CHECK(copy_to_host(m, h_grads, m->grads));
     return HD_OK;
 }
 
@@ -962,19 +1046,19 @@ int hd_mlp_train_step(hd_mlp* m, const uint64_t* d_states, const float* d_params
                       float lambda, float lr, float* loss)
 {
     if (!m || !d_states || !d_params || !d_targets || n <= 0) return fail(HD_ERR_ARG, "hd_mlp_train_step: bad argument");
-    HD_CHECK(gradients_impl(m, d_states, d_params, d_targets, n, lambda, 0, loss));
+    int splits = 0;
+    HD_CHECK(batch_pass(m, d_states, d_params, d_targets, n, lambda, 0, &splits));
     m->step += 1;
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.f - std::pow(b1, (float)m->step), c2 = 1.f - std::pow(b2, (float)m->step);
-    for (int l = 0; l < 4; ++l) {
-        const int64_t nw = (int64_t)m->rows[l] * m->cols[l];
-        hipLaunchKernelGGL(k_adam, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, m->stream, nw, m->w[l], m->gw[l],
-                           m->mw[l], m->vw[l], lr, b1, b2, c1, c2, 1e-8f);
-        hipLaunchKernelGGL(k_adam, dim3((unsigned)((m->rows[l] + 255) / 256)), dim3(256), 0, m->stream,
-                           (int64_t)m->rows[l], m->b[l], m->gb[l], m->mb[l], m->vb[l], lr, b1, b2, c1, c2, 1e-8f);
-    }
+    ParamArgs a = param_args(m, splits);
+    a.lr = lr;
+    a.b1 = 0.9f;
+    a.b2 = 0.999f;
+    a.c1 = 1.f - std::pow(a.b1, (float)m->step);
+    a.c2 = 1.f - std::pow(a.b2, (float)m->step);
+    a.eps = 1e-8f;
+    hipLaunchKernelGGL((k_params<true, true, true>), kParamGrid, dim3(256), 0, m->stream, a);
     HD_HIP(hipGetLastError());
-    return mlp_refresh_bf16(m);
+    return mlp_loss(m, pad64(n), loss);
 }
 
 int hd_mlp_start_vector(hd_mlp* m, const hd_basis* basis, const float* h_params, double* d_vec)

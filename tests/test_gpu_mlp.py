@@ -200,3 +200,29 @@ def test_start_vector_large_sector_matches_forward():
         a = np.exp((out[:, 2 * s] - out[:, 2 * s].max()).astype(np.float64)) * np.where(out[:, 2 * s + 1] >= 0, 1.0, -1.0)
         want += a / np.linalg.norm(a)
     assert np.linalg.norm(v - want) <= 1e-13 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("n_states,n", [(1, 1), (2, 63), (16, 65), (5, 1000), (3, 1025), (5, 4097)])
+def test_gradients_at_batch_edges(n_states, n):
+    """Gradients at the edges of the 64-sample padding and of the batch splits
+    (a block of at least 64 samples, 16 blocks at most) against the oracle,
+    and a training step against Adam's first step on those gradients."""
+    say("gradients", n_states, n)
+    rng = np.random.default_rng(n)
+    n_bits = 28
+    net = learned.AmplitudeNet(n_bits, 3, seed=6, n_states=n_states)
+    w = net.get_weights()
+    states, params, _ = _data(rng, n, n_bits)
+    targets = np.concatenate([_data(rng, n, n_bits)[2] for _ in range(n_states)], axis=1)
+    loss, g = net.gradients(states, params, targets, lam=0.5)
+    lref, gref = mo.loss_and_grads(w, states, params, targets, n_bits, 3, lam=0.5, bf=True)
+    assert abs(loss - lref) <= 1e-3 * abs(lref)
+    # BF16 deltas: 2^-9 relative rounding per factor, amplified by cancellation
+    # in the batch sum (the bound of test_forward_and_gradients_match_oracle)
+    assert np.linalg.norm(g - gref) <= 2e-2 * np.linalg.norm(gref)
+    bufs = [hd.DeviceBuffer.from_array(a) for a in (states, params, targets)]
+    l2 = net.train_step(*bufs, n, 0.5, 1e-3)
+    assert l2 == loss
+    # first step: both moments corrected to g and g^2
+    want = w - np.float32(1e-3) * g / (np.abs(g) + np.float32(1e-8))
+    assert np.max(np.abs(net.get_weights() - want)) <= 1e-3 * 1e-4
