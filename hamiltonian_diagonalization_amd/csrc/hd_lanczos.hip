@@ -191,6 +191,7 @@ struct LzStep {
     int first;              // j == k: the couplings to the kept vectors are the arrow
     int must;               // a full pass whatever the estimates say
     double eps_op, om_cycle;
+    double skip_tol;        // see k_lz_project
 };
 
 template <int NT>
@@ -474,12 +475,13 @@ k_lz_coefs(LzStep p, int pass, int nb, LzState* __restrict__ st, const double* _
 }
 
 // After the local step, w's components along the basis are at rounding level.
-// When every one of them is below kSkipTol |w| the projection is skipped and the
+// When every one of them is below skip_tol |w| the projection is skipped and the
 // coefficients count as zero (the recurrence then holds for the w actually kept):
 // each new vector is measured against the whole basis, so the basis stays
-// orthogonal to kSkipTol throughout.
-constexpr double kSkipTol = 1e-12;
-
+// orthogonal to skip_tol throughout.  What a skipped projection leaves in w the
+// recurrence misses, so skip_tol is 1e-12, and 0.02 tol where that is less (with
+// 1e-12 at tol = 1e-12, N=7, 2S=18 missed tol and was solved again: 239 products
+// instead of 118).
 // w -= sum_{i<=j} V_i coef_i unless the step has no pass or skips it;
 // partial_p[block] = |w|^2 of the result.
 template <bool C>
@@ -497,7 +499,7 @@ k_lz_project(LzStep p, int may_skip, const typename E<C>::T* __restrict__ V, con
         cm = fmax(cm, norm2(sc[i]));
     }
     __syncthreads();
-    const bool skip = may_skip && block_max<kVB>(cm) <= kSkipTol * kSkipTol * st->wn2;
+    const bool skip = may_skip && block_max<kVB>(cm) <= p.skip_tol * p.skip_tol * st->wn2;
     if (blockIdx.x == 0 && threadIdx.x == 0) st->skip = skip;
     if (skip) return;
     double nrm = 0.0;
@@ -609,7 +611,7 @@ k_lz_small(LzStep p, const typename E<C>::T* __restrict__ V, typename E<C>::T* _
         if (pass == 1 && !p.first) {
             double cm = 0.0;
             for (int i = threadIdx.x; i < nv; i += NT) cm = fmax(cm, norm2(sc[i]));
-            if (block_max<NT>(cm) <= kSkipTol * kSkipTol * wn2) break;
+            if (block_max<NT>(cm) <= p.skip_tol * p.skip_tol * wn2) break;
         }
         double nrm = 0.0;
         for (int i = threadIdx.x; i < n; i += NT) {
@@ -912,7 +914,7 @@ struct Lanczos {
     // first cancelled more than a factor 100 of the norm (the "twice is enough"
     // test of Daniel, Gragg, Kaufman and Stewart, Math. Comp. 30 (1976) 772),
     // or always in the first step of a cycle.
-    int step(int j, int k, int prec, bool must, double eps_op, double om_cycle)
+    int step(int j, int k, int prec, bool must, double eps_op, double om_cycle, double skip_tol)
     {
         const bool timing = n >= 65536 || steps % 16 == 0;
         ++steps;
@@ -920,7 +922,7 @@ struct Lanczos {
         mark(timing);
         HD_CHECK(apply(vec(j), w, prec));
         mark(timing);
-        const LzStep p{n, j, k, j == k, must, eps_op, om_cycle};
+        const LzStep p{n, j, k, j == k, must, eps_op, om_cycle, skip_tol};
         if (n <= (C ? kSmallComplex : kSmallReal)) {
             hipLaunchKernelGGL(k_lz_small<C>, dim3(1), dim3(kSmallThreads), 0, st, p, V, w, dst);
         } else {
@@ -944,11 +946,11 @@ struct Lanczos {
         T* w = vec(j + 1);
         hipLaunchKernelGGL(k_lz_clear, dim3(1), dim3(1), 0, st, dst);
         if (why == kStopSecond) {
-            const LzStep p{n, j, -1, 0, 1, 0.0, 0.0};
+            const LzStep p{n, j, -1, 0, 1, 0.0, 0.0, 0.0};
             pass(p, 2, false, w);
             hipLaunchKernelGGL(k_lz_finish<C>, dim3(nb), dim3(kVB), 0, st, p, 1, w, dst, pp);
         } else {
-            const LzStep p{n, j, -1, 1, 1, 0.0, 0.0};
+            const LzStep p{n, j, -1, 1, 1, 0.0, 0.0, 0.0};
             HD_CHECK(random_start(seed, (*rng_stream)++, w));
             pass(p, 1, false, w);
             pass(p, 2, false, w);
@@ -1218,7 +1220,7 @@ static int run_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* eval
             if (ended || done >= m) break;
             const int upto = check_in_cycle ? std::min(m, done + (L.n >= 65536 ? 1 : 4)) : m;
             for (int j = done; j < upto; ++j)
-                HD_CHECK(L.step(j, k, prec, !pro || j == m - 1, eps_op, om_cycle));
+                HD_CHECK(L.step(j, k, prec, !pro || j == m - 1, eps_op, om_cycle, std::min(1e-12, 0.02 * tol)));
             HD_CHECK(L.read_state(hs.get()));
             if (hs->stop) {
                 HD_CHECK(L.resume(hs->stop_step, hs->stop, o.seed, &rng_stream));
