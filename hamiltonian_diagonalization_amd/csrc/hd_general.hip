@@ -12,17 +12,17 @@
 // (k1 != k2), and the terms that land on one column are no longer the four
 // terms of one pair hop, so the pair tables of hd_build.hip do not apply.
 // Every term is evaluated per row, and duplicates are summed afterwards:
-//   1. k_gcount: one thread per row walks the terms in the reference's order
+//   1. k_gwalk: 32 or 64 lanes per row walk the terms in the reference's order
 //      and counts the ones the reference inserts into its map (|el| > tol,
 //      out >= in).
 //   2. exclusive scan -> raw row offsets.
-//   3. k_gfill: the same walk writes (column, value) in term order; an out
+//   3. k_gwalk again: the same walk writes (column, value) in term order; an out
 //      state outside the sector (FindFockStateIndex's miss, skipped by the
 //      reference) gets a sentinel column and is dropped in 4.
-//   4. k_gmerge: one workgroup per row sorts (column << 32 | position) keys in
-//      LDS (bitonic; the position makes equal columns keep term order), sums
+//   4. k_gmerge_wave, k_gmerge_block, k_gmerge, by the row's length: sort (column,
+//      position) keys (bitonic; the position makes equal columns keep term order), sum
 //      each run of equal columns from +0.0 in term order -- the reference's
-//      map += sequence -- drops |sum| < tol (Trim, counted) and writes the
+//      map += sequence -- drop |sum| < tol (Trim, counted) and write the
 //      kept entries packed at the row's raw offset.
 //   5. scan of the kept counts -> CRS row pointers; k_gcompact copies each
 //      row into the final FP64 / FP32 arrays.
@@ -43,6 +43,7 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <type_traits>
 
 #include "hd_internal.hpp"
 
@@ -81,8 +82,7 @@ struct GenArgs {
     const void* e;         // [K * max_q1] T
 };
 
-// The terms of one row in the reference's order, f(out, el) for each term the
-// reference inserts into its map.  Quadratic terms (Add_CdC_Terms :172-228):
+// The terms of one row in the reference's order, those it inserts into its map.  Quadratic terms (Add_CdC_Terms :172-228):
 // k2 over occupied orbitals ascending, k1 over GetK1(k2); k1 == k2 is the
 // diagonal E, otherwise k1 must be empty and c+_k1 c_k2 gives the sign
 // (Evaluate_CdC, fermions.hpp:155-227).  Quartic terms (Add_CdCdCC_Terms
@@ -90,116 +90,148 @@ struct GenArgs {
 // over mask ^ (occupied orbitals above k3 other than k4), k1 over
 // GetK1(k2,k3,k4), the occupation filter of :351-355, the sign of
 // c+_k1 c+_k2 c_k3 c_k4 (Evaluate_CdCdCC, fermions.hpp:52-144).
-template <bool CPLX, bool UPPER, typename Fn>
-HD_DEV void for_each_term(uint64_t s, const GenArgs& A, Fn&& f)
+
+// One quartic term: accepted, its out state and signed value.
+template <bool CPLX, bool UPPER>
+HD_DEV bool quartic_term(uint64_t s, const GenArgs& A, uint64_t b4, uint64_t b3, uint64_t b2, int idx, uint64_t& out,
+                         typename GT<CPLX>::T& el)
 {
     using T = typename GT<CPLX>::T;
-    if (A.has_quad) {
-        const T* E = static_cast<const T*>(A.e);
-        for (uint64_t t2 = s; t2; t2 &= t2 - 1) {
-            const int k2 = __builtin_ctzll(t2);
-            const uint64_t b2 = 1ull << k2;
-            const int n = A.nq1[k2];
-            for (int j = 0; j < n; ++j) {
-                const int idx = k2 * A.max_q1 + j;
-                const int k1 = A.q1[idx];
-                if (k1 == k2) {
-                    const T el = E[idx];
-                    if (gabs(el) > A.tol) f(s, el);
-                    continue;
-                }
-                const uint64_t b1 = 1ull << k1;
-                if (b1 & s) continue;  // c+_k1 on an occupied orbital
-                int c = __popcll(s & (b2 - 1));
-                uint64_t out = s ^ b2;
-                c += __popcll(out & (b1 - 1));
-                out |= b1;
-                if (UPPER && out < s) continue;
-                T el = E[idx];
-                if (c & 1) el = gneg(el);
-                if (gabs(el) > A.tol) f(out, el);
-            }
-        }
-    }
-    const T* V = static_cast<const T*>(A.v);
-    const int K = A.K;
-    for (uint64_t t4 = s; t4; t4 &= t4 - 1) {
-        const int k4 = __builtin_ctzll(t4);
-        const uint64_t b4 = 1ull << k4;
-        uint64_t t3 = s ^ b4;
-        while (t3) {
-            const uint64_t b3 = t3 & (0 - t3);
-            const int k3 = __builtin_ctzll(t3);
-            const uint64_t b34 = b3 | b4;
-            const int ebase = (k4 * K + k3) * K;
-            for (uint64_t t2 = A.mask ^ (t3 ^ b3); t2; t2 &= t2 - 1) {
-                const int k2 = __builtin_ctzll(t2);
-                const uint64_t b2 = 1ull << k2;
-                if ((b2 & s) && !(b2 & b34)) continue;
-                const int ent = ebase + k2;
-                const int n = A.nk1[ent];
-                for (int j = 0; j < n; ++j) {
-                    const int idx = ent * A.max_k1 + j;
-                    const uint64_t b1 = 1ull << A.k1[idx];
-                    if ((b1 & s) && !(b1 & b34)) continue;
-                    if (b1 & b2) continue;
-                    int c = __popcll(s & (b4 - 1));
-                    uint64_t out = s ^ b4;
-                    c += __popcll(out & (b3 - 1));
-                    out ^= b3;
-                    c += __popcll(out & (b2 - 1));
-                    out |= b2;
-                    c += __popcll(out & (b1 - 1));
-                    out |= b1;
-                    if (UPPER && out < s) continue;
-                    T el = V[idx];
-                    if (c & 1) el = gneg(el);
-                    if (gabs(el) > A.tol) f(out, el);
-                }
-            }
-            t3 ^= b3;
-        }
-    }
+    const uint64_t b1 = 1ull << A.k1[idx];
+    if (((b1 & s) && !(b1 & (b3 | b4))) || (b1 & b2)) return false;
+    int c = __popcll(s & (b4 - 1));
+    out = s ^ b4;
+    c += __popcll(out & (b3 - 1));
+    out ^= b3;
+    c += __popcll(out & (b2 - 1));
+    out |= b2;
+    c += __popcll(out & (b1 - 1));
+    out |= b1;
+    if (UPPER && out < s) return false;
+    el = static_cast<const T*>(A.v)[idx];
+    if (c & 1) el = gneg(el);
+    return gabs(el) > A.tol;
 }
 
+// One quadratic term.
 template <bool CPLX, bool UPPER>
-__global__ void __launch_bounds__(256)
-k_gcount(const uint64_t* __restrict__ states, int64_t dim, GenArgs A, int32_t* __restrict__ counts)
+HD_DEV bool quadratic_term(uint64_t s, const GenArgs& A, int k2, int idx, uint64_t& out, typename GT<CPLX>::T& el)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; row < dim; row += stride) {
-        int cnt = 0;
-        for_each_term<CPLX, UPPER>(states[row], A, [&](uint64_t, const typename GT<CPLX>::T&) { ++cnt; });
-        counts[row] = cnt;
+    using T = typename GT<CPLX>::T;
+    const int k1 = A.q1[idx];
+    el = static_cast<const T*>(A.e)[idx];
+    out = s;
+    if (k1 != k2) {
+        const uint64_t b1 = 1ull << k1, b2 = 1ull << k2;
+        if (b1 & s) return false;  // c+_k1 on an occupied orbital
+        int c = __popcll(s & (b2 - 1));
+        out = s ^ b2;
+        c += __popcll(out & (b1 - 1));
+        out |= b1;
+        if (UPPER && out < s) return false;
+        if (c & 1) el = gneg(el);
     }
+    return gabs(el) > A.tol;
 }
 
-template <bool CPLX, bool UPPER, bool LZ>
+// The walk by W lanes per row (W = 32 up to 32 orbitals, else 64):
+// lane k2 takes the list of (k2, k3, k4) for each ordered pair (k4, k3) in turn, and a
+// prefix sum over the lanes gives every list its place, so the terms keep the
+// reference's order while neighbouring lanes write neighbouring entries.  One thread
+// per row wrote each entry 64 rows apart (6x5 N=6 Wannier: fill 10.6 -> 7.2 ms,
+// count 2.1 -> 1.4 ms).  FILL = false counts only.  The rows of a
+// wavefront stay in step: every state has the same particle number.
+template <bool CPLX, bool UPPER, bool LZ, bool FILL, int W>
 __global__ void __launch_bounds__(256)
-k_gfill(const uint64_t* __restrict__ states, int64_t dim, GenArgs A, const int32_t* __restrict__ rank_blob,
-        int rank_words, const int64_t* __restrict__ rowptr, int32_t* __restrict__ col_out,
+k_gwalk(const uint64_t* __restrict__ states, int64_t dim, int N, GenArgs A, const int32_t* __restrict__ rank_blob,
+        int rank_words, const int64_t* __restrict__ rowptr, int32_t* __restrict__ counts, int32_t* __restrict__ col_out,
         typename GT<CPLX>::T* __restrict__ val_out, unsigned int* __restrict__ err)
 {
     using T = typename GT<CPLX>::T;
     extern __shared__ int32_t lds[];
-    block_copy_words(lds, rank_blob, rank_words);
-    __syncthreads();
+    if (FILL) {
+        block_copy_words(lds, rank_blob, rank_words);
+        __syncthreads();
+    }
     const RankView rv = rank_view(lds);
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; row < dim; row += stride) {
-        int64_t pos = rowptr[row];
-        const int64_t end = rowptr[row + 1];
-        for_each_term<CPLX, UPPER>(states[row], A, [&](uint64_t out, const T& el) {
-            if (pos >= end) {  // more terms than the count pass saw: never write past the row
+    const int k2 = threadIdx.x & (W - 1);
+    const uint64_t b2 = 1ull << k2;
+    const bool orb = k2 < A.K;
+    const int64_t stride = (int64_t)gridDim.x * (256 / W);
+    const int64_t rows_up = (dim + 256 / W - 1) / (256 / W) * (256 / W);
+    for (int64_t row = (int64_t)blockIdx.x * (256 / W) + threadIdx.x / W; row < rows_up; row += stride) {
+        const bool live = row < dim;
+        const uint64_t s = live ? states[row] : 0ull;
+        int64_t pos = FILL && live ? rowptr[row] : 0;
+        const int64_t end = FILL && live ? rowptr[row + 1] : 0;
+        int total = 0;
+        // places n terms of this lane after those of the lanes below; returns the first
+        auto place = [&](int n) {
+            int incl = n;
+#pragma unroll
+            for (int d = 1; d < W; d <<= 1) {
+                const int v = __shfl_up(incl, d, W);
+                if (k2 >= d) incl += v;
+            }
+            const int64_t at = pos + (incl - n);
+            pos += __shfl(incl, W - 1, W);
+            return at;
+        };
+        auto put = [&](int64_t& at, uint64_t out, const T& el) {
+            if (at >= end) {  // more terms than the count pass saw: never write past the row
                 atomicOr(err, 4u);
                 return;
             }
             uint64_t r;
-            col_out[pos] = rank_state<LZ>(rv, out, r) ? (int32_t)r : kNoColumn;
-            val_out[pos] = el;
-            ++pos;
-        });
-        if (pos != end) atomicOr(err, 2u);
+            col_out[at] = rank_state<LZ>(rv, out, r) ? (int32_t)r : kNoColumn;
+            val_out[at] = el;
+            ++at;
+        };
+        uint64_t out;
+        T el;
+        if (A.has_quad) {
+            const int len = live && orb && (b2 & s) ? A.nq1[k2] : 0, i0 = k2 * A.max_q1;
+            int n = 0;
+            for (int j = 0; j < len; ++j) n += quadratic_term<CPLX, UPPER>(s, A, k2, i0 + j, out, el);
+            if (FILL) {
+                int64_t at = place(n);
+                for (int j = 0; j < len && n; ++j)
+                    if (quadratic_term<CPLX, UPPER>(s, A, k2, i0 + j, out, el)) put(at, out, el);
+            } else {
+                total += n;
+            }
+        }
+        uint64_t t4 = s;
+        for (int i4 = 0; i4 < N; ++i4) {
+            const uint64_t b4 = t4 & (0 - t4);
+            const int k4 = live ? __builtin_ctzll(t4) : 0;
+            t4 &= t4 - 1;
+            uint64_t t3 = s ^ b4;
+            for (int i3 = 0; i3 + 1 < N; ++i3) {
+                const uint64_t b3 = t3 & (0 - t3);
+                const int k3 = live ? __builtin_ctzll(t3) : 0;
+                t3 &= t3 - 1;  // the occupied orbitals above k3 other than k4
+                const bool cand = live && orb && (b2 & (A.mask ^ t3)) && (!(b2 & s) || (b2 & (b3 | b4)));
+                const int ent = (k4 * A.K + k3) * A.K + k2;
+                const int len = cand ? A.nk1[ent] : 0, i0 = ent * A.max_k1;
+                int n = 0;
+                for (int j = 0; j < len; ++j) n += quartic_term<CPLX, UPPER>(s, A, b4, b3, b2, i0 + j, out, el);
+                if (FILL) {
+                    int64_t at = place(n);
+                    for (int j = 0; j < len && n; ++j)
+                        if (quartic_term<CPLX, UPPER>(s, A, b4, b3, b2, i0 + j, out, el)) put(at, out, el);
+                } else {
+                    total += n;
+                }
+            }
+        }
+        if (FILL) {
+            if (live && k2 == 0 && pos != end) atomicOr(err, 2u);
+        } else {
+#pragma unroll
+            for (int d = W / 2; d > 0; d >>= 1) total += __shfl_xor(total, d, W);
+            if (live && k2 == 0) counts[row] = total;
+        }
     }
 }
 
@@ -220,7 +252,7 @@ k_gmerge(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __restr
     for (int64_t row = blockIdx.x; row < dim; row += gridDim.x) {
         const int64_t start = rowptr[row];
         const int L = (int)(rowptr[row + 1] - start);
-        if (L <= min_len) continue;  // merged by k_gmerge_wave (uniform over the block)
+        if (L <= min_len) continue;  // merged by another kernel (uniform over the block)
         int n = 1;
         while (n < L) n <<= 1;
         for (int q = tid; q < n; q += kMergeThreads)
@@ -486,20 +518,129 @@ k_gmerge_wave(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __
     if (trimmed) atomicAdd(ntrim, trimmed);
 }
 
-// Rows of at most 512 raw terms by k_gmerge_wave, the longer ones by
-// k_gmerge<CAP> (CAP >= the longest row).  (A 512-thread block sorting rows of
-// up to 4,096 terms in registers was no faster than k_gmerge on them: 11.3
-// against 10.4 ms on the 6x5, N=8 hash tables.)
-template <bool CPLX, int CAP>
-void launch_merge(int grid, hipStream_t st, int64_t dim, const int64_t* raw_ptr, const int32_t* rcol,
-                  const typename GT<CPLX>::T* rval, double tol, int32_t* mcol, typename GT<CPLX>::T* mval,
-                  int32_t* kept, unsigned long long* ntrim)
+// k_gmerge for rows of more than min_len and at most 8 THREADS raw terms: a block's
+// keys (column << pos_bits | position) sorted in registers (bitonic_blocked), 32-bit
+// keys where column and position fit, the values staged in LDS with coalesced
+// loads.  Each thread sums the runs that start among its eight sorted keys once, in
+// term order from +0.0, and a prefix sum over the block places the kept ones.
+// k_gmerge sorts 64-bit keys in LDS with a barrier per stage, reads the values in
+// sorted order from L2 twice and adds up the counts on one thread (6x5 N=6
+// Wannier, rows of up to 4,096 raw terms: 19.8 -> 7.3 + 2.9 ms).
+template <bool CPLX, int THREADS, typename Key>
+__global__ void __launch_bounds__(THREADS)
+k_gmerge_block(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col_in,
+               const typename GT<CPLX>::T* __restrict__ val_in, double tol, int32_t* __restrict__ col_out,
+               typename GT<CPLX>::T* __restrict__ val_out, int32_t* __restrict__ kept,
+               unsigned long long* __restrict__ ntrim, int min_len, int pos_bits)
 {
+    using T = typename GT<CPLX>::T;
+    constexpr int CAP = 8 * THREADS;
+    __shared__ Key key[CAP];
+    __shared__ int wave_sum[THREADS / 64];
+    extern __shared__ double2 val_lds[];
+    T* const vals = reinterpret_cast<T*>(val_lds);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const Key none = (Key)~(Key)0 >> pos_bits, pos_mask = ((Key)1 << pos_bits) - 1;  // none: the no-column key
+    unsigned long long trimmed = 0;
+    for (int64_t row = blockIdx.x; row < dim; row += gridDim.x) {
+        const int64_t start = rowptr[row];
+        const int L = (int)(rowptr[row + 1] - start);
+        if (L <= min_len || L > CAP) continue;  // another kernel's row (uniform over the block)
+        for (int q = tid; q < CAP; q += THREADS) {
+            Key k = ~(Key)0;
+            if (q < L) {
+                const int32_t c = col_in[start + q];
+                k = ((c == kNoColumn ? none : (Key)(uint32_t)c) << pos_bits) | (Key)q;
+                vals[q] = val_in[start + q];
+            }
+            key[q] = k;
+        }
+        __syncthreads();
+        int P = 512;
+        while (P < L) P <<= 1;
+        bitonic_blocked<Key, THREADS>(key, P);
+        T sum[8];
+        unsigned keep = 0;
+        int c = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            sum[e] = gzero<T>();
+            const int i = 8 * tid + e;
+            if (i >= L) continue;
+            const Key col = key[i] >> pos_bits;
+            if (col == none || (i > 0 && (key[i - 1] >> pos_bits) == col)) continue;  // not the head of a run
+            T acc = gzero<T>();
+            for (int q = i; q < L && (key[q] >> pos_bits) == col; ++q) acc = gadd(acc, vals[(int)(key[q] & pos_mask)]);
+            if (gabs(acc) < tol) {
+                ++trimmed;
+            } else {
+                sum[e] = acc;
+                keep |= 1u << e;
+                ++c;
+            }
+        }
+        int incl = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(incl, d);
+            if (lane >= d) incl += v;
+        }
+        if (lane == 63) wave_sum[wave] = incl;
+        __syncthreads();
+        int before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < THREADS / 64; ++w) {
+            if (w < wave) before += wave_sum[w];
+            all += wave_sum[w];
+        }
+        if (tid == 0) kept[row] = all;
+        int64_t dst = start + before + (incl - c);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (!(keep & (1u << e))) continue;
+            col_out[dst] = (int32_t)(uint32_t)(key[8 * tid + e] >> pos_bits);
+            val_out[dst] = sum[e];
+            ++dst;
+        }
+        __syncthreads();  // the keys, values and sums have been read
+    }
+    if (trimmed) atomicAdd(ntrim, trimmed);
+}
+
+// Rows by their raw terms: up to 512 k_gmerge_wave, up to 2,048 and 4,096
+// k_gmerge_block with 256 and 512 threads, beyond that k_gmerge<CAP> (CAP >= the
+// longest row; its 64-bit keys in LDS).
+template <bool CPLX, int CAP>
+int launch_merge(int grid, hipStream_t st, int64_t dim, const int64_t* raw_ptr, const int32_t* rcol,
+                 const typename GT<CPLX>::T* rval, double tol, int32_t* mcol, typename GT<CPLX>::T* mval,
+                 int32_t* kept, unsigned long long* ntrim)
+{
+    using T = typename GT<CPLX>::T;
     hipLaunchKernelGGL((k_gmerge_wave<CPLX>), dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((dim + 3) / 4, 65536))),
                        dim3(256), 0, st, dim, raw_ptr, rcol, rval, tol, mcol, mval, kept, ntrim);
-    if (CAP > 512)
+    // the columns and the no-column key in 32 bits less the position's
+    auto block = [&](auto threads, int min_len, int bits) -> int {
+        constexpr int TH = decltype(threads)::value;
+        const size_t lds = sizeof(T) * 8 * TH;
+        const bool small = dim < ((int64_t)1 << (32 - bits));
+        const void* fn = small ? reinterpret_cast<const void*>(&k_gmerge_block<CPLX, TH, uint32_t>)
+                               : reinterpret_cast<const void*>(&k_gmerge_block<CPLX, TH, uint64_t>);
+        if (lds > 32 * 1024) HD_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (small)
+            hipLaunchKernelGGL((k_gmerge_block<CPLX, TH, uint32_t>), dim3(grid), dim3(TH), lds, st, dim, raw_ptr, rcol, rval,
+                               tol, mcol, mval, kept, ntrim, min_len, bits);
+        else
+            hipLaunchKernelGGL((k_gmerge_block<CPLX, TH, uint64_t>), dim3(grid), dim3(TH), lds, st, dim, raw_ptr, rcol, rval,
+                               tol, mcol, mval, kept, ntrim, min_len, 32);
+        HD_HIP(hipGetLastError());
+        return HD_OK;
+    };
+    if (CAP > 512) HD_CHECK(block(std::integral_constant<int, 256>{}, 512, 11));
+    if (CAP > 2048) HD_CHECK(block(std::integral_constant<int, 512>{}, 2048, 12));
+    if constexpr (CAP > 4096)
         hipLaunchKernelGGL((k_gmerge<CPLX, CAP>), dim3(grid), dim3(kMergeThreads), 0, st, dim, raw_ptr, rcol, rval,
-                           tol, mcol, mval, kept, ntrim, 512);
+                           tol, mcol, mval, kept, ntrim, 4096);
+    return HD_OK;
 }
 
 template <bool CPLX>
@@ -562,7 +703,6 @@ int run_general(hd_hamiltonian* h, const hd_basis* b, const hd_tables* t, double
     A.q1 = d_q1;
     A.e = d_e;
     const bool upper = h->storage == HD_STORAGE_UPPER_REF;
-    const int grid_rows = (int)std::max<int64_t>(1, std::min<int64_t>((dim + 255) / 256, (int64_t)n_cu * 8));
     EventTimer ev;
 
     // ---- count
@@ -570,7 +710,16 @@ int run_general(hd_hamiltonian* h, const hd_basis* b, const hd_tables* t, double
     ev.start(st);
     // the terms of the upper triangle (out >= in) in both storages; full
     // storage completes it below
-    hipLaunchKernelGGL((k_gcount<CPLX, true>), dim3(grid_rows), dim3(256), 0, st, b->d_states, dim, A, d_counts);
+    const int rows_per_block = K <= 32 ? 8 : 4;
+    const int walk_grid = (int)std::max<int64_t>(1, std::min<int64_t>((dim + rows_per_block - 1) / rows_per_block,
+                                                                      (int64_t)n_cu * 16));
+    // LZ only matters to the ranking of the fill
+    if (K <= 32)
+        hipLaunchKernelGGL((k_gwalk<CPLX, true, false, false, 32>), dim3(walk_grid), dim3(256), 0, st, b->d_states, dim,
+                           b->N, A, nullptr, 0, nullptr, d_counts, nullptr, nullptr, nullptr);
+    else
+        hipLaunchKernelGGL((k_gwalk<CPLX, true, false, false, 64>), dim3(walk_grid), dim3(256), 0, st, b->d_states, dim,
+                           b->N, A, nullptr, 0, nullptr, d_counts, nullptr, nullptr, nullptr);
     HD_ENQ(q, hipGetLastError());
     h->t_count = ev.stop(st);
     HD_GTRY(q.status());
@@ -600,17 +749,22 @@ int run_general(hd_hamiltonian* h, const hd_basis* b, const hd_tables* t, double
         }
         const bool lz = b->rt.is_lz != 0;
         unsigned int* d_err = reinterpret_cast<unsigned int*>(d_misc + 1);
-#define HD_GFILL(U, LZV)                                                                                      \
+#define HD_GFILL(LZV, W)                                                                                       \
     do {                                                                                                      \
         if (lds > 64 * 1024)                                                                                  \
-            HD_ENQ(q, hipFuncSetAttribute((const void*)k_gfill<CPLX, U, LZV>,                                 \
+            HD_ENQ(q, hipFuncSetAttribute((const void*)k_gwalk<CPLX, true, LZV, true, W>,                     \
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));             \
-        hipLaunchKernelGGL((k_gfill<CPLX, U, LZV>), dim3(grid_rows), dim3(256), lds, st, b->d_states, dim, A, \
-                           b->d_rank, rank_words, d_raw, d_rcol, d_rval, d_err);                              \
+        hipLaunchKernelGGL((k_gwalk<CPLX, true, LZV, true, W>), dim3(walk_grid), dim3(256), lds, st,          \
+                           b->d_states, dim, b->N, A, b->d_rank, rank_words, d_raw, nullptr, d_rcol, d_rval, d_err); \
     } while (0)
         ev.start(st);
-        if (lz) HD_GFILL(true, true);
-        else HD_GFILL(true, false);
+        if (lz) {
+            if (K <= 32) HD_GFILL(true, 32);
+            else HD_GFILL(true, 64);
+        } else {
+            if (K <= 32) HD_GFILL(false, 32);
+            else HD_GFILL(false, 64);
+        }
 #undef HD_GFILL
         HD_ENQ(q, hipGetLastError());
         h->t_fill = ev.stop(st);
@@ -636,11 +790,11 @@ int run_general(hd_hamiltonian* h, const hd_basis* b, const hd_tables* t, double
     {
         const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(dim, (int64_t)n_cu * 8));
         ev.start(st);
-        if (raw_max <= 512) launch_merge<CPLX, 512>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc);
-        else if (raw_max <= 1024) launch_merge<CPLX, 1024>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc);
-        else if (raw_max <= 4096) launch_merge<CPLX, 4096>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc);
-        else if (raw_max <= 8192) launch_merge<CPLX, 8192>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc);
-        else launch_merge<CPLX, 16384>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc);
+        if (raw_max <= 512) HD_GTRY((launch_merge<CPLX, 512>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc)));
+        else if (raw_max <= 1024) HD_GTRY((launch_merge<CPLX, 1024>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc)));
+        else if (raw_max <= 4096) HD_GTRY((launch_merge<CPLX, 4096>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc)));
+        else if (raw_max <= 8192) HD_GTRY((launch_merge<CPLX, 8192>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc)));
+        else HD_GTRY((launch_merge<CPLX, 16384>(grid, st, dim, d_raw, d_rcol, d_rval, tol, d_mcol, d_mval, d_counts, d_misc)));
         HD_ENQ(q, hipGetLastError());
         HD_GTRY(q.status());
         dfree(d_rcol);

@@ -274,3 +274,39 @@ def test_state_list_basis(oracle, case):
     assert np.abs(hf.spmv(x) - want).max() <= 1e-12 * np.abs(want).max()
     w = np.linalg.eigvalsh(up.to_dense(len(bas)))[:4]
     assert np.abs(np.asarray(hf.lanczos(nev=4, tol=1e-10).evals) - w).max() < 1e-9
+
+
+@pytest.mark.parametrize("n,two_s", [(7, 20), (10, 24), (12, 30)])
+def test_hash_lists_equal_pair_build(n, two_s):
+    """The general build of a sphere's hash lists against the pair-structure build
+    of the same tables, bit for bit in upper storage on row ranges across the
+    sector: rows of one wavefront (up to 512 raw terms) and of a block with 32-bit
+    keys, and at N=12, 2S=30 (more than 2^21 states) with 64-bit keys."""
+    say("hash lists vs pair build, upper storage, N", n, "2S", two_s)
+    K = two_s + 1
+    basis = hd.FockBasis(hd.Sector.lz((n * two_s) % 2, two_s), n, K)
+    t = models.sphere_tables(two_s, models.coulomb_list(two_s))
+    lists = hd.hash_lists_from_array(hd.LAYOUT_SPHERE, K, t.ktable, t.vtable)
+    a = hd.Hamiltonian(basis, t, storage=hd.STORAGE_UPPER_REF, values=(hd.F64,))
+    b = hd.Hamiltonian(basis, hd.TermTables.hash(K, **lists), storage=hd.STORAGE_UPPER_REF, values=(hd.F64,))
+    say("dim", basis.dim, "nnz", a.nnz, b.nnz)
+    assert n != 12 or basis.dim >= 1 << 21
+    assert a.nnz == b.nnz
+    for r0 in np.linspace(0, max(basis.dim - 1500, 0), 12).astype(np.int64):
+        r1 = min(int(r0) + 1500, basis.dim)
+        for x, y in zip(a.crs(int(r0), r1), b.crs(int(r0), r1)):
+            assert np.array_equal(x, y)
+
+
+def test_merge_row_lengths(oracle):
+    """Rows on both sides of the merge kernels' limits (512, 2048, 4096 raw terms)
+    in one matrix, against the oracle bit for bit."""
+    say("merge row lengths")
+    K, n = 12, 5
+    for seed, max_k1, fill in ((1, 4, 0.9), (2, 10, 0.8), (3, 16, 0.95)):
+        t = models.random_hash_tables(K, seed=seed, max_k1=max_k1, fill=fill)
+        basis = hd.FockBasis(hd.Sector.none(), n, K)
+        h = hd.Hamiltonian(basis, hd.TermTables.hash(K, **t), storage=hd.STORAGE_UPPER_REF)
+        ref = oracle.build_general(K, basis.states(), K, t["nk1"], t["k1"], t["v"], t["nq1"], t["q1"], t["e"])
+        rp, col, val = h.crs()
+        assert np.array_equal(rp, ref.rowptr) and np.array_equal(col, ref.col) and np.array_equal(val, ref.values())
