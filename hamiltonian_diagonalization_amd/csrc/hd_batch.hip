@@ -19,7 +19,7 @@
 //    cache line serves PT problems.  The dictionary of the block's PT points
 //    sits in LDS, and each XCD works on one tile of points.
 //  - Every Lanczos vector operation is one launch over all problems; inner
-//    products reduce per 1024-row chunk (chunks never straddle sectors) and
+//    products reduce per chunk of rows (chunks never straddle sectors) and
 //    then per sector in a fixed order, so results are deterministic.
 //  - The recurrence coefficients stay on the device.  The projected matrices
 //    of all problems are diagonalised on the device (one wavefront per
@@ -59,7 +59,11 @@ struct hd_batch {
 namespace hd {
 namespace {
 
-constexpr int kChunk = 1024;  // rows per reduction chunk
+// Rows per reduction chunk: kMaxChunk, halved down to kMinChunk until the chip has
+// eight chunks per CU.  A chunk is one block's serial walk, so few long chunks leave
+// the CUs waiting on memory (N=8, 2S=21, 16 points, 164,000 rows: chunks of 1,024
+// make 215 blocks; with 128 the dot kernel goes 60 -> 19 us, the update 62 -> 19 us).
+constexpr int kMaxChunk = 1024, kMinChunk = 128;
 constexpr int kVB = 256;      // threads of the chunked vector kernels
 constexpr int kMaxM = 64;     // Krylov basis limit: one lane per projected row
 constexpr int kGrp = 16;      // basis vectors per pass over w in the dot and update kernels
@@ -233,18 +237,25 @@ k_bdots(int nv, const double* __restrict__ V0, int64_t vstride, const double* __
 }
 
 // out[(s*PS + i)*Pp + p] = sum over the sector's chunks, in chunk order.
-__global__ void k_breduce(int nout, const double* __restrict__ partial, int PS, const int32_t* __restrict__ lsec,
-                          const int32_t* __restrict__ sec_c0, const int32_t* __restrict__ sec_c1, int Pp,
-                          double* __restrict__ out, const int* __restrict__ any, const int* __restrict__ sany)
+__global__ void __launch_bounds__(kVB)
+k_breduce(int nout, const double* __restrict__ partial, int PS, const int32_t* __restrict__ lsec,
+          const int32_t* __restrict__ sec_c0, const int32_t* __restrict__ sec_c1, int Pp,
+          double* __restrict__ out, const int* __restrict__ any, const int* __restrict__ sany)
 {
     if (any && *any == 0) return;
     const int s = lsec[blockIdx.x];
     if (sany && sany[s] == 0) return;
+    __shared__ double red[kVB];
     const int i = blockIdx.y;
-    const int p = threadIdx.x;
-    if (i >= nout || p >= Pp) return;
+    if (i >= nout) return;
+    // kVB / Pp lanes per point take the chunks in turn; their sums are added in order
+    const int p = threadIdx.x % Pp, cl = threadIdx.x / Pp, CL = kVB / Pp;
     double sum = 0.0;
-    for (int c = sec_c0[s]; c < sec_c1[s]; ++c) sum += partial[((size_t)c * PS + i) * Pp + p];
+    for (int c = sec_c0[s] + cl; c < sec_c1[s] && cl < CL; c += CL) sum += partial[((size_t)c * PS + i) * Pp + p];
+    red[threadIdx.x] = sum;
+    __syncthreads();
+    if (cl) return;
+    for (int q = 1; q < CL; ++q) sum += red[q * Pp + p];
     out[((size_t)s * PS + i) * Pp + p] = sum;
 }
 
@@ -610,10 +621,15 @@ __global__ void k_bfinish(Problems pr, int S, int m, int j, int k, int local, co
     inv[q] = live ? 1.0 / be : 0.0;
 }
 
-// Cyclic Jacobi on the symmetric n x n matrix A (LDS, row-major) by one
+// Jacobi on the symmetric n x n matrix A (LDS, row-major, n <= 64) by one
 // wavefront: A becomes diagonal, Z (LDS) collects the rotations, d the
 // eigenvalues (unsorted).  Rotation formulas of Rutishauser (Numer. Math. 9
 // (1966) 1): t = sgn(th)/(|th| + sqrt(th^2 + 1)), th = (a_qq - a_pp)/(2 a_pq).
+// A sweep takes the pairs in the rounds of a round-robin tournament (Brent and Luk,
+// SIAM J. Sci. Stat. Comput. 6 (1985) 69): the n/2 pairs of a round are disjoint, so
+// a lane per pair finds the rotations and the wavefront applies them together.  Pair
+// by pair, each rotation's square roots, divisions and four barriers were a
+// serial chain (912 problems of 27 x 27: 1.77 ms per restart against 0.51 ms).
 HD_DEV double wave_sum(double v)
 {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -622,7 +638,14 @@ HD_DEV double wave_sum(double v)
 
 HD_DEV void wave_jacobi(double* A, double* Z, double* d, int n)
 {
+    __shared__ double rc[32], rs[32];
+    __shared__ int rp[32], rq[32];
     const int lane = threadIdx.x;
+    const int n2 = (n + 1) / 2 * 2, np = n2 / 2, ring = n2 - 1;  // an odd n has one idle index per round
+    // column updates: np pairs side by side, as many rows at once as fit
+    const int rows_at = 64 / np, prow = lane / np, pcol = lane - prow * np;
+    // row updates: a pair's columns side by side
+    const int pairs_at = n <= 32 ? 2 : 1, half = n <= 32 ? lane >> 5 : 0, ccol = n <= 32 ? lane & 31 : lane;
     for (int i = lane; i < n * n; i += 64) Z[i] = (i / n == i % n) ? 1.0 : 0.0;
     __syncthreads();
     for (int sweep = 0; sweep < 60; ++sweep) {
@@ -635,38 +658,68 @@ HD_DEV void wave_jacobi(double* A, double* Z, double* d, int n)
         off = wave_sum(off);
         tot = wave_sum(tot);
         if (!(off > 1e-28 * tot)) break;
-        for (int p = 0; p < n - 1; ++p)
-            for (int q = p + 1; q < n; ++q) {
-                const double apq = A[p * n + q];
-                if (fabs(apq) <= 1e-300) continue;  // uniform: every lane read the same value
-                const double app = A[p * n + p], aqq = A[q * n + q];
-                const double th = (aqq - app) / (2.0 * apq);
-                const double t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-                const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-                __syncthreads();
-                if (lane < n) {  // columns p, q
-                    const double akp = A[lane * n + p], akq = A[lane * n + q];
-                    A[lane * n + p] = c * akp - s * akq;
-                    A[lane * n + q] = s * akp + c * akq;
+        for (int round = 0; round < ring; ++round) {
+            double app = 0.0, aqq = 0.0, tpq = 0.0;
+            int p = 0, q = 0;
+            if (lane < np) {
+                int u = round + lane, v = round - lane;
+                if (u >= ring) u -= ring;
+                if (v < 0) v += ring;
+                if (lane == 0) u = ring;  // the fixed player
+                p = u < v ? u : v;
+                q = u < v ? v : u;
+                double c = 1.0, s = 0.0;
+                if (q < n && n > 1) {
+                    const double apq = A[p * n + q];
+                    app = A[p * n + p];
+                    aqq = A[q * n + q];
+                    if (!(fabs(apq) <= 1e-300)) {
+                        const double th = (aqq - app) / (2.0 * apq);
+                        const double t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
+                        c = 1.0 / sqrt(t * t + 1.0);
+                        s = t * c;
+                        tpq = t * apq;
+                    }
+                } else {
+                    q = -1;  // paired with the idle index
                 }
-                __syncthreads();
-                if (lane < n) {  // rows p, q
-                    const double apk = A[p * n + lane], aqk = A[q * n + lane];
-                    A[p * n + lane] = c * apk - s * aqk;
-                    A[q * n + lane] = s * apk + c * aqk;
-                    const double zkp = Z[lane * n + p], zkq = Z[lane * n + q];
-                    Z[lane * n + p] = c * zkp - s * zkq;
-                    Z[lane * n + q] = s * zkp + c * zkq;
-                }
-                __syncthreads();
-                if (lane == 0) {  // the rotated 2x2 block takes its exact values
-                    A[p * n + q] = 0.0;
-                    A[q * n + p] = 0.0;
-                    A[p * n + p] = app - t * apq;
-                    A[q * n + q] = aqq + t * apq;
-                }
-                __syncthreads();
+                rc[lane] = c;
+                rs[lane] = s;
+                rp[lane] = p;
+                rq[lane] = q;
             }
+            __syncthreads();
+            if (prow < rows_at && rq[pcol] >= 0) {  // columns p, q of A and Z
+                const int cp = rp[pcol], cq = rq[pcol];
+                const double c = rc[pcol], s = rs[pcol];
+                for (int r = prow; r < n; r += rows_at) {
+                    const double akp = A[r * n + cp], akq = A[r * n + cq];
+                    const double zkp = Z[r * n + cp], zkq = Z[r * n + cq];
+                    A[r * n + cp] = c * akp - s * akq;
+                    A[r * n + cq] = s * akp + c * akq;
+                    Z[r * n + cp] = c * zkp - s * zkq;
+                    Z[r * n + cq] = s * zkp + c * zkq;
+                }
+            }
+            __syncthreads();
+            if (ccol < n)
+                for (int k = half; k < np; k += pairs_at) {  // rows p, q
+                    const int cp = rp[k], cq = rq[k];
+                    if (cq < 0) continue;
+                    const double c = rc[k], s = rs[k];
+                    const double apk = A[cp * n + ccol], aqk = A[cq * n + ccol];
+                    A[cp * n + ccol] = c * apk - s * aqk;
+                    A[cq * n + ccol] = s * apk + c * aqk;
+                }
+            __syncthreads();
+            if (lane < np && q >= 0 && tpq != 0.0) {  // the rotated 2x2 blocks take their exact values
+                A[p * n + q] = 0.0;
+                A[q * n + p] = 0.0;
+                A[p * n + p] = app - tpq;
+                A[q * n + q] = aqq + tpq;
+            }
+            __syncthreads();
+        }
     }
     for (int i = lane; i < n; i += 64) d[i] = A[i * n + i];
     __syncthreads();
@@ -1181,13 +1234,19 @@ int hd_batch_solve(hd_batch* b, const hd_batch_opts* o, double* h_evals, double*
     if (!lsec.empty()) {
         const int nls = (int)lsec.size();
         // chunks of the Lanczos sectors
+        int n_cu = 256;
+        HD_CHECK(device_props(&n_cu, nullptr));
+        int64_t lrows = 0;
+        for (int s : lsec) lrows += b->dim[(size_t)s];
+        int64_t chunk = kMaxChunk;
+        while (chunk > kMinChunk && lrows / chunk < 8 * (int64_t)n_cu) chunk /= 2;
         std::vector<int64_t> ck_r0, ck_r1;
         std::vector<int32_t> ck_sec, sec_c0((size_t)S, 0), sec_c1((size_t)S, 0);
         for (int s : lsec) {
             sec_c0[(size_t)s] = (int)ck_r0.size();
-            for (int64_t r = 0; r < b->dim[(size_t)s]; r += kChunk) {
+            for (int64_t r = 0; r < b->dim[(size_t)s]; r += chunk) {
                 ck_r0.push_back(b->row0[(size_t)s] + r);
-                ck_r1.push_back(b->row0[(size_t)s] + std::min<int64_t>(r + kChunk, b->dim[(size_t)s]));
+                ck_r1.push_back(b->row0[(size_t)s] + std::min<int64_t>(r + chunk, b->dim[(size_t)s]));
                 ck_sec.push_back(s);
             }
             sec_c1[(size_t)s] = (int)ck_r0.size();
@@ -1276,7 +1335,7 @@ int hd_batch_solve(hd_batch* b, const hd_batch_opts* o, double* h_evals, double*
                         const int* sany = nullptr) {
             hipLaunchKernelGGL(k_bdots, dim3((unsigned)nck), dim3(kVB), 0, st, nv, base, vstride, wv, want_norm, ck,
                                Pp, PS, partial, any, sany);
-            hipLaunchKernelGGL(k_breduce, dim3((unsigned)nls, (unsigned)(nv + want_norm)), dim3(Pp), 0, st,
+            hipLaunchKernelGGL(k_breduce, dim3((unsigned)nls, (unsigned)(nv + want_norm)), dim3(kVB), 0, st,
                                nv + want_norm, partial, PS, d_lsec, d_sec_c0, d_sec_c1, Pp, out, any, sany);
         };
         auto update = [&](int nv, const double* base, const double* coef, int64_t cs, int64_t ci, const double* mask,
@@ -1385,7 +1444,7 @@ int hd_batch_solve(hd_batch* b, const hd_batch_opts* o, double* h_evals, double*
             HD_CHECK(spmm(b, Vj(i), W, st));
             hipLaunchKernelGGL(k_bresid, dim3((unsigned)nck), dim3(kVB), 0, st, W, Vj(i), d_ev + i,
                                (int64_t)Pp * nev, (int64_t)nev, ck, Pp, partial);
-            hipLaunchKernelGGL(k_breduce, dim3((unsigned)nls, 1u), dim3(Pp), 0, st, 1, partial, 1, d_lsec, d_sec_c0,
+            hipLaunchKernelGGL(k_breduce, dim3((unsigned)nls, 1u), dim3(kVB), 0, st, 1, partial, 1, d_lsec, d_sec_c0,
                                d_sec_c1, Pp, R2, nullptr, nullptr);
             HD_HIP(hipGetLastError());
             std::vector<double> tmp((size_t)S * Pp);

@@ -176,3 +176,26 @@ def test_batch_solve_large_krylov_basis(oracle, ncv):
                 M[i, ref.col[ref.rowptr[i]:ref.rowptr[i + 1]]] = ref.values()[ref.rowptr[i]:ref.rowptr[i + 1]]
             want = np.linalg.eigvalsh(M)[:4]
             assert np.max(np.abs(ev[s, p] - want) / np.maximum(1, np.abs(want))) < 1e-10, (lzs[s], p)
+
+
+@pytest.mark.parametrize("ncv, dense_below, n_pts", [(8, 1, 3), (17, 2, 1), (32, 63, 5), (33, 64, 17), (64, 65, 2)])
+def test_batch_projected_sizes(oracle, ncv, dense_below, n_pts):
+    """The device eigensolver of the dense sectors and of the projected matrices at
+    the edges of its lane layout (odd and even orders, 32 to 64, a basis that ends
+    early in a small sector) and the vector chunks at one to 32 padded points."""
+    say("batch projected sizes", ncv, dense_below, n_pts)
+    n, two_s = 6, 15
+    bp, bases, tables = _batch(n, two_s, list(range(0, 61, 2)), _points(n_pts, ncv))
+    ev, _, st = bp.solve(nev=3, tol=1e-10, ncv=ncv, seed=0, dense_below=dense_below)
+    assert st["converged"] == st["problems"]
+    for s, b in enumerate(bases):
+        bas = b.states()
+        for p in {0, n_pts - 1}:
+            ref = _oracle_full(oracle, n, two_s, bas, tables[p])
+            M = np.zeros((b.dim, b.dim))
+            for i in range(b.dim):
+                M[i, ref.col[ref.rowptr[i]:ref.rowptr[i + 1]]] = ref.values()[ref.rowptr[i]:ref.rowptr[i + 1]]
+            want = np.linalg.eigvalsh(M)[:3]
+            got = ev[s, p, :len(want)]
+            # a residual r bounds an eigenvalue's error by r (here r <= 1e-10 max(1, |E|))
+            assert np.max(np.abs(got - want) / np.maximum(1, np.abs(want))) < 1e-10, (s, p)
