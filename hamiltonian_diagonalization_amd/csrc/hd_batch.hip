@@ -23,7 +23,7 @@
 //    then per sector in a fixed order, so results are deterministic.
 //  - The recurrence coefficients stay on the device.  The projected matrices
 //    of all problems are diagonalised on the device (one wavefront per
-//    problem, cyclic Jacobi in LDS), which also decides convergence and forms
+//    problem, Jacobi in LDS), which also decides convergence and forms
 //    the restart rotation.  A restart cycle is therefore a fixed sequence of
 //    launches; from the second cycle on it is captured once as a hipGraph and
 //    replayed, and the host reads one counter per cycle.
@@ -236,7 +236,7 @@ k_bdots(int nv, const double* __restrict__ V0, int64_t vstride, const double* __
     }
 }
 
-// out[(s*PS + i)*Pp + p] = sum over the sector's chunks, in chunk order.
+// out[(s*PS + i)*Pp + p] = sum over the sector's chunks, in a fixed order.
 __global__ void __launch_bounds__(kVB)
 k_breduce(int nout, const double* __restrict__ partial, int PS, const int32_t* __restrict__ lsec,
           const int32_t* __restrict__ sec_c0, const int32_t* __restrict__ sec_c1, int Pp,

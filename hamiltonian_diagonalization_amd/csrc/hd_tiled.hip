@@ -55,7 +55,7 @@ constexpr int kMaxLines = 5120;    // distinct lines per group (load factor 0.62
 constexpr int kMaxChunks = kMaxLines / kTC;
 constexpr int kU = 8;              // entries each SpMV lane has in flight
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
-constexpr int kBuildThreads = 512;
+constexpr int kBuildThreads = 1024;  // one build block per CU (its LDS): all 16 wavefronts hide latency
 constexpr int kLU = 8;             // entries each build thread loads ahead
 constexpr int kSpmvThreads = 1024;  // one block per group: kSpmvThreads / TG lanes per row
 
@@ -99,7 +99,6 @@ struct TilePlanLds {
     uint32_t keys[kHashSlots];
     uint32_t sorted[kHashSlots];
     uint16_t rank_of[kHashSlots];
-    uint8_t chunk_of[kHashSlots];
     uint32_t counts[kMaxChunks * TG];
     uint32_t cum[kMaxChunks * TG];
     uint32_t T[kMaxChunks * (TG + 1)];
@@ -126,10 +125,12 @@ __device__ __forceinline__ int row_of(const TilePlanLds<TG>& S, int nrows, int64
 // Builds the plan in LDS; S.flags != 0 when the group does not fit.
 // LS: log2 of the x values per 128-byte line (4 real, 3 complex).  QA: every
 // (chunk, row) block is padded to a multiple of 4 entries (the 3-byte layout,
-// read as 12-byte quads).
+// read as 12-byte quads).  known: the group's sorted lines where an earlier pass
+// kept them, n_known of them; then no entry is read for them.
 template <int TG, int LS, bool QA>
 __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const int64_t* __restrict__ rowptr,
-                          const int32_t* __restrict__ col, const uint16_t* __restrict__ code, int64_t g)
+                          const int32_t* __restrict__ col, const uint16_t* __restrict__ code, int64_t g,
+                          const uint32_t* __restrict__ known, int n_known)
 {
     const int t = threadIdx.x;
     const int64_t r0 = g * TG, r1 = min(r0 + TG, dim);
@@ -142,74 +143,91 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
     for (int i = t; i < TG; i += kBuildThreads) S.dpos[i] = -1;
     if (t == 0) S.n_lines = S.n_chunks = S.flags = 0;
     __syncthreads();
-    const int64_t e0 = S.rp[0], e1 = S.rp[nrows];
-    // kLU entries per thread loaded before any is inserted: one block per CU
-    // leaves few waves to hide the load latency
-    for (int64_t jb = e0; jb < e1; jb += (int64_t)kBuildThreads * kLU) {
-        uint32_t qv[kLU], cv[kLU];
-#pragma unroll
-        for (int u = 0; u < kLU; ++u) {  // clamped, not guarded: the loads issue together
-            const int64_t j = min(jb + u * kBuildThreads + t, e1 - 1);
-            qv[u] = code[j];
-            cv[u] = (uint32_t)col[j];
+    if (known) {
+        for (int i = t; i < n_known; i += kBuildThreads) {
+            const uint32_t line = known[i];
+            S.sorted[i] = line;
+            const int h = hash_insert(S.keys, line);
+            if (h >= 0) S.rank_of[h] = (uint16_t)i;
+            else atomicOr(&S.flags, 1);
         }
-#pragma unroll
-        for (int u = 0; u < kLU; ++u) {
-            const int64_t j = jb + u * kBuildThreads + t;
-            if (j >= e1) continue;
-            if (qv[u] == 0xFFFFu) {
-                S.dpos[row_of(S, nrows, j)] = j;
-                continue;
+        if (t == 0) S.n_lines = n_known;
+        for (int r = t; r < nrows; r += kBuildThreads) {  // the diagonal entry, at column r0 + r
+            int64_t lo = S.rp[r], hi = S.rp[r + 1];
+            while (lo < hi) {
+                const int64_t mid = (lo + hi) >> 1;
+                if (col[mid] < r0 + r) lo = mid + 1;
+                else hi = mid;
             }
-            if (hash_insert(S.keys, cv[u] >> LS) < 0) atomicOr(&S.flags, 1);
+            if (lo < S.rp[r + 1] && col[lo] == r0 + r && code[lo] == 0xFFFFu) S.dpos[r] = lo;
         }
-    }
-    __syncthreads();
-    {
-        const int lane = t & 63;
-        for (int i = t; i < kHashSlots; i += kBuildThreads) {
-            const uint32_t k = S.keys[i];
-            const uint64_t m = __ballot(k != kEmpty);
-            int basei = 0;
-            if (lane == 0 && m) basei = atomicAdd(&S.n_lines, __popcll(m));
-            basei = __shfl(basei, 0);
-            if (k != kEmpty) S.sorted[basei + __popcll(m & ((1ull << lane) - 1ull))] = k;
-        }
-    }
-    __syncthreads();
-    const int L = S.n_lines;
-    if (L > kMaxLines) {
-        if (t == 0) S.flags |= 2;
         __syncthreads();
-        return;
-    }
-    int P = 1;
-    while (P < L) P <<= 1;
-    if (P <= 8 * kBuildThreads) {
-        bitonic_blocked<uint32_t, kBuildThreads>(S.sorted, P);
     } else {
-        for (int k = 2; k <= P; k <<= 1)
-            for (int jj = k >> 1; jj > 0; jj >>= 1) {
-                for (int i = t; i < P; i += kBuildThreads) {
-                    const int ixj = i ^ jj;
-                    if (ixj > i) {
-                        const uint32_t a = S.sorted[i], b = S.sorted[ixj];
-                        if ((a > b) == ((i & k) == 0)) {
-                            S.sorted[i] = b;
-                            S.sorted[ixj] = a;
+        const int64_t e0 = S.rp[0], e1 = S.rp[nrows];
+        // kLU entries per thread loaded before any is inserted: one block per CU
+        // leaves few waves to hide the load latency
+        for (int64_t jb = e0; jb < e1; jb += (int64_t)kBuildThreads * kLU) {
+            uint32_t qv[kLU], cv[kLU];
+#pragma unroll
+            for (int u = 0; u < kLU; ++u) {  // clamped, not guarded: the loads issue together
+                const int64_t j = min(jb + u * kBuildThreads + t, e1 - 1);
+                qv[u] = code[j];
+                cv[u] = (uint32_t)col[j];
+            }
+#pragma unroll
+            for (int u = 0; u < kLU; ++u) {
+                const int64_t j = jb + u * kBuildThreads + t;
+                if (j >= e1) continue;
+                if (qv[u] == 0xFFFFu) {
+                    S.dpos[row_of(S, nrows, j)] = j;
+                    continue;
+                }
+                if (hash_insert(S.keys, cv[u] >> LS) < 0) atomicOr(&S.flags, 1);
+            }
+        }
+        __syncthreads();
+        {
+            const int lane = t & 63;
+            for (int i = t; i < kHashSlots; i += kBuildThreads) {
+                const uint32_t k = S.keys[i];
+                const uint64_t m = __ballot(k != kEmpty);
+                int basei = 0;
+                if (lane == 0 && m) basei = atomicAdd(&S.n_lines, __popcll(m));
+                basei = __shfl(basei, 0);
+                if (k != kEmpty) S.sorted[basei + __popcll(m & ((1ull << lane) - 1ull))] = k;
+            }
+        }
+        __syncthreads();
+        if (S.n_lines > kMaxLines) {
+            if (t == 0) S.flags |= 2;
+            __syncthreads();
+            return;
+        }
+        const int L = S.n_lines;
+        int P = 1;
+        while (P < L) P <<= 1;
+        if (P <= 8 * kBuildThreads) {
+            bitonic_blocked<uint32_t, kBuildThreads>(S.sorted, P);
+        } else {
+            for (int k = 2; k <= P; k <<= 1)
+                for (int jj = k >> 1; jj > 0; jj >>= 1) {
+                    for (int i = t; i < P; i += kBuildThreads) {
+                        const int ixj = i ^ jj;
+                        if (ixj > i) {
+                            const uint32_t a = S.sorted[i], b = S.sorted[ixj];
+                            if ((a > b) == ((i & k) == 0)) {
+                                S.sorted[i] = b;
+                                S.sorted[ixj] = a;
+                            }
                         }
                     }
+                    __syncthreads();
                 }
-                __syncthreads();
-            }
+        }
+        for (int i = t; i < L; i += kBuildThreads) S.rank_of[hash_find(S.keys, S.sorted[i])] = (uint16_t)i;
     }
-    // ranks, and the chunks: 256 consecutive lines each
-    for (int i = t; i < L; i += kBuildThreads) {
-        const int h = hash_find(S.keys, S.sorted[i]);
-        S.rank_of[h] = (uint16_t)i;
-        S.chunk_of[i] = (uint8_t)(i / kTC);
-    }
-    const int nch = (L + kTC - 1) / kTC;
+    // the chunks: kTC consecutive lines each
+    const int L = S.n_lines, nch = (L + kTC - 1) / kTC;
     for (int c = t; c <= nch; c += kBuildThreads) S.ls[c] = (uint32_t)min(c * kTC, L);
     if (t == 0) S.n_chunks = nch;
     __syncthreads();
@@ -266,16 +284,23 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
     __syncthreads();
 }
 
-// Pass 1: per group, the distinct lines, the chunks and the padded entries.
+// Pass 1: per group, the distinct lines, the chunks and the padded entries.  keep (may
+// be null): kMaxLines words per group for its sorted lines, which pass 2 then reads
+// in place of finding them again from every entry (N=12, 2S=33: pass 2 37.4 -> 15.4
+// ms with these and the 1,024-thread blocks, pass 1 21.9 -> 18.5 ms with the blocks
+// alone).  Both passes are bound by the chains of dependent LDS reads per entry and
+// by the plan's searches.
 template <int TG, int LS, bool QA>
 __global__ void __launch_bounds__(kBuildThreads)
 k_tile_count(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
              const uint16_t* __restrict__ code, int64_t* __restrict__ n_lines, int64_t* __restrict__ n_entries,
-             int64_t* __restrict__ n_chunks, int* __restrict__ overflow)
+             int64_t* __restrict__ n_chunks, uint32_t* __restrict__ keep, int* __restrict__ overflow)
 {
     __shared__ TilePlanLds<TG> S;
     const int64_t g = blockIdx.x;
-    tile_plan<TG, LS, QA>(S, dim, rowptr, col, code, g);
+    tile_plan<TG, LS, QA>(S, dim, rowptr, col, code, g, nullptr, 0);
+    if (keep && !S.flags)
+        for (int i = threadIdx.x; i < S.n_lines; i += kBuildThreads) keep[g * kMaxLines + i] = S.sorted[i];
     if (threadIdx.x == 0) {
         n_lines[g] = S.n_lines;
         n_chunks[g] = S.n_chunks;
@@ -291,18 +316,19 @@ template <int TG, int W, bool QA>
 __global__ void __launch_bounds__(kBuildThreads)
 k_tile_fill(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
             const uint16_t* __restrict__ code, const double* __restrict__ diag, const int64_t* __restrict__ base,
-            int64_t groups, uint32_t* __restrict__ entries, uint32_t* __restrict__ lines,
-            uint32_t* __restrict__ meta, double* __restrict__ tdiag, int* __restrict__ error)
+            int64_t groups, const uint32_t* __restrict__ keep, uint32_t* __restrict__ entries,
+            uint32_t* __restrict__ lines, uint32_t* __restrict__ meta, double* __restrict__ tdiag,
+            int* __restrict__ error)
 {
     constexpr int LS = W == 2 ? 3 : 4;
     __shared__ TilePlanLds<TG> S;
     const int t = threadIdx.x;
     const int64_t g = blockIdx.x;
-    tile_plan<TG, LS, QA>(S, dim, rowptr, col, code, g);
+    const int64_t lb = base[groups + 1 + g], ln = base[groups + 1 + g + 1] - lb;
+    tile_plan<TG, LS, QA>(S, dim, rowptr, col, code, g, keep ? keep + g * kMaxLines : nullptr, (int)ln);
     const int64_t r0 = g * TG, r1 = min(r0 + TG, dim);
     const int nrows = (int)(r1 - r0);
     const int64_t eb = base[g], en = base[g + 1] - eb;
-    const int64_t lb = base[groups + 1 + g], ln = base[groups + 1 + g + 1] - lb;
     const int64_t mb = base[2 * (groups + 1) + g], mn = base[2 * (groups + 1) + g + 1] - mb;
     const int L = S.n_lines, nch = S.n_chunks;
     if (S.flags || L != ln || (int64_t)nch * (TG + 2) + 1 != mn || (int64_t)S.cbase[nch] != en) {
@@ -343,7 +369,7 @@ k_tile_fill(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __re
                 const int h = hash_find(S.keys, cj >> LS);
                 if (h < 0) continue;  // flagged by the plan
                 const int rank = S.rank_of[h];
-                const int c = S.chunk_of[rank];
+                const int c = rank / kTC;
                 const int64_t i_off = (j - S.rp[r]) - (S.dpos[r] >= 0 && S.dpos[r] < j ? 1 : 0);
                 const int64_t pos = (int64_t)S.T[c * (TG + 1) + r] + (i_off - S.cum[c * TG + r]);
                 if (pos < S.T[c * (TG + 1) + r] || pos >= S.T[c * (TG + 1) + r + 1] || pos >= en) {
@@ -351,7 +377,7 @@ k_tile_fill(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __re
                     continue;
                 }
                 const uint32_t code20 = ((q >> 15) << 19) | (q & 0x7FFFu);
-                entries[eb + pos] = ((uint32_t)(rank - (int)S.ls[c]) << 24) | ((cj & ((1u << LS) - 1u)) << 20) | code20;
+                entries[eb + pos] = ((uint32_t)(rank % kTC) << 24) | ((cj & ((1u << LS) - 1u)) << 20) | code20;
             }
         }
     }
@@ -717,6 +743,9 @@ static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
     if (rc == HD_OK) rc = dalloc_t(&d_ne, (size_t)G, "tile entry counts");
     if (rc == HD_OK) rc = dalloc_t(&d_nc, (size_t)G, "tile chunk counts");
     if (rc == HD_OK) rc = dalloc_t(&d_flag, 2, "tile flags");
+    // room for the groups' lines between the passes; without it pass 2 finds them again
+    uint32_t* d_keep = nullptr;
+    if (rc == HD_OK && dalloc_t(&d_keep, (size_t)G * kMaxLines, "tile lines of pass 1") != HD_OK) d_keep = nullptr;
     HipErrors q;
     std::vector<int64_t> nl(G), ne(G), nc(G);
     int flags[2] = {0, 0};
@@ -724,13 +753,13 @@ static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
         HD_ENQ(q, hipMemsetAsync(d_flag, 0, 2 * sizeof(int), st));
         if (h->is_complex)
             hipLaunchKernelGGL((k_tile_count<TG, 3, false>), dim3((unsigned)G), dim3(kBuildThreads), 0, st, h->dim,
-                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_flag);
+                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_keep, d_flag);
         else if (entry_bytes == 3)
             hipLaunchKernelGGL((k_tile_count<TG, 4, true>), dim3((unsigned)G), dim3(kBuildThreads), 0, st, h->dim,
-                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_flag);
+                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_keep, d_flag);
         else
             hipLaunchKernelGGL((k_tile_count<TG, 4, false>), dim3((unsigned)G), dim3(kBuildThreads), 0, st, h->dim,
-                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_flag);
+                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_keep, d_flag);
         HD_ENQ(q, hipGetLastError());
         HD_ENQ(q, hipMemcpyAsync(nl.data(), d_nl, G * sizeof(int64_t), hipMemcpyDeviceToHost, st));
         HD_ENQ(q, hipMemcpyAsync(ne.data(), d_ne, G * sizeof(int64_t), hipMemcpyDeviceToHost, st));
@@ -762,19 +791,28 @@ static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
         h->tg_lines = l;
         h->tg_offs = o;
     }
-    if (rc == HD_OK) rc = dalloc_t(&h->d_tg_base, base.size(), "tile bases");
-    if (rc == HD_OK) rc = dalloc_t(&h->d_tg_entries, (size_t)std::max<int64_t>(h->tg_entries, 1), "tile entries");
-    if (rc == HD_OK) rc = dalloc_t(&h->d_tg_lines, (size_t)std::max<int64_t>(h->tg_lines, 1), "tile lines");
-    if (rc == HD_OK) rc = dalloc_t(&h->d_tg_offs, (size_t)std::max<int64_t>(h->tg_offs, 1), "tile chunk tables");
+    auto get = [&](auto** ptr, size_t n, const char* what) {
+        int r = dalloc_t(ptr, n, what);
+        if (r != HD_OK && d_keep) {  // the layout goes before the kept lines
+            dfree(d_keep);
+            d_keep = nullptr;
+            r = dalloc_t(ptr, n, what);
+        }
+        return r;
+    };
+    if (rc == HD_OK) rc = get(&h->d_tg_base, base.size(), "tile bases");
+    if (rc == HD_OK) rc = get(&h->d_tg_entries, (size_t)std::max<int64_t>(h->tg_entries, 1), "tile entries");
+    if (rc == HD_OK) rc = get(&h->d_tg_lines, (size_t)std::max<int64_t>(h->tg_lines, 1), "tile lines");
+    if (rc == HD_OK) rc = get(&h->d_tg_offs, (size_t)std::max<int64_t>(h->tg_offs, 1), "tile chunk tables");
     const int W = h->is_complex ? 2 : 1;  // doubles per value
-    if (rc == HD_OK) rc = dalloc_t(&h->d_tg_diag, (size_t)h->dim * W, "tile diagonal");
+    if (rc == HD_OK) rc = get(&h->d_tg_diag, (size_t)h->dim * W, "tile diagonal");
     if (rc == HD_OK) {
         HD_ENQ(q, hipMemcpyAsync(h->d_tg_base, base.data(), base.size() * sizeof(int64_t), hipMemcpyHostToDevice, st));
         HD_ENQ(q, hipMemsetAsync(d_flag + 1, 0, sizeof(int), st));
 #define HD_TF(WV, QAV)                                                                                             \
     hipLaunchKernelGGL((k_tile_fill<TG, WV, QAV>), dim3((unsigned)G), dim3(kBuildThreads), 0, st, h->dim,            \
                        h->d_rowptr, h->d_col, h->d_code, static_cast<const double*>(h->d_diag), h->d_tg_base, G,     \
-                       h->d_tg_entries, h->d_tg_lines, h->d_tg_offs, h->d_tg_diag, d_flag + 1)
+                       d_keep, h->d_tg_entries, h->d_tg_lines, h->d_tg_offs, h->d_tg_diag, d_flag + 1)
         if (W == 2) HD_TF(2, false);
         else if (entry_bytes == 3) HD_TF(1, true);
         else HD_TF(1, false);
@@ -787,6 +825,8 @@ static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
             rc = fail(HD_ERR_HIP, "tiled layout build found inconsistent counts (flags " + std::to_string(flags[1]) +
                                       ")");
     }
+    dfree(d_keep);
+    d_keep = nullptr;
     if (rc == HD_OK && entry_bytes == 3 && h->tg_entries > 0) {
         // entries are a multiple of 4; two zero pad words let the SpMV read
         // the dword after any entry
