@@ -285,53 +285,96 @@ HD_DEV uint64_t unrank_state(const RankView& v, uint64_t r)
     return s;
 }
 
-HD_DEV uint32_t shfl_xor_key(uint32_t v, int m) { return (uint32_t)__shfl_xor((int)v, m); }
-HD_DEV uint64_t shfl_xor_key(uint64_t v, int m)
+// The pair (a, b) of v and its value in lane ^ m, in either order; m is a power of
+// two and a constant where the call is unrolled.  DPP moves within a row of 16 lanes
+// and lane swaps beyond (gfx950): no LDS, which a shuffle goes through.
+HD_DEV void lane_pair(uint32_t v, int m, uint32_t& a, uint32_t& b)
 {
-    const int lo = __shfl_xor((int)(uint32_t)v, m);
-    const int hi = __shfl_xor((int)(uint32_t)(v >> 32), m);
-    return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
+    a = v;
+    if (m == 1) b = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);       // quad 1 0 3 2
+    else if (m == 2) b = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);  // quad 2 3 0 1
+    else if (m == 4)                                                                        // ^ 7 (half mirror), ^ 3
+        b = (uint32_t)__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true), 0x1B, 0xF,
+                                               0xF, true);
+    else if (m == 8) b = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);  // rotation by 8 of 16
+    else {
+        const auto r = m == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
+                               : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        a = r[0];
+        b = r[1];
+    }
+}
+HD_DEV void lane_pair(uint64_t v, int m, uint64_t& a, uint64_t& b)
+{
+    uint32_t al, bl, ah, bh;
+    lane_pair((uint32_t)v, m, al, bl);
+    lane_pair((uint32_t)(v >> 32), m, ah, bh);
+    a = ((uint64_t)ah << 32) | al;
+    b = ((uint64_t)bh << 32) | bl;
 }
 
+// The smaller of a and b for z = 0, the larger for z = ~0 (one v_med3_u32).
+HD_DEV uint32_t pick(uint32_t a, uint32_t b, uint32_t z)
+{
+    const uint32_t lo = a < b ? a : b, hi = a < b ? b : a, hz = hi < z ? hi : z;
+    return lo > hz ? lo : hz;
+}
+HD_DEV uint64_t pick(uint64_t a, uint64_t b, uint32_t z) { return (a < b) == (z == 0u) ? a : b; }
+
 // Ascending bitonic sort of a wavefront's 512 keys, lane l holding elements
-// 8l .. 8l+7 in registers: distances below 8 within a lane, the others
-// between lanes (shfl_xor).
+// 8l .. 8l+7 in registers: distances below 8 within a lane, the others between
+// lanes.  The directions are lane masks (0 ascending, ~0 descending), so that a
+// 32-bit comparison is one instruction and a lane exchange one or two: with LDS
+// shuffles and compare-and-select the sort was a third of the 3,144 vector
+// instructions per row of the fill, which they bound (74% of its cycles).
 template <typename Key>
 HD_DEV void sort512_regs(Key (&key)[8], int lane)
 {
+    uint32_t bit[7];  // bit i of the lane as a mask
+#pragma unroll
+    for (int i = 0; i < 7; ++i) bit[i] = i < 6 ? 0u - (((uint32_t)lane >> i) & 1u) : 0u;
 #pragma unroll
     for (int k = 2; k <= 512; k <<= 1) {
 #pragma unroll
         for (int j = k >> 1; j > 0; j >>= 1) {
             if (j >= 8) {
-                const int lj = j >> 3;
-                const bool lower = (lane & lj) == 0;
+                const uint32_t z = bit[__builtin_ctz(k) - 3] ^ bit[__builtin_ctz(j) - 3];
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
-                    const Key other = shfl_xor_key(key[t], lj);
-                    const bool up = ((lane * 8 + t) & k) == 0;
-                    key[t] = (lower == up) ? (key[t] < other ? key[t] : other) : (key[t] > other ? key[t] : other);
+                    Key a, b;
+                    lane_pair(key[t], j >> 3, a, b);
+                    key[t] = pick(a, b, z);
                 }
             } else {
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
                     if (t & j) continue;
-                    const int t2 = t | j;
-                    const bool up = ((lane * 8 + t) & k) == 0;
-                    const Key a = key[t], b = key[t2];
-                    const Key lo = a < b ? a : b, hi = a < b ? b : a;
-                    key[t] = up ? lo : hi;
-                    key[t2] = up ? hi : lo;
+                    const uint32_t z = k >= 8 ? bit[__builtin_ctz(k) - 3] : (t & k) ? ~0u : 0u;
+                    const Key a = key[t], b = key[t | j];
+                    key[t] = pick(a, b, z);
+                    key[t | j] = pick(a, b, ~z);
                 }
             }
         }
     }
 }
 
+// One bitonic stage between lanes at distance M, for a lane's 8 keys.
+template <int M, typename Key>
+HD_DEV void lane_stage(Key (&key)[8], uint32_t z)
+{
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        Key a, b;
+        lane_pair(key[e], M, a, b);
+        key[e] = pick(a, b, z);
+    }
+}
+
 // Ascending bitonic sort of v[0, P) (P a power of two, P <= 8 * THREADS) by a
 // block of THREADS threads, in registers: thread t holds elements 8t .. 8t+7.
 // Stages of distance below 8 run within a thread, those below 512 between the
-// lanes of a wavefront (shfl_xor), and only the longer ones exchange through
+// lanes of a wavefront (lane_pair), and only the longer ones exchange through
 // v, with a barrier.  Elements from P to 8 * THREADS take part (as a separate
 // network) and must hold values that may move among themselves (all equal).
 template <typename Key, int THREADS>
@@ -342,29 +385,23 @@ HD_DEV void bitonic_blocked(Key* v, int P)
 #pragma unroll
     for (int e = 0; e < 8; ++e) a[e] = v[8 * t + e];
     for (int k = 2; k <= P; k <<= 1) {
+        // element 8t + e and its partner: distances and directions from 8 on depend on t alone
+        const uint32_t down = ((8 * t) & k) ? ~0u : 0u;
         for (int j = k >> 1; j >= 8; j >>= 1) {
+            const uint32_t z = down ^ (((8 * t) & j) ? ~0u : 0u);
             if (j >= 512) {
                 __syncthreads();
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[8 * t + e] = a[e];
                 __syncthreads();
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int i = 8 * t + e;
-                    const Key b = v[i ^ j];
-                    const bool keep_min = ((i & j) == 0) == ((i & k) == 0);
-                    a[e] = keep_min ? (a[e] < b ? a[e] : b) : (a[e] < b ? b : a[e]);
-                }
-            } else {
-                const int d = j >> 3;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int i = 8 * t + e;
-                    const Key b = shfl_xor_key(a[e], d);
-                    const bool keep_min = ((i & j) == 0) == ((i & k) == 0);
-                    a[e] = keep_min ? (a[e] < b ? a[e] : b) : (a[e] < b ? b : a[e]);
-                }
-            }
+                for (int e = 0; e < 8; ++e) a[e] = pick(a[e], v[(8 * t + e) ^ j], z);
+            } else if (j == 256) lane_stage<32>(a, z);
+            else if (j == 128) lane_stage<16>(a, z);
+            else if (j == 64) lane_stage<8>(a, z);
+            else if (j == 32) lane_stage<4>(a, z);
+            else if (j == 16) lane_stage<2>(a, z);
+            else lane_stage<1>(a, z);
         }
 #pragma unroll
         for (int j = 4; j >= 1; j >>= 1) {
@@ -372,12 +409,10 @@ HD_DEV void bitonic_blocked(Key* v, int P)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 if (e & j) continue;
-                const bool asc = ((8 * t + e) & k) == 0;
+                const uint32_t z = ((8 * t + e) & k) ? ~0u : 0u;
                 const Key lo = a[e], hi = a[e | j];
-                if ((lo > hi) == asc) {
-                    a[e] = hi;
-                    a[e | j] = lo;
-                }
+                a[e] = pick(lo, hi, z);
+                a[e | j] = pick(lo, hi, ~z);
             }
         }
     }

@@ -94,3 +94,19 @@ def test_matrix_free_paths(monkeypatch, path):
         y_free = hd.Hamiltonian(b, t, storage=hd.STORAGE_MATRIX_FREE).spmv(x)
         assert np.max(np.abs(y_free - y_crs)) <= 1e-13 * np.max(np.abs(y_crs))
 
+
+
+@pytest.mark.parametrize("n, two_s, v", [(2, 55, None), (3, 40, {1: 1.0}), (11, 16, None), (12, 15, {1: 1.0, 3: 0.3}),
+                                         (13, 18, {1: 1.0}), (6, 15, {13: 1.0})])
+def test_fill_pair_masks_bit_exact(oracle, n, two_s, v):
+    """The mask walk of the sphere's rows: one pair, 56 orbitals (sums of two beyond 63),
+    55, 66 and 78 pairs around the 64 of a pass, and tables with trimmed or absent entries."""
+    say("pair masks", n, two_s, v)
+    b, t = models.sphere_problem(n, two_s)
+    if v:
+        vm = np.zeros(two_s - 1)
+        vm[list(v)] = list(v.values())
+        t = models.sphere_tables(two_s, vm)
+    for storage, full in ((hd.STORAGE_UPPER_REF, False), (hd.STORAGE_FULL, True)):
+        ref = oracle.build(n, two_s + 1, b.states(), oracle.LAYOUT_SPHERE, two_s + 1, t.ktable, t.vtable, full=full)
+        _assert_crs_equal(hd.Hamiltonian(b, t, storage=storage), ref)
