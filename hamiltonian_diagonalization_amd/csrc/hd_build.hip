@@ -902,19 +902,6 @@ k_sort512(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __rest
     }
 }
 
-// Inclusive sum over the lanes of a wavefront (DPP: within rows of 16, then the row
-// ends into the rows after).
-HD_DEV int wave_scan(int v)
-{
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
-    return v;
-}
-
 // The fill and the row sort in one pass, for rows of at most 512 entries and
 // columns below 2^23: one wavefront per row walks the candidates as k_fill_wave
 // does, but keeps all of the row's hops in LDS, ranks them 64 at a time into

@@ -285,6 +285,19 @@ HD_DEV uint64_t unrank_state(const RankView& v, uint64_t r)
     return s;
 }
 
+// Inclusive sum over the lanes of a wavefront (DPP: within rows of 16, then the row
+// ends into the rows after).
+HD_DEV int wave_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
 // The pair (a, b) of v and its value in lane ^ m, in either order; m is a power of
 // two and a constant where the call is unrolled.  DPP moves within a row of 16 lanes
 // and lane swaps beyond (gfx950): no LDS, which a shuffle goes through.

@@ -39,6 +39,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -53,6 +55,7 @@ constexpr int kLineWords = 16;     // doubles per 128-byte line
 constexpr int kHashSlots = 8192;   // LDS hash set of a group's lines
 constexpr int kMaxLines = 5120;    // distinct lines per group (load factor 0.625)
 constexpr int kMaxChunks = kMaxLines / kTC;
+constexpr int kBitWords = 20480;   // LDS bitmap of all x lines (10.4M real rows, 5.2M complex)
 constexpr int kU = 8;              // entries each SpMV lane has in flight
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 constexpr int kBuildThreads = 1024;  // one build block per CU (its LDS): all 16 wavefronts hide latency
@@ -90,15 +93,25 @@ __device__ __forceinline__ int hash_find(const uint32_t* keys, uint32_t line)
     return -1;
 }
 
+// Words per group that pass 1 keeps for pass 2: the sorted lines, cum and the place
+// of the diagonal in every row.
+template <int TG> constexpr int kKeepWords = kMaxLines + kMaxChunks * TG + TG;
+
 // The plan of one row group, shared by both build passes: the sorted distinct
 // lines, their chunks (kTC consecutive lines each), entry counts per (chunk,
 // row), the per-chunk row starts T (chunk blocks padded to 4 entries) and the
 // row's entries in earlier chunks (cum).
 template <int TG>
 struct TilePlanLds {
-    uint32_t keys[kHashSlots];
+    union {
+        struct {
+            uint32_t keys[kHashSlots];
+            uint16_t rank_of[kHashSlots];
+        };
+        uint32_t bits[kBitWords];
+    };
     uint32_t sorted[kHashSlots];
-    uint16_t rank_of[kHashSlots];
+    int wsum[kBuildThreads / 64];
     uint32_t counts[kMaxChunks * TG];
     uint32_t cum[kMaxChunks * TG];
     uint32_t T[kMaxChunks * (TG + 1)];
@@ -125,19 +138,26 @@ __device__ __forceinline__ int row_of(const TilePlanLds<TG>& S, int nrows, int64
 // Builds the plan in LDS; S.flags != 0 when the group does not fit.
 // LS: log2 of the x values per 128-byte line (4 real, 3 complex).  QA: every
 // (chunk, row) block is padded to a multiple of 4 entries (the 3-byte layout,
-// read as 12-byte quads).  known: the group's sorted lines where an earlier pass
-// kept them, n_known of them; then no entry is read for them.
-template <int TG, int LS, bool QA>
+// read as 12-byte quads).
+//
+// BITS (the sector's lines fit the bitmap): the lines are a bitmap's set bits, which
+// come out in order; else a hash set, sorted.  known: the words kept by pass 1, with
+// n_known lines; then no entry is read for the plan.
+template <int TG, int LS, bool QA, bool BITS>
 __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const int64_t* __restrict__ rowptr,
                           const int32_t* __restrict__ col, const uint16_t* __restrict__ code, int64_t g,
                           const uint32_t* __restrict__ known, int n_known)
 {
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int64_t r0 = g * TG, r1 = min(r0 + TG, dim);
     const int nrows = (int)(r1 - r0);
-    for (int i = t; i < kHashSlots; i += kBuildThreads) {
-        S.keys[i] = kEmpty;
-        S.sorted[i] = kEmpty;
+    const int nbits = (int)(((dim + (1 << LS) - 1) >> LS) + 31) >> 5;  // words, with BITS
+    if (BITS && !known) {
+        for (int i = t; i < nbits; i += kBuildThreads) S.bits[i] = 0u;
+    } else {
+        for (int i = t; i < kHashSlots; i += kBuildThreads) S.keys[i] = kEmpty;
+        if (!known)
+            for (int i = t; i < kHashSlots; i += kBuildThreads) S.sorted[i] = kEmpty;
     }
     for (int i = t; i <= nrows; i += kBuildThreads) S.rp[i] = rowptr[r0 + i];
     for (int i = t; i < TG; i += kBuildThreads) S.dpos[i] = -1;
@@ -152,14 +172,10 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
             else atomicOr(&S.flags, 1);
         }
         if (t == 0) S.n_lines = n_known;
-        for (int r = t; r < nrows; r += kBuildThreads) {  // the diagonal entry, at column r0 + r
-            int64_t lo = S.rp[r], hi = S.rp[r + 1];
-            while (lo < hi) {
-                const int64_t mid = (lo + hi) >> 1;
-                if (col[mid] < r0 + r) lo = mid + 1;
-                else hi = mid;
-            }
-            if (lo < S.rp[r + 1] && col[lo] == r0 + r && code[lo] == 0xFFFFu) S.dpos[r] = lo;
+        for (int i = t; i < (n_known + kTC - 1) / kTC * TG; i += kBuildThreads) S.cum[i] = known[kMaxLines + i];
+        for (int r = t; r < nrows; r += kBuildThreads) {
+            const uint32_t d = known[kMaxLines + kMaxChunks * TG + r];
+            if (d != kEmpty) S.dpos[r] = S.rp[r] + d;
         }
         __syncthreads();
     } else {
@@ -182,12 +198,35 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
                     S.dpos[row_of(S, nrows, j)] = j;
                     continue;
                 }
-                if (hash_insert(S.keys, cv[u] >> LS) < 0) atomicOr(&S.flags, 1);
+                const uint32_t line = cv[u] >> LS;
+                if (BITS) {
+                    const uint32_t m = 1u << (line & 31u);  // most lines are already in: no atomic for them
+                    if ((int)(line >> 5) >= nbits) atomicOr(&S.flags, 1);  // no column of the sector
+                    else if (!(S.bits[line >> 5] & m)) atomicOr(&S.bits[line >> 5], m);
+                } else if (hash_insert(S.keys, line) < 0) {
+                    atomicOr(&S.flags, 1);
+                }
             }
         }
         __syncthreads();
-        {
-            const int lane = t & 63;
+        if (BITS) {
+            // each thread's run of words, its lines counted, then written from the sum before
+            const int W = (nbits + kBuildThreads - 1) / kBuildThreads, w0 = t * W, w1 = min(w0 + W, nbits);
+            int n = 0;
+            for (int w = w0; w < w1; ++w) n += __popc(S.bits[w]);
+            const int incl = wave_scan(n);
+            if (lane == 63) S.wsum[wave] = incl;
+            __syncthreads();
+            int pos = incl - n, total = 0;
+            for (int w = 0; w < kBuildThreads / 64; ++w) {
+                if (w < wave) pos += S.wsum[w];
+                total += S.wsum[w];
+            }
+            if (total <= kMaxLines)
+                for (int w = w0; w < w1; ++w)
+                    for (uint32_t m = S.bits[w]; m; m &= m - 1) S.sorted[pos++] = (uint32_t)w * 32u + __builtin_ctz(m);
+            if (t == 0) S.n_lines = total;
+        } else {
             for (int i = t; i < kHashSlots; i += kBuildThreads) {
                 const uint32_t k = S.keys[i];
                 const uint64_t m = __ballot(k != kEmpty);
@@ -203,28 +242,30 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
             __syncthreads();
             return;
         }
-        const int L = S.n_lines;
-        int P = 1;
-        while (P < L) P <<= 1;
-        if (P <= 8 * kBuildThreads) {
-            bitonic_blocked<uint32_t, kBuildThreads>(S.sorted, P);
-        } else {
-            for (int k = 2; k <= P; k <<= 1)
-                for (int jj = k >> 1; jj > 0; jj >>= 1) {
-                    for (int i = t; i < P; i += kBuildThreads) {
-                        const int ixj = i ^ jj;
-                        if (ixj > i) {
-                            const uint32_t a = S.sorted[i], b = S.sorted[ixj];
-                            if ((a > b) == ((i & k) == 0)) {
-                                S.sorted[i] = b;
-                                S.sorted[ixj] = a;
+        if (!BITS) {
+            const int L = S.n_lines;
+            int P = 1;
+            while (P < L) P <<= 1;
+            if (P <= 8 * kBuildThreads) {
+                bitonic_blocked<uint32_t, kBuildThreads>(S.sorted, P);
+            } else {
+                for (int k = 2; k <= P; k <<= 1)
+                    for (int jj = k >> 1; jj > 0; jj >>= 1) {
+                        for (int i = t; i < P; i += kBuildThreads) {
+                            const int ixj = i ^ jj;
+                            if (ixj > i) {
+                                const uint32_t a = S.sorted[i], b = S.sorted[ixj];
+                                if ((a > b) == ((i & k) == 0)) {
+                                    S.sorted[i] = b;
+                                    S.sorted[ixj] = a;
+                                }
                             }
                         }
+                        __syncthreads();
                     }
-                    __syncthreads();
-                }
+            }
+            for (int i = t; i < L; i += kBuildThreads) S.rank_of[hash_find(S.keys, S.sorted[i])] = (uint16_t)i;
         }
-        for (int i = t; i < L; i += kBuildThreads) S.rank_of[hash_find(S.keys, S.sorted[i])] = (uint16_t)i;
     }
     // the chunks: kTC consecutive lines each
     const int L = S.n_lines, nch = (L + kTC - 1) / kTC;
@@ -235,20 +276,42 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
     // of consecutive sorted lines, so the row's entries in chunks below c are
     // those with columns below chunk c's first column: cum is a binary search
     // of the row's columns (less its diagonal), and counts are differences.
-    for (int i = t; i < nch * TG; i += kBuildThreads) {
-        const int c = i / TG, r = i % TG;
-        uint32_t below = 0;
-        if (r < nrows && c > 0) {
-            const uint32_t bound = S.sorted[S.ls[c]] << LS;
-            int64_t lo = S.rp[r], hi = S.rp[r + 1];
-            while (lo < hi) {
-                const int64_t mid = (lo + hi) >> 1;
-                if ((uint32_t)col[mid] < bound) lo = mid + 1;
-                else hi = mid;
-            }
-            below = (uint32_t)(lo - S.rp[r]) - (S.dpos[r] >= 0 && S.dpos[r] < lo ? 1u : 0u);
+    if (!known) {  // a thread's searches side by side: their loads overlap
+        constexpr int Q = (kMaxChunks * TG + kBuildThreads - 1) / kBuildThreads;
+        const int64_t e1 = S.rp[nrows];
+        int64_t lo[Q], hi[Q];
+        uint32_t bound[Q];
+        bool more = false;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = q * kBuildThreads + t, c = i / TG, r = i % TG;
+            const bool on = i < nch * TG && r < nrows && c > 0;
+            lo[q] = on ? S.rp[r] : 0;
+            hi[q] = on ? S.rp[r + 1] : 0;
+            bound[q] = on ? S.sorted[S.ls[c]] << LS : 0u;
+            more = more || lo[q] < hi[q];
         }
-        S.cum[c * TG + r] = below;
+        while (more) {
+            uint32_t v[Q];
+#pragma unroll
+            for (int q = 0; q < Q; ++q) v[q] = (uint32_t)col[min((lo[q] + hi[q]) >> 1, e1 - 1)];
+            more = false;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                if (lo[q] >= hi[q]) continue;
+                const int64_t mid = (lo[q] + hi[q]) >> 1;
+                if (v[q] < bound[q]) lo[q] = mid + 1;
+                else hi[q] = mid;
+                more = more || lo[q] < hi[q];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = q * kBuildThreads + t, c = i / TG, r = i % TG;
+            if (i >= nch * TG) continue;
+            S.cum[i] = r < nrows && c > 0 ? (uint32_t)(lo[q] - S.rp[r]) - (S.dpos[r] >= 0 && S.dpos[r] < lo[q] ? 1u : 0u)
+                                          : 0u;
+        }
     }
     __syncthreads();
     for (int i = t; i < nch * TG; i += kBuildThreads) {
@@ -261,23 +324,33 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
         S.counts[c * TG + r] = n;
     }
     __syncthreads();
-    // T: per chunk, the row starts; chunk blocks start on 4-entry boundaries
-    if (t < nch) {
-        uint32_t run = 0;
-        for (int r = 0; r < TG; ++r) {
-            S.T[t * (TG + 1) + r] = run;
-            run += QA ? (S.counts[t * TG + r] + 3u) & ~3u : S.counts[t * TG + r];
+    // T: per chunk (a wavefront each), the row starts; chunk blocks start on 4-entry boundaries
+    for (int c = wave; c < nch; c += kBuildThreads / 64) {
+        constexpr int R = TG / 64;
+        int n[R], sum = 0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int v = (int)S.counts[c * TG + lane * R + k];
+            n[k] = QA ? (v + 3) & ~3 : v;
+            sum += n[k];
         }
-        S.T[t * (TG + 1) + TG] = run;  // chunk size, made absolute below
+        const int incl = wave_scan(sum);
+        int run = incl - sum;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            S.T[c * (TG + 1) + lane * R + k] = (uint32_t)run;
+            run += n[k];
+        }
+        if (lane == 63) S.T[c * (TG + 1) + TG] = (uint32_t)incl;  // chunk size, made absolute below
     }
     __syncthreads();
-    if (t == 0) {
-        uint32_t b = 0;
-        for (int c = 0; c < nch; ++c) {
-            S.cbase[c] = b;
-            b += (S.T[c * (TG + 1) + TG] + 3u) & ~3u;
-        }
-        S.cbase[nch] = b;
+    if (wave == 0) {
+        static_assert(kMaxChunks <= 64, "a lane per chunk");
+        const int v = lane < nch ? (int)((S.T[lane * (TG + 1) + TG] + 3u) & ~3u) : 0;
+        const int incl = wave_scan(v);
+        if (lane < nch) S.cbase[lane] = (uint32_t)(incl - v);
+        if (lane == nch - 1) S.cbase[nch] = (uint32_t)incl;
+        if (nch == 0 && lane == 0) S.cbase[0] = 0u;
     }
     __syncthreads();
     for (int i = t; i < nch * (TG + 1); i += kBuildThreads) S.T[i] += S.cbase[i / (TG + 1)];
@@ -285,12 +358,11 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
 }
 
 // Pass 1: per group, the distinct lines, the chunks and the padded entries.  keep (may
-// be null): kMaxLines words per group for its sorted lines, which pass 2 then reads
-// in place of finding them again from every entry (N=12, 2S=33: pass 2 37.4 -> 15.4
-// ms with these and the 1,024-thread blocks, pass 1 21.9 -> 18.5 ms with the blocks
-// alone).  Both passes are bound by the chains of dependent LDS reads per entry and
-// by the plan's searches.
-template <int TG, int LS, bool QA>
+// be null): kKeepWords per group for what of the plan pass 2 would otherwise find again
+// from every entry.  Both passes are bound by chains of dependent LDS and L2 reads, one
+// block per CU.  N=12, 2S=33: pass 1 21.9 -> 10.3 ms (the bitmap, searches side by side,
+// chunk tables by wavefronts, 1,024 threads instead of 512), pass 2 37.4 -> 11.8 ms.
+template <int TG, int LS, bool QA, bool BITS>
 __global__ void __launch_bounds__(kBuildThreads)
 k_tile_count(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
              const uint16_t* __restrict__ code, int64_t* __restrict__ n_lines, int64_t* __restrict__ n_entries,
@@ -298,9 +370,14 @@ k_tile_count(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __r
 {
     __shared__ TilePlanLds<TG> S;
     const int64_t g = blockIdx.x;
-    tile_plan<TG, LS, QA>(S, dim, rowptr, col, code, g, nullptr, 0);
-    if (keep && !S.flags)
-        for (int i = threadIdx.x; i < S.n_lines; i += kBuildThreads) keep[g * kMaxLines + i] = S.sorted[i];
+    tile_plan<TG, LS, QA, BITS>(S, dim, rowptr, col, code, g, nullptr, 0);
+    if (keep && !S.flags) {
+        uint32_t* k = keep + g * kKeepWords<TG>;
+        for (int i = threadIdx.x; i < S.n_lines; i += kBuildThreads) k[i] = S.sorted[i];
+        for (int i = threadIdx.x; i < S.n_chunks * TG; i += kBuildThreads) k[kMaxLines + i] = S.cum[i];
+        for (int r = threadIdx.x; r < TG; r += kBuildThreads)
+            k[kMaxLines + kMaxChunks * TG + r] = S.dpos[r] >= 0 ? (uint32_t)(S.dpos[r] - S.rp[r]) : kEmpty;
+    }
     if (threadIdx.x == 0) {
         n_lines[g] = S.n_lines;
         n_chunks[g] = S.n_chunks;
@@ -325,7 +402,7 @@ k_tile_fill(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __re
     const int t = threadIdx.x;
     const int64_t g = blockIdx.x;
     const int64_t lb = base[groups + 1 + g], ln = base[groups + 1 + g + 1] - lb;
-    tile_plan<TG, LS, QA>(S, dim, rowptr, col, code, g, keep ? keep + g * kMaxLines : nullptr, (int)ln);
+    tile_plan<TG, LS, QA, false>(S, dim, rowptr, col, code, g, keep ? keep + g * kKeepWords<TG> : nullptr, (int)ln);
     const int64_t r0 = g * TG, r1 = min(r0 + TG, dim);
     const int nrows = (int)(r1 - r0);
     const int64_t eb = base[g], en = base[g + 1] - eb;
@@ -743,23 +820,27 @@ static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
     if (rc == HD_OK) rc = dalloc_t(&d_ne, (size_t)G, "tile entry counts");
     if (rc == HD_OK) rc = dalloc_t(&d_nc, (size_t)G, "tile chunk counts");
     if (rc == HD_OK) rc = dalloc_t(&d_flag, 2, "tile flags");
-    // room for the groups' lines between the passes; without it pass 2 finds them again
+    // room for the groups' plans between the passes; without it pass 2 makes them again
     uint32_t* d_keep = nullptr;
-    if (rc == HD_OK && dalloc_t(&d_keep, (size_t)G * kMaxLines, "tile lines of pass 1") != HD_OK) d_keep = nullptr;
+    const char* plan = std::getenv("HD_TILE_PLAN");  // "hash": no bitmap, "again": nothing kept (as for larger sectors)
+    const bool again = plan && !std::strcmp(plan, "again"), hash = plan && !std::strcmp(plan, "hash");
+    if (rc == HD_OK && !again && dalloc_t(&d_keep, (size_t)G * kKeepWords<TG>, "tile plans of pass 1") != HD_OK) d_keep = nullptr;
     HipErrors q;
     std::vector<int64_t> nl(G), ne(G), nc(G);
     int flags[2] = {0, 0};
     if (rc == HD_OK) {
         HD_ENQ(q, hipMemsetAsync(d_flag, 0, 2 * sizeof(int), st));
-        if (h->is_complex)
-            hipLaunchKernelGGL((k_tile_count<TG, 3, false>), dim3((unsigned)G), dim3(kBuildThreads), 0, st, h->dim,
-                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_keep, d_flag);
-        else if (entry_bytes == 3)
-            hipLaunchKernelGGL((k_tile_count<TG, 4, true>), dim3((unsigned)G), dim3(kBuildThreads), 0, st, h->dim,
-                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_keep, d_flag);
-        else
-            hipLaunchKernelGGL((k_tile_count<TG, 4, false>), dim3((unsigned)G), dim3(kBuildThreads), 0, st, h->dim,
-                               h->d_rowptr, h->d_col, h->d_code, d_nl, d_ne, d_nc, d_keep, d_flag);
+        // the bitmap where the sector's lines fit it (no probing, no sort)
+        const int ls = h->is_complex ? 3 : 4;
+        const bool bits = !hash && ((h->dim + (1 << ls) - 1) >> ls) <= (int64_t)kBitWords * 32;
+#define HD_TC(LSV, QAV)                                                                                           \
+    hipLaunchKernelGGL((bits ? k_tile_count<TG, LSV, QAV, true> : k_tile_count<TG, LSV, QAV, false>),              \
+                       dim3((unsigned)G), dim3(kBuildThreads), 0, st, h->dim, h->d_rowptr, h->d_col, h->d_code,    \
+                       d_nl, d_ne, d_nc, d_keep, d_flag)
+        if (h->is_complex) HD_TC(3, false);
+        else if (entry_bytes == 3) HD_TC(4, true);
+        else HD_TC(4, false);
+#undef HD_TC
         HD_ENQ(q, hipGetLastError());
         HD_ENQ(q, hipMemcpyAsync(nl.data(), d_nl, G * sizeof(int64_t), hipMemcpyDeviceToHost, st));
         HD_ENQ(q, hipMemcpyAsync(ne.data(), d_ne, G * sizeof(int64_t), hipMemcpyDeviceToHost, st));
@@ -793,7 +874,7 @@ static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
     }
     auto get = [&](auto** ptr, size_t n, const char* what) {
         int r = dalloc_t(ptr, n, what);
-        if (r != HD_OK && d_keep) {  // the layout goes before the kept lines
+        if (r != HD_OK && d_keep) {  // the layout goes before the kept plans
             dfree(d_keep);
             d_keep = nullptr;
             r = dalloc_t(ptr, n, what);

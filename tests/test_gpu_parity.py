@@ -293,6 +293,33 @@ def test_tiled_spmv_and_lanczos_config1(oracle):
     assert np.array_equal(h.spmv(x, precision=hd.TILED), got)
 
 
+@pytest.mark.parametrize("n, two_s, rows", [(3, 6, 0), (7, 18, 64), (8, 21, 128)])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_tiled_plans_identical(monkeypatch, n, two_s, rows, cplx):
+    """The build's plans (bitmap or hash set of lines, kept for pass 2 or made again)
+    give the same layout: same sizes and the same product, bit for bit, on a part of
+    a group, a few and many groups."""
+    say("tiled plans", n, two_s, rows, cplx)
+    if cplx:
+        kt, vt, eps = models.ofl_tables(3, 4, 6)
+        b = hd.FockBasis(hd.Sector.k2d(1, 2, 3, 4), n if n < 7 else 6, 12)
+        t = hd.TermTables(hd.LAYOUT_OFL, 12, kt, vt, eps)
+    else:
+        b, t = models.sphere_problem(n, two_s)
+    x = np.random.default_rng(n).normal(size=b.dim) * (1 + 1j if cplx else 1)
+    got = []
+    for plan in ("", "hash", "again"):
+        monkeypatch.setenv("HD_TILE_PLAN", plan)
+        h = hd.Hamiltonian(b, t, storage=hd.STORAGE_FULL)
+        h.tile(rows)
+        info = h.tile_info()
+        got.append((info["entries"], info["lines"], h.spmv(x, precision=hd.TILED)))
+    y = h.spmv(x, precision=hd.F64)
+    for e, l, g in got:
+        assert (e, l) == got[0][:2] and np.array_equal(g, got[0][2])
+    assert np.max(np.abs(y - got[0][2])) <= 1e-13 * max(1.0, np.max(np.abs(y)))
+
+
 def test_tiled_block_orders_identical():
     """The block order only changes which workgroup runs a row group, so
     every order (launch order, windows with a partial last one, one window
