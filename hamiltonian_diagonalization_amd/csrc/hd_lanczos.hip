@@ -4,8 +4,9 @@
 // drives PARPACK p?naupd/p?neupd by reverse communication, WHICH = 'SR',
 // NCV = min(N, 2*NEV+21), exact shifts, maxiter 2000 (arpack_wrapper.cpp:38-49),
 // with every mat-vec a host round trip through MatrixVectorFunction::Simple.
-// Here the Krylov basis, the operator and all vector work stay in HBM; the host
-// only sees the small projected matrix.  Method: thick-restart Lanczos (Wu and
+// Here the Krylov basis, the operator and all vector work stay in HBM, and so do the
+// coefficients and decisions inside a cycle; the host queues the cycle's launches and
+// sees the small projected matrix at its end.  Method: thick-restart Lanczos (Wu and
 // Simon, SIAM J. Matrix Anal. Appl. 22 (2000) 602) with full
 // reorthogonalisation: each step first removes the three-term part locally
 // (w -= beta v_{j-1}; alpha = v_j.w; w -= alpha v_j), then one classical
@@ -13,8 +14,7 @@
 // drops by more than 100x (the DGKS criterion); the first step after a restart
 // (whose projection is the arrow, not tridiagonal) always takes two passes
 // (Giraud et al., Numer. Math. 101 (2005) 87).  The projected
-// tridiagonal-plus-arrow matrix is diagonalised by cyclic Jacobi rotations on
-// the host.
+// tridiagonal-plus-arrow matrix is diagonalised on the host.
 //
 // Mixed precision (precision = HD_F32) chooses the operator per restart
 // cycle.  An operator error F_j in the product of basis vector v_j enters the
@@ -33,7 +33,7 @@
 // f32_budget * tol * max(1, |theta_i|).  The prediction cannot see an
 // eigenvalue that enters the wanted window during the cycle, so the estimate
 // is checked again with the cycle's actual coefficients, and a cycle beyond
-// the budget is discarded (its starting state was kept) and run in FP64.
+// the budget is discarded (its starting state is still there) and run in FP64.
 // Convergence is the usual Ritz test;
 // the eigenpairs are then checked with the FP64 operator, and hd_lanczos
 // repeats the solve with the FP64 operator should a residual miss tol.  All

@@ -406,7 +406,7 @@ int hd_ham_tile_info(const hd_hamiltonian* h, hd_tile_info_t* info);
  * every XCD w consecutive row groups, so neighbouring groups, which read
  * mostly the same x lines, share an L2.  0 keeps the launch order; -1 times
  * the candidates (0, 16, 64, 256, one window over the grid) and keeps the
- * fastest, which hd_ham_tile also does after building the layout. */
+ * fastest.  hd_ham_tile sets 64 for layouts of at least 512 groups, else 0. */
 int hd_ham_tile_order(hd_hamiltonian* h, int64_t groups_per_xcd);
 /* Zero-copy view of the tiled layout: group bases (3 x (groups+1) int64:
  * entries, lines, offset table), entries (uint32 words, or with entry_bytes 3

@@ -109,4 +109,6 @@ def test_fill_pair_masks_bit_exact(oracle, n, two_s, v):
         t = models.sphere_tables(two_s, vm)
     for storage, full in ((hd.STORAGE_UPPER_REF, False), (hd.STORAGE_FULL, True)):
         ref = oracle.build(n, two_s + 1, b.states(), oracle.LAYOUT_SPHERE, two_s + 1, t.ktable, t.vtable, full=full)
-        _assert_crs_equal(hd.Hamiltonian(b, t, storage=storage), ref)
+        h = hd.Hamiltonian(b, t, storage=storage)
+        _assert_crs_equal(h, ref)
+        assert h.info()["n_trimmed"] == ref.n_trimmed
