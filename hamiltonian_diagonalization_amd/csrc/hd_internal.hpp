@@ -573,6 +573,6 @@ void jacobi_eigh(int n, std::vector<double>& A, std::vector<double>& w, std::vec
 bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<double>& Z, int row0 = 0);
 // Block thick-restart Lanczos for opts.block > 1 (hd_block.hip).
 int run_block_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* evals, hd_lanczos_stats* stats);
-int spmv_autotune(hd_hamiltonian* h, int formats = 7);  // bit p: format p (hd_precision)
+int spmv_autotune(hd_hamiltonian* h, int formats = 7, bool for_solve = false);  // bit p: format p (hd_precision)
 void lanczos_state_free(hd_lanczos_state* s);
 }  // namespace hd

@@ -1050,7 +1050,7 @@ static int run_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* eval
     int untuned = 0;
     for (int p : {L.prec64, mixed ? prec32 : L.prec64})
         if (p < HD_TILED && h->spmv_sched[p] < 0) untuned |= 1 << p;
-    if (!free_ && untuned) HD_CHECK(spmv_autotune(h, untuned));
+    if (!free_ && untuned) HD_CHECK(spmv_autotune(h, untuned, true));
     HD_CHECK(L.alloc(nev, mixed, mixed && prec32 == HD_F32));
     const double tol = o.tol > 0 ? o.tol : 1e-10;
     const double budget = o.f32_budget > 0 ? std::min(o.f32_budget, 1.0) : 1.0;

@@ -285,25 +285,25 @@ __global__ void __launch_bounds__(256) k_stream_copy(const int4* __restrict__ sr
 }
 
 // Times every schedule on the requested formats of the matrix (bit p of `formats`:
-// format p) and keeps the fastest of each.
+// format p) and keeps the fastest of each.  for_solve: the caller makes some hundred
+// products at most, so below kTuneNnz entries, where a product is one short wave of
+// blocks (N=8, 2S=21, 0.9M entries: 5.5 us with 32 lanes per row, 5.6-6.7 us with 16)
+// and timing the nine schedules of a format costs 36 of them, the row length chooses.
+// Products on request are always timed first: a solver's choice is up to 9% slower for
+// them, so it leaves lanes_per_row open.
 constexpr int64_t kTuneNnz = (int64_t)1 << 22;
 
-int spmv_autotune(hd_hamiltonian* h, int formats)
+int spmv_autotune(hd_hamiltonian* h, int formats, bool for_solve)
 {
     if (h->storage == HD_STORAGE_MATRIX_FREE) {  // one kernel, nothing to choose
         h->lanes_per_row = 1;
         return HD_OK;
     }
     const bool have[3] = {h->d_val64 != nullptr, h->d_val32 != nullptr, h->d_code != nullptr};
-    // Below kTuneNnz entries a product is one short wave of blocks (N=8, 2S=21,
-    // 0.9M entries: 5.5 us with 32 lanes per row, 5.6-6.7 us with 16) and timing
-    // the nine schedules of a format costs 36 of them: lanes by the row length.
-    if (h->nnz < kTuneNnz) {
+    if (for_solve && h->nnz < kTuneNnz) {
         const double avg = h->dim ? (double)h->nnz / (double)h->dim : 0.0;
         for (int prec = 0; prec < 3; ++prec)
             if (have[prec] && (formats >> prec & 1)) h->spmv_sched[prec] = sched_for_lanes(avg > 24 ? 32 : 16);
-        const int si = h->spmv_sched[default_precision(h)];
-        if (formats >> default_precision(h) & 1) h->lanes_per_row = kScheds[si >= 0 ? si : pick_default_sched(h)].lpr;
         return HD_OK;
     }
     // one schedule per requested resident value format, each timed on zero vectors
