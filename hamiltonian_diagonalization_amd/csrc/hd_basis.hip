@@ -62,12 +62,13 @@ struct PoolDevice {
 };
 
 struct Pool {
-    struct Live {
+    struct Block {
         size_t bytes;
         int dev;
+        bool live;  // handed out; false while it is returned and idle
     };
     std::mutex mu;
-    std::unordered_map<void*, Live> live;
+    std::unordered_map<void*, Block> blocks;  // every block that the driver has given and not got back
     std::unordered_map<hipStream_t, int> stream_dev;
     PoolDevice dev[kPoolDevices];
 };
@@ -88,12 +89,13 @@ size_t pool_size(size_t bytes)
 }
 
 // Takes idle blocks of `d` (largest first) until at most `keep` bytes stay.
-void pool_take_excess(PoolDevice& d, size_t keep, std::vector<void*>& out)
+void pool_take_excess(Pool& P, PoolDevice& d, size_t keep, std::vector<void*>& out)
 {
     while (d.idle_bytes > keep && !d.idle.empty()) {
         auto it = std::prev(d.idle.end());
         d.idle_bytes -= it->first;
         out.push_back(it->second);
+        P.blocks.erase(it->second);
         d.idle.erase(it);
     }
 }
@@ -144,7 +146,7 @@ int dalloc(void** p, size_t bytes, const char* what)
             auto it = d.idle.lower_bound(need);
             if (it != d.idle.end() && it->first <= need + need / 8) {
                 *p = it->second;
-                P.live[*p] = {it->first, dev};
+                P.blocks[*p].live = true;
                 d.live_bytes += it->first;
                 d.idle_bytes -= it->first;
                 d.idle.erase(it);
@@ -158,7 +160,7 @@ int dalloc(void** p, size_t bytes, const char* what)
             std::vector<void*> drop;
             {
                 std::lock_guard<std::mutex> lock(P.mu);
-                pool_take_excess(P.dev[dev], 0, drop);
+                pool_take_excess(P, P.dev[dev], 0, drop);
             }
             for (void* q : drop) (void)hipFree(q);
             got = std::max<size_t>(bytes, 16);  // without the rounding: what was asked for may still fit
@@ -166,7 +168,7 @@ int dalloc(void** p, size_t bytes, const char* what)
         }
         if (e == hipSuccess) {
             std::lock_guard<std::mutex> lock(P.mu);
-            P.live[*p] = {got, dev};
+            P.blocks[*p] = {got, dev, true};
             P.dev[dev].live_bytes += got;
             return HD_OK;
         }
@@ -181,13 +183,16 @@ hipError_t dfree_status(void* p)
 {
     if (!p) return hipSuccess;
     Pool& P = pool();
-    Pool::Live b;
+    Pool::Block b;
     {
         std::lock_guard<std::mutex> lock(P.mu);
-        auto it = P.live.find(p);
-        if (it == P.live.end()) return hipFree(p);  // not from dalloc: the driver reports it
+        auto it = P.blocks.find(p);
+        if (it == P.blocks.end()) return hipFree(p);  // not from dalloc: the driver's answer
+        // Given back already.  The driver still has the block as allocated and would
+        // free it under the idle list.
+        if (!it->second.live) return hipErrorInvalidValue;
+        it->second.live = false;
         b = it->second;
-        P.live.erase(it);
         P.dev[b.dev].live_bytes -= b.bytes;
     }
     hipError_t e = hipSuccess;
@@ -201,9 +206,10 @@ hipError_t dfree_status(void* p)
                 d.idle.emplace(b.bytes, p);
                 d.idle_bytes += b.bytes;
             } else {
+                P.blocks.erase(p);
                 drop.push_back(p);
             }
-            if (d.live_bytes == 0) pool_take_excess(d, kKeepBytes, drop);
+            if (d.live_bytes == 0) pool_take_excess(P, d, kKeepBytes, drop);
         }
         for (void* q : drop) {
             const hipError_t f = hipFree(q);

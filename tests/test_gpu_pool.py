@@ -87,3 +87,21 @@ def test_builds_in_a_loop_are_identical():
             got = [*h.crs(), h.spmv(x, precision=hd.TILED), h.spmv(x, precision=hd.CODED)]
             for a, w in zip(got, want.setdefault(n, got)):
                 assert np.array_equal(a, w)
+
+
+@pytest.mark.parametrize("nbytes", [64, 3 << 20])
+def test_second_free_is_an_error(nbytes):
+    """A pointer given back twice is refused the second time, as the driver refuses it,
+    and its block goes to one owner only."""
+    say("pool: block of", nbytes, "given back twice")
+    L = hd.lib()
+    keep = hd.DeviceBuffer(16)
+    p = ctypes.c_void_p()
+    assert L.hd_malloc(ctypes.byref(p), nbytes) == hd.HD_OK
+    assert L.hd_free(p) == hd.HD_OK
+    assert L.hd_free(p) == hd.HD_ERR_HIP
+    a, b = (np.full(nbytes, k, dtype=np.uint8) for k in (3, 5))
+    da, db = hd.DeviceBuffer.from_array(a), hd.DeviceBuffer.from_array(b)
+    assert da.ptr.value != db.ptr.value
+    assert np.array_equal(da.to_array(np.uint8, nbytes), a) and np.array_equal(db.to_array(np.uint8, nbytes), b)
+    del keep
