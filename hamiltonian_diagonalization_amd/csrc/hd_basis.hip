@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdint>
 #include <cstring>
 #include <iterator>
 #include <map>
@@ -79,10 +80,12 @@ Pool& pool()
     return *p;
 }
 
-// Powers of two up to 1 MiB, then multiples of 2 MiB.
+// Powers of two up to 1 MiB, then multiples of 2 MiB; 0 where that exceeds size_t.
 size_t pool_size(size_t bytes)
 {
-    if (bytes > (size_t)1 << 20) return (bytes + ((size_t)2 << 20) - 1) / ((size_t)2 << 20) * ((size_t)2 << 20);
+    constexpr size_t step = (size_t)2 << 20;
+    if (bytes > SIZE_MAX - (step - 1)) return 0;
+    if (bytes > (size_t)1 << 20) return (bytes + step - 1) / step * step;
     size_t s = 256;
     while (s < bytes) s <<= 1;
     return s;
@@ -139,6 +142,7 @@ int dalloc(void** p, size_t bytes, const char* what)
     if (e == hipSuccess && (dev < 0 || dev >= kPoolDevices)) e = hipErrorInvalidDevice;
     if (e == hipSuccess) e = pool_device(dev);
     const size_t need = pool_size(bytes);
+    if (e == hipSuccess && !need) e = hipErrorOutOfMemory;
     if (e == hipSuccess) {
         {
             std::lock_guard<std::mutex> lock(P.mu);

@@ -105,3 +105,12 @@ def test_second_free_is_an_error(nbytes):
     assert da.ptr.value != db.ptr.value
     assert np.array_equal(da.to_array(np.uint8, nbytes), a) and np.array_equal(db.to_array(np.uint8, nbytes), b)
     del keep
+
+
+@pytest.mark.parametrize("nbytes", [-1, -(1 << 20), 1 - (2 << 20)])
+def test_sizes_beyond_rounding_are_refused(nbytes):
+    """Sizes in the last 2 MiB of size_t, where rounding up to whole blocks would wrap."""
+    say("pool: block of", nbytes % (1 << 64))
+    with pytest.raises(hd.HDError) as e:
+        hd.DeviceBuffer(nbytes)
+    assert e.value.code == hd.HD_ERR_NOMEM
