@@ -108,6 +108,7 @@ SIGNATURES = {
     "hd_version": (ctypes.c_int, []),
     "hd_malloc": (ctypes.c_int, [_PP, ctypes.c_size_t]),
     "hd_free": (ctypes.c_int, [_P]),
+    "hd_mem_trim": (ctypes.c_int, [ctypes.c_size_t, ctypes.POINTER(ctypes.c_size_t)]),
     "hd_memcpy_h2d": (ctypes.c_int, [_P, _P, ctypes.c_size_t]),
     "hd_memcpy_d2h": (ctypes.c_int, [_P, _P, ctypes.c_size_t]),
     "hd_memset": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_size_t]),
@@ -245,6 +246,14 @@ class DeviceBuffer:
         if getattr(self, "ptr", None) is not None and _lib is not None:
             _lib.hd_free(self.ptr)
             self.ptr = None
+
+
+def trim_memory(keep_bytes: int = 0) -> int:
+    """Give the idle device blocks that the library keeps for its next calls back to
+    the driver until at most keep_bytes are idle; returns the bytes still idle."""
+    idle = ctypes.c_size_t()
+    _check(lib().hd_mem_trim(keep_bytes, ctypes.byref(idle)))
+    return idle.value
 
 
 # --------------------------------------------------------------------- sectors

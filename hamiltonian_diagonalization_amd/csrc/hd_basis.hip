@@ -352,6 +352,8 @@ int hd_free(void* d_ptr)
     return HD_OK;
 }
 
+int hd_mem_trim(size_t keep_bytes, size_t* idle_bytes) { return pool_trim(keep_bytes, idle_bytes); }
+
 int hd_memcpy_h2d(void* d, const void* h, size_t bytes)
 {
     HD_HIP(hipMemcpy(d, h, bytes, hipMemcpyHostToDevice));

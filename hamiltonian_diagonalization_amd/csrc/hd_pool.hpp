@@ -1,9 +1,10 @@
 // The library's device blocks and streams, included by hd_basis.hip.  It calls the HIP
-// runtime only through hipMalloc, hipFree, the device and the stream
+// runtime only through hipMalloc, hipFree, hipMemGetInfo, the device and the stream
 // calls, so the bookkeeping also compiles against a stand-in runtime on the CPU.
 #pragma once
 
 #include <algorithm>
+#include <chrono>
 #include <cstdint>
 #include <iterator>
 #include <map>
@@ -24,20 +25,28 @@ namespace hd {
 // build + tiled layout + product 190-770 -> 190 ms.  A stream costs about 0.5 ms
 // to create and destroy (57 builds of a batch: 348 -> 317 ms with the solve).
 //
-// Bounds: idle blocks of a device never exceed a sixth of its memory, and go back to
-// the driver down to kKeepBytes when the device's last live block is returned, and
-// entirely when an allocation fails.  A returned block is idle only after the
-// whole device has finished its work (hipFree waits in the same way), so it may
-// be handed to any thread and any stream.  The pool is never destroyed: handles
-// may be released while the process ends.
+// Bounds: idle blocks of a device never exceed a sixth of its memory, nor, above
+// kUnasked, a quarter of what would be free without them when a block is returned, so
+// that other allocators of the process and other processes find three quarters of it.
+// The driver's answer takes 10 us (asked at each return, a build of 0.9 GB was 3% and a
+// basis of 8,512 states 30% slower), so it stands for kAskAgain.  They go back to the
+// driver down to kKeepBytes when the device's last live block is returned, entirely
+// when an allocation of the library fails, and on request (hd_mem_trim).  A returned
+// block is idle only after the whole device has finished its work (hipFree waits in
+// the same way), so it may be handed to any thread and any stream.  The pool is never
+// destroyed: handles may be released while the process ends.
 namespace {
 constexpr int kPoolDevices = 64;
 constexpr size_t kKeepBytes = (size_t)256 << 20;
+constexpr size_t kUnasked = (size_t)1 << 30;
+constexpr std::chrono::milliseconds kAskAgain(10);
 constexpr size_t kKeepStreams = 64;  // idle streams per device
 
 struct PoolDevice {
     std::multimap<size_t, void*> idle;  // by size
     size_t idle_bytes = 0, live_bytes = 0, cap = 0;
+    size_t bound = 0;  // of idle_bytes, as of `asked`
+    std::chrono::steady_clock::time_point asked;
     std::vector<hipStream_t> streams;
     int n_cu = 0;
     size_t max_lds = 0;
@@ -187,14 +196,26 @@ hipError_t dfree_status(void* p)
         {
             std::lock_guard<std::mutex> lock(P.mu);
             PoolDevice& d = P.dev[b.dev];
-            if (e == hipSuccess && d.idle_bytes + b.bytes <= d.cap) {
+            const size_t all = d.idle_bytes + b.bytes;
+            size_t bound = d.live_bytes ? std::min(d.cap, kUnasked) : kKeepBytes;
+            if (d.live_bytes && all > bound) {
+                const auto now = std::chrono::steady_clock::now();
+                if (all > d.bound || now - d.asked > kAskAgain) {
+                    size_t free_ = 0, total = 0;
+                    if (hipMemGetInfo(&free_, &total) != hipSuccess) free_ = 0;
+                    d.bound = std::min(d.cap, std::max(kUnasked, (free_ + all) / 4));
+                    d.asked = now;
+                }
+                bound = d.bound;
+            }
+            if (e == hipSuccess && all <= bound) {
                 d.idle.emplace(b.bytes, p);
                 d.idle_bytes += b.bytes;
             } else {
                 P.blocks.erase(p);
                 drop.push_back(p);
             }
-            if (d.live_bytes == 0) pool_take_excess(P, d, kKeepBytes, drop);
+            pool_take_excess(P, d, bound, drop);
         }
         for (void* q : drop) {
             const hipError_t f = hipFree(q);
@@ -205,6 +226,28 @@ hipError_t dfree_status(void* p)
 }
 
 void dfree(void* p) { (void)dfree_status(p); }
+
+// hd_mem_trim
+int pool_trim(size_t keep, size_t* idle)
+{
+    int dev = -1;
+    HD_HIP(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kPoolDevices) return fail(HD_ERR_HIP, "device index beyond the pool's table");
+    Pool& P = pool();
+    std::vector<void*> drop;
+    {
+        std::lock_guard<std::mutex> lock(P.mu);
+        pool_take_excess(P, P.dev[dev], keep, drop);
+        if (idle) *idle = P.dev[dev].idle_bytes;
+    }
+    hipError_t e = hipSuccess;
+    for (void* q : drop) {
+        const hipError_t f = hipFree(q);
+        if (e == hipSuccess) e = f;
+    }
+    HD_HIP(e);
+    return HD_OK;
+}
 
 hipError_t stream_get(hipStream_t* s)
 {

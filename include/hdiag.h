@@ -114,6 +114,12 @@ int hd_version(void);
 /* Device buffers for hosts without their own device allocator. */
 int hd_malloc(void** d_ptr, size_t bytes);
 int hd_free(void* d_ptr);
+/* The library keeps device blocks that its calls return (and hd_free) for the next
+ * calls: at most a sixth of the device, above 1 GiB at most a quarter of what is free
+ * without them, and 256 MiB once nothing is in use.  hd_mem_trim gives the idle blocks of the
+ * current device back to the driver until at most keep_bytes are idle (0: all), for
+ * other allocators in the process; *idle_bytes (nullable) is what stays. */
+int hd_mem_trim(size_t keep_bytes, size_t* idle_bytes);
 int hd_memcpy_h2d(void* d_dst, const void* h_src, size_t bytes);
 int hd_memcpy_d2h(void* h_dst, const void* d_src, size_t bytes);
 int hd_memset(void* d_dst, int value, size_t bytes);

@@ -186,10 +186,38 @@ static bool bounded()
     return ok && used() <= 256 * kMiB;  // nothing is in use
 }
 
+// Most of the device in use: what is returned leaves three quarters of the rest.
+static bool quarter()
+{
+    void *keep = get(16), *big = get(5 * kGiB);
+    std::vector<void*> v;
+    for (int i = 0; i < 6; ++i) v.push_back(get(kGiB));
+    const size_t rest = kTotal - used() + 6 * kGiB;
+    for (void* p : v) dfree(p);
+    const bool ok = kTotal - used() >= rest * 3 / 4 && used() >= 6 * kGiB;  // some of it is kept
+    dfree(big);
+    dfree(keep);
+    return ok;
+}
+
+static bool trim()
+{
+    void* keep = get(16);
+    std::vector<void*> v;
+    for (int i = 0; i < 4; ++i) v.push_back(get(kGiB / 4));
+    for (void* p : v) dfree(p);
+    size_t idle = 0;
+    bool ok = used() >= kGiB && pool_trim(kGiB / 2, &idle) == HD_OK && idle <= kGiB / 2 && idle >= kGiB / 4;
+    ok = ok && pool_trim(0, &idle) == HD_OK && idle == 0 && used() < kMiB;
+    dfree(keep);
+    return ok && pool_trim(0, nullptr) == HD_OK && used() == 0;
+}
+
 int main(int argc, char** argv)
 {
     const std::pair<const char*, bool (*)()> checks[] = {
-        {"threads", threads}, {"twice", twice}, {"sizes", sizes}, {"drain", drain}, {"bounded", bounded}};
+        {"threads", threads}, {"twice", twice}, {"sizes", sizes}, {"drain", drain}, {"bounded", bounded},
+        {"quarter", quarter}, {"trim", trim}};
     for (const auto& c : checks)
         if (argc == 2 && !std::strcmp(argv[1], c.first)) return c.second() ? 0 : 1;
     return 2;

@@ -2,6 +2,8 @@
 threads, blocks of every size class, and the bound on what it keeps."""
 import ctypes
 import gc
+import os
+import subprocess
 import sys
 import threading
 
@@ -116,3 +118,63 @@ def test_sizes_beyond_rounding_are_refused(nbytes):
     with pytest.raises(hd.HDError) as e:
         hd.DeviceBuffer(nbytes)
     assert e.value.code == hd.HD_ERR_NOMEM
+
+
+def test_idle_blocks_leave_three_quarters_of_the_free_memory():
+    """With most of the card in use, returned blocks go back to the driver: another
+    allocator finds at least three quarters of what is not in use."""
+    say("pool: 4 blocks of 8 GiB returned beside a large one")
+    gc.collect()
+    keep = hd.DeviceBuffer(16)
+    hd.trim_memory()
+    blocks = [hd.DeviceBuffer(8 << 30) for _ in range(4)]
+    ballast = hd.DeviceBuffer(_mem_info()[0] - (20 << 30))
+    not_in_use = _mem_info()[0] + (32 << 30)
+    del blocks
+    assert _mem_info()[0] >= not_in_use * 3 // 4 - (1 << 28)
+    del ballast, keep
+
+
+def test_trim_gives_idle_blocks_back():
+    say("pool: trim of 4 idle GiB")
+    gc.collect()
+    keep = hd.DeviceBuffer(16)
+    hd.trim_memory()
+    free0 = _mem_info()[0]
+    for b in [hd.DeviceBuffer(1 << 30) for _ in range(4)]:
+        del b
+    assert _mem_info()[0] <= free0 - (3 << 30)  # idle in the library
+    assert hd.trim_memory(1 << 30) <= 1 << 30
+    assert _mem_info()[0] >= free0 - (1 << 30) - (1 << 26)
+    assert hd.trim_memory() == 0
+    assert _mem_info()[0] >= free0 - (1 << 26)
+    del keep
+
+
+def test_allocation_takes_idle_blocks_of_other_sizes_back():
+    """A request that fits only without the idle blocks succeeds."""
+    say("pool: 4 idle blocks of 8 GiB in the way of a large one")
+    gc.collect()
+    keep = hd.DeviceBuffer(16)
+    hd.trim_memory()
+    free0 = _mem_info()[0]
+    blocks = [hd.DeviceBuffer(8 << 30) for _ in range(4)]
+    del blocks
+    free1 = _mem_info()[0]
+    assert free1 <= free0 - (30 << 30)
+    big = hd.DeviceBuffer(free1 + (10 << 30))
+    del big, keep
+
+
+def test_last_block_returns_the_pool():
+    """When nothing is in use any more, at most 256 MiB stay idle."""
+    say("pool: last block returned in a process of its own")
+    code = ("import hamiltonian_diagonalization_amd as hd\n"
+            "keep = hd.DeviceBuffer(16)\n"
+            "b = hd.DeviceBuffer(2 << 30)\n"
+            "del b\n"
+            "assert hd.trim_memory(1 << 40) >= 2 << 30\n"
+            "del keep\n"
+            "assert hd.trim_memory(1 << 40) <= 256 << 20\n")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run([sys.executable, "-c", code], cwd=root, check=True, timeout=100)

@@ -18,6 +18,6 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["threads", "twice", "sizes", "drain", "bounded"])
+@pytest.mark.parametrize("name", ["threads", "twice", "sizes", "drain", "bounded", "quarter", "trim"])
 def test_pool(check, name):
     assert subprocess.run([check, name], timeout=100).returncode == 0
