@@ -503,8 +503,8 @@ struct hd_hamiltonian {
     void* d_diag = nullptr;   // double or double2, dim entries
     void* d_dict = nullptr;   // double or double2, ndict entries
     int ndict = 0;
-    int lanes_per_row = 0;    // SpMV lanes per row (0 = pick on first use)
-    int spmv_sched[4] = {-1, -1, -1, -1};  // SpMV schedule per precision (hd_precision); -1 = default
+    int sched_chosen = 0;                  // bit p: format p's schedule was timed or set
+    int spmv_sched[4] = {-1, -1, -1, -1};  // SpMV schedule per precision (hd_precision); -1 = by row length
     // tiled coded layout (hd_tiled.hip): row groups, x lines staged in LDS
     int64_t tg_groups = 0, tg_entries = 0, tg_lines = 0, tg_offs = 0;
     int tg_rows = 0;  // rows per group (128, or 64 for denser matrices)
@@ -573,6 +573,8 @@ void jacobi_eigh(int n, std::vector<double>& A, std::vector<double>& w, std::vec
 bool sym_eig(int n, std::vector<double>& A, std::vector<double>& w, std::vector<double>& Z, int row0 = 0);
 // Block thick-restart Lanczos for opts.block > 1 (hd_block.hip).
 int run_block_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* evals, hd_lanczos_stats* stats);
-int spmv_autotune(hd_hamiltonian* h, int formats = 7, bool for_solve = false);  // bit p: format p (hd_precision)
+constexpr int kAllFormats = 7;                       // bit p: format p (hd_precision)
+constexpr int64_t kLongNnz = (int64_t)1 << 22;       // entries from which a product is long (hd_spmv.hip)
+int spmv_autotune(hd_hamiltonian* h, int formats);
 void lanczos_state_free(hd_lanczos_state* s);
 }  // namespace hd

@@ -1046,11 +1046,12 @@ static int run_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* eval
                : (o.precision == HD_TILED || (mixed && h->d_tg_base)) ? HD_TILED
                : (o.precision == HD_CODED || !h->d_val64) ? (h->d_code ? HD_CODED : HD_TILED)
                                                           : HD_F64;
-    // schedules of the CRS formats that the solve uses, where not chosen yet
+    // a long solve times the schedules of the CRS formats that it uses
     int untuned = 0;
     for (int p : {L.prec64, mixed ? prec32 : L.prec64})
-        if (p < HD_TILED && h->spmv_sched[p] < 0) untuned |= 1 << p;
-    if (!free_ && untuned) HD_CHECK(spmv_autotune(h, untuned, true));
+        if (p < HD_TILED) untuned |= 1 << p;
+    untuned &= ~h->sched_chosen;
+    if (!free_ && untuned && h->nnz >= kLongNnz) HD_CHECK(spmv_autotune(h, untuned));
     HD_CHECK(L.alloc(nev, mixed, mixed && prec32 == HD_F32));
     const double tol = o.tol > 0 ? o.tol : 1e-10;
     const double budget = o.f32_budget > 0 ? std::min(o.f32_budget, 1.0) : 1.0;
@@ -1362,7 +1363,6 @@ int hd_lanczos(hd_hamiltonian* h, const hd_lanczos_opts* opts, double* h_evals, 
     if (h->storage == HD_STORAGE_MATRIX_FREE && (opts->precision != HD_F64 || opts->block > 1))
         return fail(HD_ERR_ARG, "matrix-free storage runs the single-vector Lanczos in FP64 (precision HD_F64)");
     if (opts->block > 1) {
-        if (!h->lanes_per_row) HD_CHECK(spmv_autotune(h));
         return run_block_lanczos(h, *opts, h_evals, stats);
     }
     auto run = [&](const hd_lanczos_opts& o, hd_lanczos_stats* s) {

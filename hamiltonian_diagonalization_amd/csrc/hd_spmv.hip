@@ -227,13 +227,29 @@ static int sched_for_lanes(int lpr)
     return 5;
 }
 
-static int pick_default_sched(const hd_hamiltonian* h)
+// The schedule of a format that was neither timed nor set, by row length.  Against
+// the fastest of the nine, over 45 matrices (sphere, lattice, two-level and random lists;
+// 10 to 1,001,402 rows, 3 to 307 entries per row) in every format, with the 3.4 us
+// that a call takes at least: 1.02 times on average, 1.17 at worst (4 lanes, 7 entries
+// per row).  4 lanes lose from 10 entries per row on (1.08-1.24), 8 from 18 on (1.12-1.23),
+// 16 from 38 on (1.03-1.4).  Long products (kLongNnz entries) hide more latency with 1,024
+// threads (up to 1.18), and there 64 lanes win for complex FP64 rows alone (1.00 against
+// 1.04-1.16).  Complex products of up to 6,144 rows leave lanes idle: 64 per row are 3-12%
+// faster than 32 at 450-4,751 rows, 1-8% slower in FP64 and 39% coded at 7,084.
+static int pick_default_sched(const hd_hamiltonian* h, int precision)
 {
     const double avg = h->dim ? (double)h->nnz / (double)h->dim : 0.0;
-    if (avg > 96) return 5;  // 32 lanes, 512 threads
-    if (avg > 48) return 3;
-    if (avg > 24) return 1;
-    return 0;
+    if (avg <= 8) return 0;
+    if (avg <= 16) return 1;
+    if (avg <= 32) return 3;
+    if (h->nnz >= kLongNnz) return h->is_complex && precision == HD_F64 && avg > 100 ? 8 : 6;
+    if (h->is_complex && h->dim <= 6144) return 7;
+    return 5;  // 32 lanes, 512 threads
+}
+
+static int sched_of(const hd_hamiltonian* h, int precision)
+{
+    return h->spmv_sched[precision] >= 0 ? h->spmv_sched[precision] : pick_default_sched(h, precision);
 }
 
 int spmv_launch(const hd_hamiltonian* h, int precision, const void* x, void* y, hipStream_t stream)
@@ -246,7 +262,7 @@ int spmv_launch(const hd_hamiltonian* h, int precision, const void* x, void* y, 
         return fail(HD_ERR_ARG, "SpMV needs full (both-triangle) storage");
     if (precision < 0 || precision > HD_TILED_X32) return fail(HD_ERR_ARG, "unknown SpMV precision");
     if (precision == HD_TILED || precision == HD_TILED_X32) return tiled_launch(h, x, y, stream, precision == HD_TILED_X32);
-    const int si = h->spmv_sched[precision] >= 0 ? h->spmv_sched[precision] : pick_default_sched(h);
+    const int si = sched_of(h, precision);
     if (h->dim == 0) return HD_OK;
     if (precision == HD_CODED) {
         if (!h->d_code) return fail(HD_ERR_ARG, "no coded values resident (value_mask & 4)");
@@ -285,27 +301,18 @@ __global__ void __launch_bounds__(256) k_stream_copy(const int4* __restrict__ sr
 }
 
 // Times every schedule on the requested formats of the matrix (bit p of `formats`:
-// format p) and keeps the fastest of each.  for_solve: the caller makes some hundred
-// products at most, so below kTuneNnz entries, where a product is one short wave of
-// blocks (N=8, 2S=21, 0.9M entries: 5.5 us with 32 lanes per row, 5.6-6.7 us with 16)
-// and timing the nine schedules of a format costs 36 of them, the row length chooses.
-// Products on request are always timed first: a solver's choice is up to 9% slower for
-// them, so it leaves lanes_per_row open.
-constexpr int64_t kTuneNnz = (int64_t)1 << 22;
-
-int spmv_autotune(hd_hamiltonian* h, int formats, bool for_solve)
+// format p) and keeps the fastest of each.  hd_spmv_time and hd_spmv_set_lanes(0) ask
+// for all formats, a solve of kLongNnz entries or more for its own; everything else
+// takes pick_default_sched where no such call came before.  (Timing the nine schedules
+// of a format takes 36 products and a wait for each, 0.4-0.6 ms of a 2.6 ms solve at
+// N=8, 2S=21.)
+int spmv_autotune(hd_hamiltonian* h, int formats)
 {
     if (h->storage == HD_STORAGE_MATRIX_FREE) {  // one kernel, nothing to choose
-        h->lanes_per_row = 1;
+        h->sched_chosen = kAllFormats;
         return HD_OK;
     }
     const bool have[3] = {h->d_val64 != nullptr, h->d_val32 != nullptr, h->d_code != nullptr};
-    if (for_solve && h->nnz < kTuneNnz) {
-        const double avg = h->dim ? (double)h->nnz / (double)h->dim : 0.0;
-        for (int prec = 0; prec < 3; ++prec)
-            if (have[prec] && (formats >> prec & 1)) h->spmv_sched[prec] = sched_for_lanes(avg > 24 ? 32 : 16);
-        return HD_OK;
-    }
     // one schedule per requested resident value format, each timed on zero vectors
     const size_t es = 8 * (h->is_complex ? 2 : 1);
     void *x = nullptr, *y = nullptr;
@@ -322,7 +329,7 @@ int spmv_autotune(hd_hamiltonian* h, int formats, bool for_solve)
     for (int prec = 0; prec < 3 && st == HD_OK; ++prec) {
         if (!have[prec] || !(formats >> prec & 1)) continue;
         float best = 1e30f;
-        int best_s = pick_default_sched(h);
+        int best_s = pick_default_sched(h, prec);
         for (int si = 0; si < kNumScheds && st == HD_OK; ++si) {
             h->spmv_sched[prec] = si;
             if ((st = spmv_launch(h, prec, x, y, h->stream)) != HD_OK) break;  // warm
@@ -337,9 +344,7 @@ int spmv_autotune(hd_hamiltonian* h, int formats, bool for_solve)
         }
         h->spmv_sched[prec] = best_s;
     }
-    if (formats >> default_precision(h) & 1)
-        h->lanes_per_row = kScheds[h->spmv_sched[default_precision(h)] >= 0 ? h->spmv_sched[default_precision(h)]
-                                                                            : pick_default_sched(h)].lpr;
+    if (st == HD_OK) h->sched_chosen |= formats;
     dfree(x);
     dfree(y);
     return st;
@@ -447,7 +452,7 @@ int hd_spmv_host(const hd_hamiltonian* h, const void* h_x, void* h_y)
 int hd_spmv_time(hd_hamiltonian* h, int32_t precision, int32_t iters, double* avg_ms)
 {
     if (!h || !avg_ms || iters <= 0) return fail(HD_ERR_ARG, "hd_spmv_time: bad argument");
-    if (!h->lanes_per_row) HD_CHECK(spmv_autotune(h));
+    if (h->sched_chosen != kAllFormats) HD_CHECK(spmv_autotune(h, kAllFormats & ~h->sched_chosen));
     const size_t z = h->is_complex ? 2 : 1;
     const size_t ex = (precision == HD_F32 || precision == HD_TILED_X32 ? 4 : 8) * z;
     const size_t ey = (precision == HD_F32 ? 4 : 8) * z;
@@ -474,10 +479,10 @@ int hd_spmv_time(hd_hamiltonian* h, int32_t precision, int32_t iters, double* av
 int hd_spmv_set_lanes(hd_hamiltonian* h, int32_t lanes)
 {
     if (!h) return fail(HD_ERR_ARG, "null handle");
-    if (lanes == 0) return spmv_autotune(h);
+    if (lanes == 0) return spmv_autotune(h, kAllFormats);
     if (lanes != 4 && lanes != 8 && lanes != 16 && lanes != 32 && lanes != 64)
         return fail(HD_ERR_ARG, "lanes per row must be 4, 8, 16, 32 or 64");
-    h->lanes_per_row = lanes;
+    h->sched_chosen = kAllFormats;
     for (int& si : h->spmv_sched) si = sched_for_lanes(lanes);
     return HD_OK;
 }
@@ -506,8 +511,7 @@ int hd_stream_copy(const void* d_src, void* d_dst, size_t bytes, int32_t iters, 
 int hd_spmv_get_lanes(const hd_hamiltonian* h, int32_t* lanes)
 {
     if (!h || !lanes) return fail(HD_ERR_ARG, "null argument");
-    const int si = h->spmv_sched[default_precision(h)];
-    *lanes = kScheds[si >= 0 ? si : pick_default_sched(h)].lpr;
+    *lanes = kScheds[sched_of(h, default_precision(h))].lpr;
     return HD_OK;
 }
 
@@ -519,7 +523,7 @@ int hd_spmv_get_schedule(const hd_hamiltonian* h, int32_t precision, int32_t* la
         *threads = 1024;
         return HD_OK;
     }
-    const int si = h->spmv_sched[precision] >= 0 ? h->spmv_sched[precision] : pick_default_sched(h);
+    const int si = sched_of(h, precision);
     *lanes = kScheds[si].lpr;
     *threads = kScheds[si].nt;
     return HD_OK;

@@ -568,3 +568,45 @@ def test_lanczos_step_forms(model, args, nev, tol):
     res = np.linalg.norm(A @ X - X * r.evals, axis=0) / np.maximum(1, np.abs(r.evals))
     assert np.all(res <= 1.01 * tol + 1e-13)
     assert np.max(np.abs(X.conj().T @ X - np.eye(nev))) < 1e-9
+
+
+@pytest.mark.parametrize("kind,args,want", [
+    ("lists", (12, 6, 0.03, False), ((4, 256), (4, 256), None)),      # 6 entries per row
+    ("lists", (12, 6, 0.1, True), ((8, 256), (8, 256), None)),        # 14
+    ("lists", (16, 6, 0.1, False), ((16, 512), (16, 512), None)),     # 25
+    ("lists", (12, 6, 0.3, True), ((64, 512), (64, 512), None)),     # 37, 924 rows, complex
+    ("sphere", (6, 15), ((32, 512),) * 3),                            # 37
+    ("lattice", (5, 4, 6), ((64, 512),) * 3),                        # 77, 1,932 rows
+    ("lattice", (5, 5, 6), ((32, 512),) * 3),                         # 113, 7,084 rows
+    ("lattice", (6, 4, 8), ((64, 1024), (32, 1024), (32, 1024)))])    # 155, 4.8M entries
+def test_untimed_schedules_by_row_length(kind, args, want):
+    """The schedule that a product takes when nothing was timed, by row length, type and
+    format; a solve of few entries leaves it, and the products match the CRS."""
+    import scipy.sparse as sp
+    say("untimed schedules", kind, args)
+    if kind == "lists":
+        K, n, fill, cplx = args
+        b = hd.FockBasis(hd.Sector.none(), n, K)
+        t = hd.TermTables.hash(K, **models.random_hash_tables(K, seed=1, max_k1=1, fill=fill, complex_values=cplx))
+    else:
+        b, t = models.sphere_problem(*args) if kind == "sphere" else models.ofl_problem(*args)
+    h = hd.Hamiltonian(b, t)
+    formats = [(p, w) for p, w in zip((hd.F64, hd.F32, hd.CODED), want) if w]
+    assert [tuple(h.schedule(p)) for p, _ in formats] == [w for _, w in formats]
+    if h.nnz < 1 << 22 and kind != "lists":
+        h.lanczos(nev=1, tol=1e-8)
+        assert [tuple(h.schedule(p)) for p, _ in formats] == [w for _, w in formats]
+    rp, col, val = h.crs()
+    A = sp.csr_matrix((val, col, rp), shape=(b.dim, b.dim))
+    rng = np.random.default_rng(1)
+    x = rng.normal(size=b.dim) + (1j * rng.normal(size=b.dim) if h.is_complex else 0)
+    scale = abs(A) @ np.abs(x)
+    m = h.info()["max_row"] + 4
+    for p, _ in formats:
+        u = 2.0 ** -24 if p == hd.F32 else 2.0 ** -53
+        # inputs rounded once, then at most max_row products (four roundings each, complex) summed
+        assert np.all(np.abs(h.spmv(x.astype(h.vec_dtype(p)), precision=p) - A @ x) <= 4 * m * u * scale), p
+    h.spmv_time_ms(precision=hd.F64, iters=1)  # times every format from here on
+    for p, _ in formats:
+        u = 2.0 ** -24 if p == hd.F32 else 2.0 ** -53
+        assert np.all(np.abs(h.spmv(x.astype(h.vec_dtype(p)), precision=p) - A @ x) <= 4 * m * u * scale), p
