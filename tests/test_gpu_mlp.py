@@ -226,3 +226,29 @@ def test_gradients_at_batch_edges(n_states, n):
     # first step: both moments corrected to g and g^2
     want = w - np.float32(1e-3) * g / (np.abs(g) + np.float32(1e-8))
     assert np.max(np.abs(net.get_weights() - want)) <= 1e-3 * 1e-4
+
+
+def test_inference_special_values():
+    """SiLU of the inference kernel at its ends: +inf where a sum overflows, and -0, not a
+    multiple of z, where the exponential does (|z| up to the largest float)."""
+    say("mlp inference, overflowing activations")
+    big = np.float32(3e38)
+    net = learned.AmplitudeNet(20, 0, seed=0, n_states=2)
+    w = np.zeros_like(net.get_weights())
+    off = 0
+    for rows, cols in ((256, 64), (256, 256), (256, 256), (64, 256)):
+        m = w[off:off + rows * cols].reshape(rows, cols)
+        if cols == 64:
+            m[:, 0:2] = big
+            m[:, 2] = -big
+            m[:, 3] = -1000.0
+        else:
+            m[:] = 1.0
+        off += rows * cols + rows
+    assert off == len(w)
+    w[-64:] = 0.25  # the outputs' biases
+    net.set_weights(w)
+    states = np.array([0b0011, 0b0100, 0b1000, 0b0000], dtype=np.uint64)
+    out = net.forward(states, np.zeros((4, 0), dtype=np.float32))
+    assert np.all(out[0] == np.inf)
+    assert np.all(out[1:] == np.float32(0.25))
