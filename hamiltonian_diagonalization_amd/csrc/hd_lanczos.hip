@@ -821,6 +821,7 @@ struct Lanczos {
     // steps, read when the host waits anyway.  Long vectors: every step; short
     // ones, where an event costs as much as a kernel: one in sixteen.
     std::vector<hipEvent_t> ev;
+    std::vector<int> ev_step;  // the step of each triple
     size_t ev_used = 0;
     double ms_spmv = 0, ms_ortho = 0;
     int timed = 0, steps = 0;
@@ -865,10 +866,12 @@ struct Lanczos {
         ev_err = hipEventRecord(ev[ev_used++], st);
     }
 
-    // Adds up the marked steps; the stream has been waited for.
-    int read_marks()
+    // Adds up the marked steps up to `last` (those queued behind a stop did nothing after
+    // their product); the stream has been waited for.
+    int read_marks(int last)
     {
         for (size_t i = 0; i + 2 < ev_used && ev_err == hipSuccess; i += 3) {
+            if (ev_step[i / 3] > last) break;
             float a = 0.f, b = 0.f;
             ev_err = hipEventElapsedTime(&a, ev[i], ev[i + 1]);
             if (ev_err == hipSuccess) ev_err = hipEventElapsedTime(&b, ev[i + 1], ev[i + 2]);
@@ -877,6 +880,7 @@ struct Lanczos {
             ++timed;
         }
         ev_used = 0;
+        ev_step.clear();
         return ev_err == hipSuccess ? HD_OK
                                     : fail(HD_ERR_HIP, std::string("Lanczos timing: ") + hipGetErrorString(ev_err));
     }
@@ -919,6 +923,7 @@ struct Lanczos {
         const bool timing = n >= 65536 || steps % 16 == 0;
         ++steps;
         T* w = vec(j + 1);
+        if (timing) ev_step.push_back(j);
         mark(timing);
         HD_CHECK(apply(vec(j), w, prec));
         mark(timing);
@@ -965,7 +970,7 @@ struct Lanczos {
     {
         HD_HIP(hipMemcpyAsync(out, dst, offsetof(LzState, theta), hipMemcpyDeviceToHost, st));
         HD_HIP(hipStreamSynchronize(st));
-        return read_marks();
+        return read_marks(out->stop ? out->stop_step : m);
     }
 
     int scale_into(const T* src, double s, T* dst_)
@@ -1181,6 +1186,14 @@ static int run_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* eval
         }
         return HD_OK;
     };
+    // Steps enqueued before the host looks for a stop.  The products of the steps queued
+    // behind a stop are lost, so after one the steps go singly and then twice as many each
+    // time: a matrix of few distinct eigenvalues stops at every few steps (constant
+    // pseudopotentials, N=10, 2S=27: 85 products with whole cycles, 30 needed).  Long
+    // vectors begin that way, and from 2^20 entries on, where four steps take a hundred
+    // times the wait, no more than four are queued.
+    const int chunk_max = L.n >= (1 << 20) ? 4 : m;
+    int chunk = L.n >= 65536 ? 2 : m;
     int done = 0;         // steps of the current cycle whose coefficients are here
     int tested = 0;       // basis sizes tested so far
     bool fresh = true;    // the next pass of the loop begins a cycle
@@ -1219,10 +1232,11 @@ static int run_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* eval
                     }
                 }
             if (ended || done >= m) break;
-            const int upto = check_in_cycle ? std::min(m, done + (L.n >= 65536 ? 1 : 4)) : m;
+            const int upto = std::min(m, done + std::min(chunk, check_in_cycle ? (L.n >= 65536 ? 1 : 4) : m));
             for (int j = done; j < upto; ++j)
                 HD_CHECK(L.step(j, k, prec, !pro || j == m - 1, eps_op, om_cycle, std::min(1e-12, 0.02 * tol)));
             HD_CHECK(L.read_state(hs.get()));
+            chunk = hs->stop ? 1 : std::min(2 * chunk, chunk_max);
             if (hs->stop) {
                 HD_CHECK(L.resume(hs->stop_step, hs->stop, o.seed, &rng_stream));
                 done = hs->stop_step + 1;

@@ -472,13 +472,13 @@ typedef struct {
     int32_t converged;
     int32_t nconv;
     int32_t restarts;
-    int32_t matvecs;      /* all operator applications */
+    int32_t matvecs;      /* all operator applications, those queued behind a breakdown included */
     int32_t matvecs_f32;
     int32_t matvecs_f64;
     double residual[64];  /* ||H x - l x|| / max(1,|l|), FP64 operator, per eigenpair */
     double time_total_ms;
-    double time_spmv_ms;
-    double time_ortho_ms;
+    double time_spmv_ms;  /* products and, below, the steps' other kernels on the device: the timed */
+    double time_ortho_ms; /* steps' mean times their number (below 65,536 rows one step in 16 is timed) */
     int32_t reorth_steps; /* steps that orthogonalised against the whole basis */
     int32_t f32_cycles_discarded; /* HD_F32: FP32 cycles run again in FP64 (their rounding
                                      estimate exceeded the budget once their coefficients

@@ -610,3 +610,19 @@ def test_untimed_schedules_by_row_length(kind, args, want):
     for p, _ in formats:
         u = 2.0 ** -24 if p == hd.F32 else 2.0 ** -53
         assert np.all(np.abs(h.spmv(x.astype(h.vec_dtype(p)), precision=p) - A @ x) <= 4 * m * u * scale), p
+
+
+@pytest.mark.parametrize("n,two_s", [(6, 15), (8, 21), (10, 27)])
+def test_lanczos_few_eigenvalues_loses_few_products(n, two_s):
+    """Equal pseudopotentials: a handful of distinct eigenvalues, so the basis breaks down
+    every few steps.  Products queued behind a breakdown are lost: no more of them than
+    steps were made since the last one, beyond the first cycle of a short vector."""
+    say("lanczos, equal pseudopotentials", n, two_s)
+    b = hd.FockBasis(hd.Sector.lz((n * two_s) % 2, two_s), n, two_s + 1)
+    h = hd.Hamiltonian(b, models.sphere_tables(two_s, np.ones(two_s - 1)), values=(hd.F64,))
+    ncv = 27
+    r = h.lanczos(nev=3, tol=1e-10, ncv=ncv)
+    say(r)
+    assert r.converged
+    # one cycle, as many products lost at most, and the residuals of the three pairs
+    assert r.matvecs <= 2 * ncv + 3 + (0 if b.dim >= 65536 else ncv)
