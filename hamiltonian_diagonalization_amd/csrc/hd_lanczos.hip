@@ -1297,9 +1297,12 @@ static int run_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* eval
             fresh = true;
             continue;
         }
-        if (all) {
+        // A basis of the whole space has nothing to continue with (vec(mc) is rounding
+        // noise): its pairs are the answer, whatever their residuals.
+        const bool spans = mc >= L.n;
+        if (all || spans) {
             HD_CHECK(ritz_pairs());
-            bool hopeless = missed == 3;
+            bool hopeless = missed == 3 || spans;
             for (int i = 0; i < nev; ++i)
                 if (missed && resid[i] * resid[i] - res_est[i] * res_est[i] > tol * tol) hopeless = true;
             if (nconv == nev || hopeless || restarts >= max_restarts) {

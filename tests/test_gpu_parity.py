@@ -626,3 +626,27 @@ def test_lanczos_few_eigenvalues_loses_few_products(n, two_s):
     assert r.converged
     # one cycle, as many products lost at most, and the residuals of the three pairs
     assert r.matvecs <= 2 * ncv + 3 + (0 if b.dim >= 65536 else ncv)
+
+
+@pytest.mark.parametrize("model,args,nev,tol", [
+    ("sphere", (3, 9, 1), 2, 1e-17), ("sphere", (3, 9, 1), 8, 1e-17), ("sphere", (4, 8, 2), 4, 1e-17),
+    ("sphere", (4, 9, 0), 4, 1e-15), ("lattice", (4, 3, 3), 3, 1e-17)])
+def test_lanczos_whole_space_with_unreachable_tol(model, args, nev, tol):
+    """A basis of the whole space whose residuals miss tol: the solve ends with those
+    pairs, unconverged, instead of restarting from rounding noise."""
+    say("lanczos, whole space, tol", tol, model, args)
+    b, t = models.sphere_problem(*args) if model == "sphere" else models.ofl_problem(*args)
+    h = hd.Hamiltonian(b, t, values=(hd.F64,))
+    rp, col, val = h.crs()
+    A = np.zeros((b.dim, b.dim), dtype=val.dtype)
+    for i in range(b.dim):
+        A[i, col[rp[i]:rp[i + 1]]] = val[rp[i]:rp[i + 1]]
+    assert b.dim <= 2 * nev + 21
+    r = h.lanczos(nev=nev, tol=tol, seed=1)
+    say(r)
+    w = np.linalg.eigvalsh(A)
+    # both solvers err by a modest multiple of the rounding of |A|
+    assert np.max(np.abs(r.evals - w[:nev])) <= 64 * b.dim * 2.0 ** -53 * np.max(np.abs(w))
+    X = np.stack([h.eigenvector(i) for i in range(nev)], axis=1)
+    assert np.max(np.abs(A @ X - X * r.evals)) <= 64 * b.dim * 2.0 ** -53 * np.max(np.abs(w))
+    assert np.max(np.abs(X.conj().T @ X - np.eye(nev))) <= 64 * b.dim * 2.0 ** -53
