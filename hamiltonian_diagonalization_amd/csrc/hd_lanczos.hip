@@ -834,9 +834,8 @@ struct Lanczos {
         dfree(coef); dfree(dscal); dfree(dY);
     }
 
-    int alloc(int nev, bool need_x32, bool need_y32)
+    int alloc(bool need_x32, bool need_y32)
     {
-        HD_CHECK(dalloc_t(&ritz, (size_t)nev * n, "eigenvectors"));
         HD_CHECK(dalloc_t(&V, (size_t)(m + 1) * n, "Lanczos basis"));
         HD_CHECK(dalloc_t(&V2, (size_t)(m + 1) * n, "restart buffer"));
         if (need_x32) HD_CHECK(dalloc_t(&x32, (size_t)n, "FP32 x"));
@@ -898,6 +897,20 @@ struct Lanczos {
         HD_CHECK(spmv_launch(h, HD_F32, x32, y32, st));
         hipLaunchKernelGGL(k_to_f64<C>, dim3(nb), dim3(kVB), 0, st, n, y32, y);
         return HD_OK;
+    }
+
+    // The Ritz vectors; where there is no room beside those of the handle's last solve,
+    // in their place.
+    int alloc_ritz(int nev)
+    {
+        if (ritz) return HD_OK;
+        int rc = dalloc_t(&ritz, (size_t)nev * n, "eigenvectors");
+        if (rc == HD_ERR_NOMEM && h->lz && h->lz->d_vec) {
+            dfree(h->lz->d_vec);
+            h->lz->d_vec = nullptr;
+            rc = dalloc_t(&ritz, (size_t)nev * n, "eigenvectors");
+        }
+        return rc;
     }
 
     // one Gram-Schmidt pass of w against V[0..j] (enqueued; the kernels decide)
@@ -1057,7 +1070,7 @@ static int run_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* eval
         if (p < HD_TILED) untuned |= 1 << p;
     untuned &= ~h->sched_chosen;
     if (!free_ && untuned && h->nnz >= kLongNnz) HD_CHECK(spmv_autotune(h, untuned));
-    HD_CHECK(L.alloc(nev, mixed, mixed && prec32 == HD_F32));
+    HD_CHECK(L.alloc(mixed, mixed && prec32 == HD_F32));
     const double tol = o.tol > 0 ? o.tol : 1e-10;
     const double budget = o.f32_budget > 0 ? std::min(o.f32_budget, 1.0) : 1.0;
     // relative rounding of one FP32-input product: x rounded to FP32, plus
@@ -1172,6 +1185,7 @@ static int run_lanczos(hd_hamiltonian* h, const hd_lanczos_opts& o, double* eval
     std::vector<double> resid(nev, 0.0);
     int nconv = 0;
     auto ritz_pairs = [&]() -> int {
+        HD_CHECK(L.alloc_ritz(nev));
         HD_CHECK(L.combine(mc, Y, mc, nev, L.ritz));
         nconv = 0;
         for (int i = 0; i < nev; ++i) {

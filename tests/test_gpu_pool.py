@@ -178,3 +178,27 @@ def test_last_block_returns_the_pool():
             "assert hd.trim_memory(1 << 40) <= 256 << 20\n")
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     subprocess.run([sys.executable, "-c", code], cwd=root, check=True, timeout=100)
+
+
+def test_second_solve_fits_where_the_first_did():
+    """A handle's second solve needs the room of its first: with memory for the basis but
+    not for two sets of eigenvectors, the new ones take the place of the old."""
+    say("pool: two solves of N=10 2S=27 in little memory")
+    gc.collect()
+    b, t = models.sphere_problem(10, 27, 0)
+    h = hd.Hamiltonian(b, t, values=(hd.F64,))
+    kw = dict(nev=20, ncv=60, tol=1e-6, seed=0)
+    vec = b.dim * 8
+    # 2 (ncv + 1) vectors of the basis buffers and 20 of eigenvectors, the old ones allocated
+    room = (2 * 61 + 10) * vec
+    first = h.lanczos(**kw)
+    hd.trim_memory()
+    ballast = []
+    while _mem_info()[0] > room + (4 << 20):  # one allocation leaves some hundred MiB more than asked for
+        ballast.append(hd.DeviceBuffer(_mem_info()[0] - room))
+    second = h.lanczos(**kw)
+    assert np.array_equal(second.evals, first.evals) or np.allclose(second.evals, first.evals, rtol=0, atol=1e-5)
+    x = h.eigenvector(0)
+    y = h.spmv(x, precision=hd.F64)
+    assert np.linalg.norm(y - second.evals[0] * x) <= 2e-6 * max(1, abs(second.evals[0]))
+    del ballast
