@@ -625,7 +625,8 @@ int launch_merge(int grid, hipStream_t st, int64_t dim, const int64_t* raw_ptr, 
         const bool small = dim < ((int64_t)1 << (32 - bits));
         const void* fn = small ? reinterpret_cast<const void*>(&k_gmerge_block<CPLX, TH, uint32_t>)
                                : reinterpret_cast<const void*>(&k_gmerge_block<CPLX, TH, uint64_t>);
-        if (lds > 32 * 1024) HD_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (lds + (small ? 4 : 8) * 8 * TH + 64 > 64 * 1024)  // with the keys and the wavefronts' counts
+            HD_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         if (small)
             hipLaunchKernelGGL((k_gmerge_block<CPLX, TH, uint32_t>), dim3(grid), dim3(TH), lds, st, dim, raw_ptr, rcol, rval,
                                tol, mcol, mval, kept, ntrim, min_len, bits);

@@ -97,10 +97,11 @@ def test_matrix_free_paths(monkeypatch, path):
 
 
 @pytest.mark.parametrize("n, two_s, v", [(2, 55, None), (3, 40, {1: 1.0}), (11, 16, None), (12, 15, {1: 1.0, 3: 0.3}),
-                                         (13, 18, {1: 1.0}), (6, 15, {13: 1.0})])
+                                         (13, 18, {1: 1.0}), (6, 15, {13: 1.0}), (2, 58, None), (3, 58, {1: 1.0})])
 def test_fill_pair_masks_bit_exact(oracle, n, two_s, v):
-    """The mask walk of the sphere's rows: one pair, 56 orbitals (sums of two beyond 63),
-    55, 66 and 78 pairs around the 64 of a pass, and tables with trimmed or absent entries."""
+    """The mask walk of the sphere's rows: one pair, 56 and 59 orbitals (sums of two beyond 63;
+    59 is the most the count's LDS holds), 55, 66 and 78 pairs around the 64 of a pass,
+    and tables with trimmed or absent entries."""
     say("pair masks", n, two_s, v)
     b, t = models.sphere_problem(n, two_s)
     if v:

@@ -310,3 +310,96 @@ def test_merge_row_lengths(oracle):
         ref = oracle.build_general(K, basis.states(), K, t["nk1"], t["k1"], t["v"], t["nq1"], t["q1"], t["e"])
         rp, col, val = h.crs()
         assert np.array_equal(rp, ref.rowptr) and np.array_equal(col, ref.col) and np.array_equal(val, ref.values())
+
+
+def _upper_row(s, K, t, states, tol=1e-14):
+    """One row of the upper-storage build, term by term in the build's order: columns,
+    sums from +0.0 in term order, and the number of raw terms."""
+    occ = [k for k in range(K) if s >> k & 1]
+    sums, raw = {}, 0
+    for k4 in occ:
+        for k3 in occ:
+            if k3 == k4:
+                continue
+            above = sum(1 << k for k in occ if k > k3 and k != k4)
+            for k2 in range(K):
+                if above >> k2 & 1 or (s >> k2 & 1 and k2 not in (k3, k4)):
+                    continue
+                ent = (k4 * K + k3) * K + k2
+                for j in range(t["nk1"][ent]):
+                    k1 = int(t["k1"][ent, j])
+                    if k1 == k2 or (s >> k1 & 1 and k1 not in (k3, k4)):
+                        continue
+                    out, c = s, 0
+                    for k in (k4, k3, k2, k1):
+                        c += bin(out & ((1 << k) - 1)).count("1")
+                        out ^= 1 << k
+                    el = t["v"][ent, j]
+                    if out < s or not abs(el) > tol:
+                        continue
+                    raw += 1
+                    sums[out] = sums.get(out, 0.0) + (-el if c & 1 else el)
+    kept = sorted((int(np.searchsorted(states, o)), v) for o, v in sums.items() if not abs(v) < tol)
+    return [c for c, _ in kept], [v for _, v in kept], raw
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+def test_merge_long_rows_of_a_large_sector(cplx):
+    """Rows of 2,049 to 4,096 raw terms in a sector of more than 2^20 states: the block
+    merge with 64-bit keys and its largest LDS.  Lists for pairs within the six lowest
+    orbitals alone keep the other rows short."""
+    say("merge of long rows, K=25 N=8, complex", cplx)
+    K, n = 25, 8
+    t = models.random_hash_tables(K, seed=4, max_k1=8, fill=0.9, complex_values=cplx, quadratic=False)
+    k4, k3 = np.divmod(np.arange(K ** 3) // K, K)
+    t["nk1"][(k4 >= 6) | (k3 >= 6)] = 0
+    basis = hd.FockBasis(hd.Sector.none(), n, K)
+    assert basis.dim > 1 << 20
+    states = basis.states()
+    h = hd.Hamiltonian(basis, hd.TermTables.hash(K, **t), storage=hd.STORAGE_UPPER_REF, values=(hd.F64,))
+    low = np.array([bin(int(x) & 63).count("1") for x in states[:200000]])
+    rows = [int(r) for r in np.flatnonzero(low == 6)[::40]] + [int(r) for r in np.flatnonzero(low == 5)[:3]] + [basis.dim - 1]
+    longest = 0
+    for r in rows:
+        col, val, raw = _upper_row(int(states[r]), K, t, states)
+        longest = max(longest, raw)
+        _, c, v = h.crs(r, r + 1)
+        assert np.array_equal(c, col), r
+        assert np.array_equal(v, np.array(val, dtype=v.dtype)), r
+    assert 2048 < longest <= 4096
+
+
+@pytest.mark.parametrize("model,args", [
+    ("sphere", (3, 31)), ("sphere", (3, 32)), ("sphere", (3, 39)), ("sphere", (4, 45)), ("sphere", (2, 55)),
+    ("lattice", (6, 6, 3)), ("lattice", (8, 4, 3)), ("lattice", (7, 5, 4))])
+def test_walk_on_both_sides_of_32_orbitals(model, args):
+    """The term walk with 32 lanes per row (up to 32 orbitals) and with 64: hash lists of
+    32 to 56 orbitals against the pair-structure build of the same tables, bit for bit in
+    upper storage; full storage adds the conjugate of it."""
+    import scipy.sparse as sp
+    say("term walk lanes", model, args)
+    if model == "sphere":
+        n, two_s = args
+        K, layout = two_s + 1, hd.LAYOUT_SPHERE
+        basis = hd.FockBasis(hd.Sector.lz((n * two_s) % 2, two_s), n, K)
+        t = models.sphere_tables(two_s, models.coulomb_list(two_s))
+        kt, vt = t.ktable, t.vtable
+        pair = t
+    else:
+        X, Y, n = args
+        K, layout = X * Y, hd.LAYOUT_OFL
+        basis = hd.FockBasis(hd.Sector.k2d(1, 2, X, Y), n, K)
+        kt, vt, _ = models.ofl_tables(X, Y, 3)
+        pair = hd.TermTables(layout, K, kt, vt, np.zeros(K))
+    lists = hd.TermTables.hash(K, **hd.hash_lists_from_array(layout, K, kt, vt))
+    a = hd.Hamiltonian(basis, pair, storage=hd.STORAGE_UPPER_REF, values=(hd.F64,))
+    b = hd.Hamiltonian(basis, lists, storage=hd.STORAGE_UPPER_REF, values=(hd.F64,))
+    say("dim", basis.dim, "nnz", a.nnz, b.nnz)
+    for x, y in zip(a.crs(), b.crs()):
+        assert np.array_equal(x, y)
+    rp, col, val = b.crs()
+    frp, fcol, fval = hd.Hamiltonian(basis, lists, storage=hd.STORAGE_FULL, values=(hd.F64,)).crs()
+    up = sp.csr_matrix((val, col, rp), shape=(basis.dim, basis.dim))
+    want = (up + sp.triu(up, 1).conj().T).tocsr()
+    want.sort_indices()
+    assert np.array_equal(frp, want.indptr) and np.array_equal(fcol, want.indices) and np.array_equal(fval, want.data)
