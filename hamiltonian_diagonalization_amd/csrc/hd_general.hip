@@ -525,7 +525,8 @@ k_gmerge_wave(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __
 // term order from +0.0, and a prefix sum over the block places the kept ones.
 // k_gmerge sorts 64-bit keys in LDS with a barrier per stage, reads the values in
 // sorted order from L2 twice and adds up the counts on one thread (6x5 N=6
-// Wannier, rows of up to 4,096 raw terms: 19.8 -> 7.3 + 2.9 ms).
+// Wannier, rows of up to 4,096 raw terms: 19.8 -> 7.3 + 2.9 ms; merge and completion on the
+// 6x5 N=8 hash tables, dim 195,143: 14.9 -> 9.2 ms).
 template <bool CPLX, int THREADS, typename Key>
 __global__ void __launch_bounds__(THREADS)
 k_gmerge_block(int64_t dim, const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col_in,

@@ -87,9 +87,6 @@ HD_DEV double2 scale(double2 a, double s) { return make_double2(a.x * s, a.y * s
 template <typename T> HD_DEV T zero();
 template <> HD_DEV double zero<double>() { return 0.0; }
 template <> HD_DEV double2 zero<double2>() { return make_double2(0.0, 0.0); }
-template <typename T> HD_DEV T real_part(double x);  // x + 0i
-template <> HD_DEV double real_part<double>(double x) { return x; }
-template <> HD_DEV double2 real_part<double2>(double x) { return make_double2(x, 0.0); }
 HD_DEV float narrow(double a) { return (float)a; }
 HD_DEV float2 narrow(double2 a) { return make_float2((float)a.x, (float)a.y); }
 HD_DEV double widen(float a) { return (double)a; }
@@ -544,8 +541,9 @@ k_lz_finish(LzStep p, int second_done, typename E<C>::T* __restrict__ w, LzState
 // A whole step after the product in one launch of one block: for a short vector
 // the six launches above cost more than their work (N=6, 2S=15, dim 338: 9.4 us
 // per step against 20 us).  Beyond the limits below one CU's loads make a full
-// pass slower than the launches (N=8, 2S=21, dim 8,512: 53 us per step against 24 us;
-// dim 3,876 complex, a pass in every step: 37 against 29 us).
+// pass slower than the launches.  Solve time per product, one launch against several, us:
+//   real     dim 1,656: 30 / 38, 3,788: 36 / 39, 4,370: 38 / 40, 5,744: 45 / 44, 8,512: 60 / 41
+//   complex  dim   490: 28 / 41, 1,932: 39 / 45, 2,130: 41 / 46, 3,876: 54 / 46, 4,751: 63 / 50
 constexpr int kSmallThreads = 1024;
 // one-launch steps up to this dimension (real, complex)
 constexpr int64_t kSmallReal = 4096, kSmallComplex = 2048;

@@ -697,9 +697,9 @@ void mlp_free_work(hd_mlp* m)
     m->cap = 0;
 }
 
-int mlp_work(hd_mlp* m, int64_t npad, bool train)
+int mlp_work(hd_mlp* m, int64_t npad)
 {
-    if (m->cap >= npad && (!train || m->hT[0])) return HD_OK;
+    if (m->cap >= npad) return HD_OK;
     mlp_free_work(m);
     const int64_t c = std::max<int64_t>(npad, 64);
     HD_CHECK(dalloc_t(&m->h[0], (size_t)c * kIn, "MLP features"));
@@ -709,16 +709,14 @@ int mlp_work(hd_mlp* m, int64_t npad, bool train)
     }
     HD_CHECK(dalloc_t(&m->out, (size_t)c * kOutPad, "MLP output"));
     HD_CHECK(dalloc_t(&m->partial, (size_t)(c / 32 + 1024), "MLP partials"));
-    if (train) {
-        HD_CHECK(dalloc_t(&m->wpart, (size_t)kMaxSplits * kParams, "MLP partial gradients"));
-        HD_CHECK(dalloc_t(&m->hT[0], (size_t)c * kIn, "MLP features^T"));
-        for (int l = 1; l < 4; ++l) HD_CHECK(dalloc_t(&m->hT[l], (size_t)c * kW, "MLP activations^T"));
-        HD_CHECK(dalloc_t(&m->d[4], (size_t)c * kOutPad, "MLP output delta"));
-        HD_CHECK(dalloc_t(&m->dT[4], (size_t)c * kOutPad, "MLP output delta^T"));
-        for (int l = 1; l < 4; ++l) {
-            HD_CHECK(dalloc_t(&m->d[l], (size_t)c * kW, "MLP deltas"));
-            HD_CHECK(dalloc_t(&m->dT[l], (size_t)c * kW, "MLP deltas^T"));
-        }
+    HD_CHECK(dalloc_t(&m->wpart, (size_t)kMaxSplits * kParams, "MLP partial gradients"));
+    HD_CHECK(dalloc_t(&m->hT[0], (size_t)c * kIn, "MLP features^T"));
+    for (int l = 1; l < 4; ++l) HD_CHECK(dalloc_t(&m->hT[l], (size_t)c * kW, "MLP activations^T"));
+    HD_CHECK(dalloc_t(&m->d[4], (size_t)c * kOutPad, "MLP output delta"));
+    HD_CHECK(dalloc_t(&m->dT[4], (size_t)c * kOutPad, "MLP output delta^T"));
+    for (int l = 1; l < 4; ++l) {
+        HD_CHECK(dalloc_t(&m->d[l], (size_t)c * kW, "MLP deltas"));
+        HD_CHECK(dalloc_t(&m->dT[l], (size_t)c * kW, "MLP deltas^T"));
     }
     m->cap = c;
     return HD_OK;
@@ -786,8 +784,8 @@ InferArgs infer_args(const hd_mlp* m, int64_t n, const uint64_t* states, const f
     return a;
 }
 
-// forward over npad rows already featurized in h[0] (and hT[0] when training)
-void mlp_forward_core(hd_mlp* m, int64_t npad, bool train)
+// training's forward pass over npad rows already featurized in h[0] and hT[0]
+void mlp_forward_core(hd_mlp* m, int64_t npad)
 {
     const int M = (int)npad;
     for (int l = 0; l < 3; ++l) {
@@ -796,7 +794,7 @@ void mlp_forward_core(hd_mlp* m, int64_t npad, bool train)
         g.C = m->z[l + 1]; g.ldc = kW;
         g.bias = m->params + kOff[l] + kRows[l] * kCols[l];
         g.H = m->h[l + 1]; g.ldh = kW;
-        if (train) { g.HT = m->hT[l + 1]; g.ldht = M; }
+        g.HT = m->hT[l + 1]; g.ldht = M;
         gemm(m->stream, EPI_BIAS_SILU, g);
     }
     GemmArgs g = ga(M, kOutPad, kW, m->h[3], kW, m->wb[3], kW);
@@ -885,13 +883,13 @@ int batch_pass(hd_mlp* m, const uint64_t* states, const float* params, const flo
 {
     if (n <= 0) return fail(HD_ERR_ARG, "empty batch");
     const int64_t npad = pad64(n);
-    HD_CHECK(mlp_work(m, npad, true));
+    HD_CHECK(mlp_work(m, npad));
     const uint64_t* ds;
     const float *dp, *dt;
     HD_CHECK(stage_batch(m, states, params, tgt, n, host != 0, &ds, &dp, &dt, 1));
     hipLaunchKernelGGL(k_featurize, dim3((unsigned)(npad / 32)), dim3(256), 0, m->stream, n, npad, ds, dp, 1, m->n_bits,
                        m->n_params, m->h[0], m->hT[0]);
-    mlp_forward_core(m, npad, true);
+    mlp_forward_core(m, npad);
     return mlp_backward(m, n, npad, dt, lambda, splits);
 }
 

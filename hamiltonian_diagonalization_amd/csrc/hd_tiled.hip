@@ -31,11 +31,12 @@
 // (Hermitian) matrices use the same layout with 8 values per line (a 3-bit word
 // field) and read their larger dictionary from L2 (k_spmv_tiled_c).
 //
-// The layout is built on the device from the coded CRS, one block per group:
-// an LDS hash set collects the group's lines, a bitonic sort orders them,
-// per-(chunk, row) counts give the row starts, and each entry is written to
-// its slot.  Every write is
-// bounds-checked against the group's counts.
+// The layout is built on the device from the coded CRS in two passes of one block per
+// group.  Pass 1 finds the group's lines: a bitmap of all x lines in LDS, whose set bits
+// come out in order, or, where the sector's lines do not fit it, a hash set and a sort.
+// Binary searches of the rows' columns give the per-(chunk, row) counts.  Pass 2 reads
+// that plan and writes each entry to its slot.  Every write is bounds-checked against
+// the group's counts.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -246,24 +247,8 @@ __device__ __forceinline__ void tile_plan(TilePlanLds<TG>& S, int64_t dim, const
             const int L = S.n_lines;
             int P = 1;
             while (P < L) P <<= 1;
-            if (P <= 8 * kBuildThreads) {
-                bitonic_blocked<uint32_t, kBuildThreads>(S.sorted, P);
-            } else {
-                for (int k = 2; k <= P; k <<= 1)
-                    for (int jj = k >> 1; jj > 0; jj >>= 1) {
-                        for (int i = t; i < P; i += kBuildThreads) {
-                            const int ixj = i ^ jj;
-                            if (ixj > i) {
-                                const uint32_t a = S.sorted[i], b = S.sorted[ixj];
-                                if ((a > b) == ((i & k) == 0)) {
-                                    S.sorted[i] = b;
-                                    S.sorted[ixj] = a;
-                                }
-                            }
-                        }
-                        __syncthreads();
-                    }
-            }
+            static_assert(kHashSlots <= 8 * kBuildThreads, "the lines are sorted in registers");
+            bitonic_blocked<uint32_t, kBuildThreads>(S.sorted, P);
             for (int i = t; i < L; i += kBuildThreads) S.rank_of[hash_find(S.keys, S.sorted[i])] = (uint16_t)i;
         }
     }
@@ -943,7 +928,10 @@ static int tiled_build_tg(hd_hamiltonian* h, int entry_bytes)
     h->bytes += h->tg_bytes;
     // Block order: 64 groups per XCD and window once every XCD has such a run.  It was
     // the fastest of the five candidates at N=12, 2S=33 (3.360 ms; 3.366 with 16,
-    // 3.372 with 256, 3.407 in launch order) and on the 6x5 lattice, and timing them
+    // 3.372 with 256, 3.407 in launch order) and on the 6x5 lattice at N=10; the four
+    // differ by 1-3% at N=10, 2S=27 (52.7 us; 52.6, 51.6, 52.9) and on the 6x5 lattice
+    // at N=8 (105.8; 106.5, 105.6, 106.7), and 0 is the fastest below 512 groups (N=8,
+    // 2S=21, 67 groups: 5.8 us against 6.5; 5x5 lattice, N=8, 338: 24.9, 25.5).  Timing them
     // all took 65 of the 190 ms from a new set of tables to the first product at
     // N=12, 2S=33.  Smaller grids are resident at once, so their order is free.
     // hd_ham_tile_order(h, -1) times the candidates.
