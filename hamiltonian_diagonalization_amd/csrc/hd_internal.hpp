@@ -102,7 +102,7 @@ int dalloc_t(T** p, size_t count, const char* what)
 }
 void dfree(void* p);
 hipError_t dfree_status(void* p);  // dfree with the driver's answer
-// Non-blocking streams, kept for reuse (hd_basis.hip); stream_put waits for the
+// Non-blocking streams, kept for reuse (hd_pool.hpp); stream_put waits for the
 // stream's work.
 hipError_t stream_get(hipStream_t* s);
 void stream_put(hipStream_t s);

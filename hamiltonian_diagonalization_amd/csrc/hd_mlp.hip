@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(256) k_params(ParamArgs a)
 //
 // Bound: the vector instructions (67% of the cycles; the SiLU is 768 of 44 cycles
 // per state) beside the MFMAs (31%) and the fragment reads from LDS.  Over the
-// N=12, 2S=33 sector (7.76M states, S = 5) 3.55 ms, 0.67 PFLOP/s on the padded
+// N=12, 2S=33 sector (7.76M states, S = 5) 3.55 ms, 0.68 PFLOP/s on the padded
 // work, against 11.6 ms for a kernel that kept the activations in LDS (512-byte
 // rows, every access a bank conflict, two barriers per 32 columns of weights).
 // Two sets of 32 states per wave, which halve the fragment reads, need the AGPRs

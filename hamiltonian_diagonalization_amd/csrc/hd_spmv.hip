@@ -8,7 +8,8 @@
 // pure gather: LPR lanes of a wavefront stream the row's column indices and
 // values with scalar non-temporal loads (the stream is read once and must not
 // evict x from L2/MALL), gather x, and reduce with cross-lane shuffles.  One
-// block handles one chunk of NT/LPR rows; (LPR, NT) is autotuned per matrix.
+// block handles one chunk of NT/LPR rows; (LPR, NT) is timed per matrix and format or
+// follows from the row length (pick_default_sched).
 // Measured on MI355X the kernel is bound by the L2-miss traffic of the x
 // gathers, not by the stream, so the block -> chunk order is chosen for L2
 // reuse (window_chunk); 16-byte vector loads, persistent grids and four

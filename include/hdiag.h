@@ -377,7 +377,8 @@ int hd_spmv_time(hd_hamiltonian* h, int32_t precision, int32_t iters, double* av
  * the calibration reference for hardware byte counters; mean kernel time from
  * HIP events on the default stream. */
 int hd_stream_copy(const void* d_src, void* d_dst, size_t bytes, int32_t iters, double* avg_ms);
-/* Rows per wavefront schedule of the SpMV (lanes per row 4..64, 0 = autotune). */
+/* Rows per wavefront schedule of the SpMV (lanes per row 4..64, 0 = time every schedule
+ * on every resident format). */
 int hd_spmv_set_lanes(hd_hamiltonian* h, int32_t lanes_per_row);
 int hd_spmv_get_lanes(const hd_hamiltonian* h, int32_t* lanes_per_row);
 /* Tiled layout of the coded operator (no reference counterpart; it replaces
@@ -421,8 +422,9 @@ int hd_ham_tile_order(hd_hamiltonian* h, int64_t groups_per_xcd);
  * the handle. */
 int hd_ham_device_tiled(const hd_hamiltonian* h, const int64_t** d_base, const uint32_t** d_entries,
                         const uint32_t** d_lines, const uint32_t** d_offsets, const double** d_diag);
-/* The SpMV schedule of one value format: lanes per row and threads per block
- * (each format is autotuned separately; no reference counterpart). */
+/* The SpMV schedule of one value format: lanes per row and threads per block, timed
+ * (hd_spmv_time, hd_spmv_set_lanes(0), a long solve in that format), set, or else by
+ * row length; no reference counterpart. */
 int hd_spmv_get_schedule(const hd_hamiltonian* h, int32_t precision, int32_t* lanes_per_row, int32_t* threads);
 
 /* ---------------------------------------------------------------- Lanczos */
