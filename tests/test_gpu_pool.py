@@ -194,10 +194,12 @@ def test_second_solve_fits_where_the_first_did():
     first = h.lanczos(**kw)
     hd.trim_memory()
     ballast = []
-    while _mem_info()[0] > room + (4 << 20):  # one allocation leaves some hundred MiB more than asked for
-        ballast.append(hd.DeviceBuffer(_mem_info()[0] - room))
+    for _ in range(16):  # one allocation leaves some hundred MiB more than asked for
+        if _mem_info()[0] > room + (4 << 20):
+            ballast.append(hd.DeviceBuffer(_mem_info()[0] - room))
     second = h.lanczos(**kw)
-    assert np.array_equal(second.evals, first.evals) or np.allclose(second.evals, first.evals, rtol=0, atol=1e-5)
+    # each eigenvalue within its residual (1e-6) of the matrix's
+    assert np.all(np.abs(second.evals - first.evals) <= 2e-6 * np.maximum(1, np.abs(first.evals)))
     x = h.eigenvector(0)
     y = h.spmv(x, precision=hd.F64)
     assert np.linalg.norm(y - second.evals[0] * x) <= 2e-6 * max(1, abs(second.evals[0]))
